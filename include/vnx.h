@@ -549,6 +549,16 @@ size_t vnx_tree_attn_workspace_args(const vnx_tree_attn_args* args);
 int vnx_tree_attn(const vnx_tree_attn_args* args, void* workspace, size_t workspace_bytes,
                   void* stream);
 
+/* The same attention for a chain of any length N >= 1 (the prompts of a
+ * prefill), one launch, no workspace: batch row b's N new rows are already in
+ * the cache at rows tp_b .. tp_b + N - 1 (tp_b = tp_batch[b] clamped to
+ * [0, Tp], or Tp), node i sits at tp_b + i and sees cache rows j <= tp_b + i.
+ * bf16 rows, d in {64, 128}.  q, k_cache / v_cache, out, scale, tp_batch, the
+ * second segment, gates, window (which may be shorter than N) and ALiBi mean
+ * what they mean above; k_tree, v_tree, anc and qkv must be NULL and f32_rows
+ * 0 (else VNX_ERR_UNSUPPORTED); the other fields are not read. */
+int vnx_chain_attn(const vnx_tree_attn_args* args, void* stream);
+
 /* The launch shape vnx_tree_attn uses: key splits, query groups (of at most
  * 64 rows for d = 64, 32 for d = 128) and keys per split. */
 int vnx_tree_attn_plan(int B, int H, int Hkv, int N, int Tp, int d, int* splits, int* groups,

@@ -29,7 +29,8 @@ same keys either way.
 Kernels of libvnx_hip.so (gfx950) on the decode and verify forwards:
 - attention of the new rows over the cache, all three TriSparse paths
   (vnx_tree_attn with per-row prefix lengths; RoPE and the cache write of
-  the new rows inside the call for bf16 verify-size forwards);
+  the new rows inside the call for bf16 verify-size forwards; vnx_chain_attn
+  for more rows than a tree call takes: prefill);
 - the target's verify-size projections and SwiGLU FFNs on vnx_gemm_bf16
   (RMSNorm staged into the q|k|v and gate-up products, the residual add in
   the output and down products' epilogues, the first layer's token
@@ -39,7 +40,7 @@ Kernels of libvnx_hip.so (gfx950) on the decode and verify forwards:
   SwiGLU / residual forms) and the verify-pass LM head (vnx_lm_head).
 Prefill-size forwards (more rows than one verify round) run their dense
 products on PyTorch-ROCm (hipBLASLt / rocBLAS); the attention of every
-forward runs on vnx_tree_attn where the head size allows it.
+forward runs on vnx_tree_attn / vnx_chain_attn where the head size allows it.
 """
 from __future__ import annotations
 
@@ -719,7 +720,7 @@ class CometSparkGPU:
         return w
 
     def _tree_call(self, q, kc, vc, cstr, tree_k, tree_v, tstr, anc, B, H, Hkv, Tp, n, d, tp, follows, out,
-                   seg2=None, gates=None, qkv=None, out_sb=None, alibi_max=1024):
+                   seg2=None, gates=None, qkv=None):
         a = _lib.TreeAttnArgs()
         if qkv is not None:
             # queries from the q|k|v rows, RoPE and the cache write in the kernel
@@ -735,12 +736,12 @@ class CometSparkGPU:
         a.f32_rows = int(self.f32_rows)
         # output rows in (B, n, H, d) order: the proj input layout
         a.out = out.data_ptr(); a.out_dtype = _lib.DTYPE_CODES[out.dtype]
-        a.out_strides[:] = [n * H * d if out_sb is None else out_sb, d, H * d]
+        a.out_strides[:] = [n * H * d, d, H * d]
         a.B, a.H, a.Hkv, a.Tp, a.N, a.d = B, H, Hkv, Tp, n, d
         a.scale = 1.0 / math.sqrt(d)
         a.window = self.cfg.window_size
         if self.cfg.use_alibi:
-            a.alibi_slopes = self.slopes.data_ptr(); a.alibi_max_keys = max(0, int(alibi_max))
+            a.alibi_slopes = self.slopes.data_ptr(); a.alibi_max_keys = 1024
             a.gates = gates.data_ptr()
         a.tp_batch = tp.data_ptr() if tp is not None else None
         a.tree_follows_prefix = 1 if follows else 0
@@ -776,28 +777,31 @@ class CometSparkGPU:
                         True, o, seg2=(Ly.gk, Ly.gv), gates=Ly.gates, qkv=qkv)
         return o
 
-    def _attn_kernel_chunked(self, q, li, lens, n, Tmax):
+    def _attn_chain(self, q, li, lens, n, Tmax):
         """bf16 forwards of more rows than one vnx_tree_attn call takes
-        (prefill): the n new rows (already in the cache) in chunks of at
-        most min(64, window) queries, chunk [c0, c1) seeing each row's
-        lens[b] + c0 prefix rows and its own rows under the chain mask.  The
-        ALiBi path keeps the whole call's rule (lens[b] + n <= 1024,
-        tri_sparse_attn.py:600-607): a chunk passes 1024 - (n - c1) as its
-        key limit.  q (B, H, n, d) bf16."""
+        (prefill): vnx_chain_attn over the cache, which already holds the n
+        new rows, all paths in one launch.  q (B, H, n, d) bf16."""
         cfg = self.cfg
         B, H, d = self.B, cfg.n_head, cfg.head_dim
         kc, vc = self.kc[li], self.vc[li]
         Ly = self.layers[li]
         o = torch.empty((B * n, H * d), dtype=self.act_dtype, device=self.dev)
-        cstr = list(kc.stride()[:3])
-        step = min(64, cfg.window_size) if cfg.window_size > 0 else 64
-        for c0 in range(0, n, step):
-            c1 = min(n, c0 + step)
-            m = c1 - c0
-            lens_c = lens + c0 if c0 else lens
-            self._tree_call(q[:, :, c0:c1], kc, vc, cstr, kc, vc, cstr, self._chain_words(m), B, H, cfg.n_kv_head,
-                            Tmax + c0, m, d, lens_c, True, o[c0:], seg2=(Ly.gk, Ly.gv), gates=Ly.gates,
-                            out_sb=n * H * d, alibi_max=1024 - (n - c1))
+        a = _lib.TreeAttnArgs()
+        a.q = q.data_ptr(); a.q_strides[:] = list(q.stride()[:3])
+        a.k_cache = kc.data_ptr(); a.v_cache = vc.data_ptr(); a.cache_strides[:] = list(kc.stride()[:3])
+        # output rows in (B, n, H, d) order: the proj input layout
+        a.out = o.data_ptr(); a.out_dtype = _lib.DTYPE_CODES[o.dtype]; a.out_strides[:] = [n * H * d, d, H * d]
+        a.B, a.H, a.Hkv, a.Tp, a.N, a.d = B, H, cfg.n_kv_head, Tmax, n, d
+        a.scale = 1.0 / math.sqrt(d)
+        a.window = cfg.window_size
+        a.tp_batch = lens.data_ptr()
+        a.gates = Ly.gates.data_ptr()
+        if cfg.use_alibi:
+            a.alibi_slopes = self.slopes.data_ptr(); a.alibi_max_keys = 1024
+        a.k_seg2 = Ly.gk.data_ptr(); a.v_seg2 = Ly.gv.data_ptr()
+        a.seg2_strides[:] = [0, Ly.gk.stride(1), Ly.gk.stride(2)]
+        a.T2 = Ly.gk.shape[2]
+        _lib.check(self.hip._L.vnx_chain_attn(ctypes.byref(a), self._st()), "chain_attn")
         return o
 
     def _attn_torch(self, q, li, lens, n, Tmax):
@@ -995,8 +999,8 @@ class CometSparkGPU:
         else:
             x = torch.empty((M, D), dtype=torch.float32, device=self.dev)                # fp32 residual stream
         use_kernel = self.kernel_attention and (self.f32_rows or (n <= 64 and n <= cfg.window_size))
-        # longer bf16 forwards (prefill): the same kernel over query chunks
-        chunked = self.kernel_attention and not use_kernel
+        # longer bf16 forwards (prefill): one vnx_chain_attn call
+        chain = self.kernel_attention and not use_kernel
         pending = None
         for li, L in enumerate(self.layers):
             # verify-size bf16 forwards: the norms and the residual adds live in
@@ -1056,8 +1060,8 @@ class CometSparkGPU:
                 return None                                # every layer's new cache rows are written
             if use_kernel:
                 o = self._attn_kernel(q, li, lens, n, Tmax, qkv=attn_qkv)
-            elif chunked:
-                o = self._attn_kernel_chunked(q, li, lens, n, Tmax)
+            elif chain:
+                o = self._attn_chain(q, li, lens, n, Tmax)
             else:
                 o = self._attn_torch(q, li, lens, n, Tmax).permute(0, 2, 1, 3).reshape(M, H * d)
                 o = o.to(self.act_dtype).contiguous()
