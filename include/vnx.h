@@ -810,6 +810,21 @@ int vnx_expert_gemm_bf16(const void* x, int64_t ldx, int64_t sxb, const void* w_
                          int32_t* rows, int32_t* counts, int32_t* slots, void* y, int y_dtype, int64_t ldy,
                          int64_t syb, void* stream);
 
+/* The same products for any M (prefill): X_z[j] = x[z*sxb + rows[z*M + j]*ldx]
+ * (rows NULL: row j), j < counts[z], with the lists vnx_mod_lists wrote; comb
+ * (VNX_EPI_SWIGLU only) weights row j by comb[row*ldc + z].  total_rows: an
+ * upper bound of the sum of counts (0: experts * M), which sizes the launch.
+ *
+ * vnx_mod_lists: L_z = { m < M : comb[m*ldc + z] != 0 } ascending, as rows[z*M
+ * + j] = l_j, counts[z] = n_z and slots[m*experts + z] = j for m = l_j, else
+ * -1. */
+int vnx_mod_lists(const float* comb, int64_t ldc, int64_t M, int experts, int32_t* rows, int32_t* counts,
+                  int32_t* slots, void* stream);
+int vnx_expert_gemm_bf16_rows(const void* x, int64_t ldx, int64_t sxb, const void* w_packed, int64_t swb, int64_t M,
+                              int64_t N, int64_t K, int experts, int epilogue, const float* comb, int64_t ldc,
+                              const int32_t* rows, const int32_t* counts, int64_t total_rows, void* y, int y_dtype,
+                              int64_t ldy, int64_t syb, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -167,6 +167,9 @@ SIGNATURES.update({
                               _c_i64, _vp]),
     "vnx_sum_experts": (_int, [_vp, _int, _c_i64, _int, _c_i64, _vp, _vp]),
     "vnx_sum_expert_rows": (_int, [_vp, _int, _c_i64, _c_i64, _vp, _c_i64, _int, _c_i64, _vp, _c_i64, _int, _vp]),
+    "vnx_mod_lists": (_int, [_vp, _c_i64, _c_i64, _int, _vp, _vp, _vp, _vp]),
+    "vnx_expert_gemm_bf16_rows": (_int, [_vp, _c_i64, _c_i64, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _int, _int, _vp,
+                                         _c_i64, _vp, _vp, _c_i64, _vp, _int, _c_i64, _c_i64, _vp]),
     "vnx_expert_gemm_bf16": (_int, [_vp, _c_i64, _c_i64, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _int, _int, _vp,
                                     _c_i64, _int, _vp, _vp, _vp, _vp, _int, _c_i64, _c_i64, _vp]),
 })

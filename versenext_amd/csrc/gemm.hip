@@ -1,4 +1,5 @@
-// Skinny bf16 GEMM for the verify forward (vnx_gemm_bf16): Y = X . W^T for
+// Skinny bf16 GEMM for the verify forward (vnx_gemm_bf16; products of many
+// output tiles go to wgemm.hip): Y = X . W^T for
 // the M <= a few hundred token rows of one speculative round (batch x (k+1)),
 // X (M, K) bf16 activations, W (N, K) bf16 (the nn.Linear layout, packed once
 // by vnx_pack_bf16), fp32 accumulation.  This is the Linear of the target's
@@ -28,17 +29,11 @@
 // ...), whose L2 then serves that group's W rows to all of them.
 #include <stdlib.h>
 
-#include "vnx_internal.h"
+#include "gemm_tiles.h"
 
 namespace vnx {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-constexpr int kVgChunk = 64;  // K per chunk
-constexpr int kVgXcds = 8;    // XCDs the dispatcher deals workgroups over
-constexpr int kVgRowB = 128;  // bytes of one staged X row (64 bf16)
 constexpr int kVgNormMaxK = 2048;  // NX: K of the normalized rows (norm weight staged in LDS)
 
 struct VgParams {
@@ -62,45 +57,6 @@ struct VgParams {
   float emb_scale;
   float* xout;
 };
-
-
-
-template <int OT>
-__device__ __forceinline__ void vg_store(char* y, int64_t off, float v) {
-  if constexpr (OT == 0) {
-    reinterpret_cast<float*>(y)[off] = v;
-  } else if constexpr (OT == 1) {
-    reinterpret_cast<__bf16*>(y)[off] = static_cast<__bf16>(v);
-  } else {
-    reinterpret_cast<_Float16*>(y)[off] = static_cast<_Float16>(v);
-  }
-}
-
-// Eight consecutive outputs of type OT from fp32 (16 bytes for bf16 / fp16,
-// 32 for fp32).
-template <int OT>
-__device__ __forceinline__ void vg_store8(char* y, int64_t off, const float (&v)[8]) {
-  if constexpr (OT == 0) {
-    float* d = reinterpret_cast<float*>(y) + off;
-    *reinterpret_cast<f32x4*>(d) = f32x4{v[0], v[1], v[2], v[3]};
-    *reinterpret_cast<f32x4*>(d + 4) = f32x4{v[4], v[5], v[6], v[7]};
-  } else if constexpr (OT == 1) {
-    __bf16 t[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) t[e] = static_cast<__bf16>(v[e]);
-    *reinterpret_cast<u32x4*>(reinterpret_cast<__bf16*>(y) + off) = __builtin_bit_cast(u32x4, t);
-  } else {
-    _Float16 t[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) t[e] = static_cast<_Float16>(v[e]);
-    *reinterpret_cast<u32x4*>(reinterpret_cast<_Float16*>(y) + off) = __builtin_bit_cast(u32x4, t);
-  }
-}
-
-__device__ __forceinline__ bf16x8 as_b8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
-
-// LDS byte offset of 16-byte column c16 (0..7) of staged row r (0..31).
-__device__ __forceinline__ int xs_off(int r, int c16) { return r * kVgRowB + ((c16 ^ ((r >> 1) & 7)) << 4); }
 
 // EPI 0: y[m, n] = acc.  EPI 1 (SwiGLU): W rows come in blocks of 32, the
 // first 16 the gate rows and the last 16 the up rows of hidden units
@@ -825,6 +781,13 @@ int vnx_gemm_bf16(const void* x, int64_t ldx, int64_t sxb, const void* w_packed,
   if (K % kVgChunk || ldx % 8 || sxb % 8 || swb % 8 || !aligned16(x) || !aligned16(w_packed))
     return VNX_ERR_UNSUPPORTED;
   if (M >= INT32_MAX || N >= INT32_MAX || K >= INT32_MAX || batch > 65535) return VNX_ERR_UNSUPPORTED;
+  if ((M + 31) / 32 * ((N + 31) / 32) * batch >= kWgMinTiles) {
+    WgParams p{};
+    p.x = static_cast<const uint16_t*>(x); p.w = static_cast<const uint16_t*>(w_packed); p.y = y; p.comb = comb;
+    p.ldx = ldx; p.sxb = sxb; p.swb = swb; p.ldy = ldy; p.syb = syb; p.ldc = ldc;
+    p.M = (int)M; p.N = (int)N; p.K = (int)K; p.batch = batch;
+    return wg_run(p, epilogue, y_dtype, static_cast<hipStream_t>(stream));
+  }
   VgParams p{};
   p.x = static_cast<const uint16_t*>(x); p.w = static_cast<const uint16_t*>(w_packed); p.y = y; p.comb = comb;
   p.ldx = ldx; p.sxb = sxb; p.swb = swb; p.ldy = ldy; p.syb = syb; p.ldc = ldc;
@@ -881,6 +844,13 @@ int vnx_gemm_bf16_residual(const void* x, int64_t ldx, const void* w_packed, int
   if (M == 0 || N == 0) return VNX_OK;
   if (K % kVgChunk || ldx % 8 || !aligned16(x) || !aligned16(w_packed)) return VNX_ERR_UNSUPPORTED;
   if (M >= INT32_MAX || N >= INT32_MAX || K >= INT32_MAX) return VNX_ERR_UNSUPPORTED;
+  if ((M + 31) / 32 * ((N + 31) / 32) >= kWgMinTiles) {
+    WgParams p{};
+    p.x = static_cast<const uint16_t*>(x); p.w = static_cast<const uint16_t*>(w_packed); p.y = res;
+    p.ldx = ldx; p.ldy = ldr;
+    p.M = (int)M; p.N = (int)N; p.K = (int)K; p.batch = 1;
+    return wg_run(p, 3, VNX_F32, static_cast<hipStream_t>(stream));
+  }
   VgParams p{};
   p.x = static_cast<const uint16_t*>(x); p.w = static_cast<const uint16_t*>(w_packed); p.y = res;
   p.ldx = ldx; p.ldy = ldr;

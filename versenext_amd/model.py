@@ -38,9 +38,11 @@ Kernels of libvnx_hip.so (gfx950) on the decode and verify forwards:
   (vnx_mod_route_x) and the routed expert products (vnx_expert_gemm_bf16);
 - the INT4 group-128 draft GEMVs (vnx_gemv_w4 and its fused RMSNorm / RoPE /
   SwiGLU / residual forms) and the verify-pass LM head (vnx_lm_head).
-Prefill-size forwards (more rows than one verify round) run their dense
-products on PyTorch-ROCm (hipBLASLt / rocBLAS); the attention of every
-forward runs on vnx_tree_attn / vnx_chain_attn where the head size allows it.
+Prefill-size forwards (more rows than one verify round) take the same calls
+with the norms apart (vnx_rmsnorm) and, for the MoD layers, the row lists
+built first (vnx_mod_lists, vnx_expert_gemm_bf16_rows); INT4 models run their
+prefill's dense products on PyTorch-ROCm.  The attention of every forward
+runs on vnx_tree_attn / vnx_chain_attn where the head size allows it.
 """
 from __future__ import annotations
 
@@ -358,8 +360,7 @@ class _Linear:
                                                                .cuda_stream)), "pack_w4_tiles")
         else:
             self.wd = w.to(dtype).contiguous()
-            # verify-size products (M <= GEMM_MAX_M) run vnx_gemm_bf16 on a
-            # packed copy; for a fused [gate; up] weight its rows are
+            # the products run vnx_gemm_bf16 on a packed copy; for a fused [gate; up] weight its rows are
             # interleaved in blocks of 16 gate + 16 up rows first (the
             # SwiGLU epilogue's order)
             if dtype == torch.bfloat16 and self.K % 64 == 0:
@@ -376,16 +377,17 @@ class _Linear:
                            "pack_bf16")
 
 
+    # rows up to which the norms are staged inside the products (gemm_norm)
     GEMM_MAX_M = 256
     # rows from which an INT4 weight also keeps the tiled copy (the LM head)
     TILES_MIN_N = 32768
 
     def gemm(self, x: torch.Tensor, epilogue: int = 0, out_dtype=None) -> Optional[torch.Tensor]:
-        """vnx_gemm_bf16 of the packed weight for x (M <= GEMM_MAX_M, bf16
-        rows): (M, N), or (M, N/2) with the SwiGLU epilogue; None when this
-        weight or x does not qualify."""
+        """vnx_gemm_bf16 of the packed weight for x (bf16 rows): (M, N), or
+        (M, N/2) with the SwiGLU epilogue; None when this weight or x does
+        not qualify."""
         M = x.shape[0]
-        if self.wp is None or M > self.GEMM_MAX_M or x.dtype != torch.bfloat16 or x.stride(1) != 1:
+        if self.wp is None or x.dtype != torch.bfloat16 or x.stride(1) != 1:
             return None
         if epilogue and not self.swiglu:
             return None
@@ -437,7 +439,7 @@ class _Linear:
         """res (M, N) fp32 += x . W^T (vnx_gemm_bf16_residual); False (nothing
         done) when this weight or x does not qualify."""
         M = x.shape[0]
-        if self.wp is None or M > self.GEMM_MAX_M or x.dtype != torch.bfloat16 or x.stride(1) != 1:
+        if self.wp is None or x.dtype != torch.bfloat16 or x.stride(1) != 1:
             return False
         _lib.check(self.hip._L.vnx_gemm_bf16_residual(
             ctypes.c_void_p(x.data_ptr()), x.stride(0), ctypes.c_void_p(self.wp.data_ptr()), M, self.N, self.K,
@@ -840,47 +842,67 @@ class CometSparkGPU:
             res = res + torch.where(use_c, Ly.gates[2] * out_c, torch.zeros_like(out_c))
         return res
 
-    def _mod_fused(self, L: _Layer, x: torch.Tensor) -> None:
-        """The MoD FFN of a verify-size forward with norm2 and the residual
-        add fused: x (M, D) fp32 residual stream += MoD(RMSNorm(x) * norm2).
-        vnx_mod_route_x normalizes, routes and writes the experts' bf16 input
-        rows; vnx_expert_gemm_bf16 runs each expert on its routed rows only
-        (gate|up with SwiGLU and routing weight fused, then down on the compact
-        rows); vnx_sum_expert_rows adds each row's experts into x."""
+    # rows routed at a time: bounds the experts' compact buffers (M rows of
+    # 2,688 + 1,024 bf16 per expert) and keeps every launch in range
+    MOD_ROWS = 32768
+
+    def _mod_routed(self, L: _Layer, h: torch.Tensor, norm_w: Optional[torch.Tensor], out: torch.Tensor,
+                    accumulate: bool) -> None:
+        """The MoD FFN of fp32 rows h (M, D) (of RMSNorm(h) * norm_w when
+        norm_w is given), written to out (M, D) fp32 or added into it (out may
+        be h).  vnx_mod_route_x routes and writes the experts' bf16 input
+        rows; vnx_expert_gemm_bf16 (up to 256 rows, the lists built in the
+        call) or vnx_mod_lists + vnx_expert_gemm_bf16_rows run each expert on
+        its routed rows only (gate|up with SwiGLU and routing weight fused,
+        then down on the compact rows); vnx_sum_expert_rows adds each row's
+        experts."""
         cfg = self.cfg
         P, E, k = cfg.num_dense_parts, cfg.num_experts_per_part, cfg.top_k
         PE, He, D = P * E, cfg.expert_hidden_eff, cfg.dim
-        M = x.shape[0]
-        P_ = ctypes.c_void_p
+        if h.shape[0] > self.MOD_ROWS:
+            for m0 in range(0, h.shape[0], self.MOD_ROWS):
+                m1 = min(h.shape[0], m0 + self.MOD_ROWS)
+                self._mod_routed(L, h[m0:m1], norm_w, out[m0:m1], accumulate)
+            return
+        M = h.shape[0]
+        P_ = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else None
         L_ = self.hip._L
         comb = torch.empty((M, PE), dtype=torch.float32, device=self.dev)
         wr = L.ffn["route"]                                                        # (P + PE, D) fp32
         xh = torch.empty((M, D), dtype=torch.bfloat16, device=self.dev)
-        _lib.check(L_.vnx_mod_route_x(P_(x.data_ptr()), x.stride(0), P_(L.norm2.data_ptr()), float(cfg.eps),
-                                      P_(wr.data_ptr()), wr.stride(0), M, D, P, E, k, P_(comb.data_ptr()), PE,
-                                      P_(xh.data_ptr()), D, 0, 1, self._st()), "mod_route_x")
+        _lib.check(L_.vnx_mod_route_x(P_(h), h.stride(0), P_(norm_w), float(cfg.eps) if norm_w is not None else 0.0,
+                                      P_(wr), wr.stride(0), M, D, P, E, k, P_(comb), PE, P_(xh), D, 0, 1,
+                                      self._st()), "mod_route_x")
         rows = torch.empty((PE, M), dtype=torch.int32, device=self.dev)
         counts = torch.empty((PE,), dtype=torch.int32, device=self.dev)
         slots = torch.empty((M, PE), dtype=torch.int32, device=self.dev)
         w1p, w2p = L.ffn["w1p"], L.ffn["w2p"]
         act = torch.empty((PE, M, He), dtype=torch.bfloat16, device=self.dev)
-        _lib.check(L_.vnx_expert_gemm_bf16(
-            P_(xh.data_ptr()), D, 0, P_(w1p.data_ptr()), w1p.stride(0), M, 2 * He, D, PE, _lib.VNX_EPI_SWIGLU,
-            P_(comb.data_ptr()), PE, 1, P_(rows.data_ptr()), P_(counts.data_ptr()), P_(slots.data_ptr()),
-            P_(act.data_ptr()), _lib.VNX_BF16, He, M * He, self._st()), "expert_gemm w1")
         y = torch.empty((PE, M, D), dtype=torch.bfloat16, device=self.dev)
-        _lib.check(L_.vnx_expert_gemm_bf16(
-            P_(act.data_ptr()), He, M * He, P_(w2p.data_ptr()), w2p.stride(0), M, D, He, PE, _lib.VNX_EPI_NONE,
-            None, 0, 0, None, P_(counts.data_ptr()), None, P_(y.data_ptr()), _lib.VNX_BF16, D, M * D,
-            self._st()), "expert_gemm w2")
-        _lib.check(L_.vnx_sum_expert_rows(P_(y.data_ptr()), _lib.VNX_BF16, D, M * D, P_(slots.data_ptr()), M, PE,
-                                          D, P_(x.data_ptr()), x.stride(0), 1, self._st()), "sum_expert_rows")
+        bf = _lib.VNX_BF16
+        if M <= 256:
+            _lib.check(L_.vnx_expert_gemm_bf16(
+                P_(xh), D, 0, P_(w1p), w1p.stride(0), M, 2 * He, D, PE, _lib.VNX_EPI_SWIGLU, P_(comb), PE, 1,
+                P_(rows), P_(counts), P_(slots), P_(act), bf, He, M * He, self._st()), "expert_gemm w1")
+            _lib.check(L_.vnx_expert_gemm_bf16(
+                P_(act), He, M * He, P_(w2p), w2p.stride(0), M, D, He, PE, _lib.VNX_EPI_NONE, None, 0, 0, None,
+                P_(counts), None, P_(y), bf, D, M * D, self._st()), "expert_gemm w2")
+        else:
+            total = M * P * min(k, E)
+            _lib.check(L_.vnx_mod_lists(P_(comb), PE, M, PE, P_(rows), P_(counts), P_(slots), self._st()),
+                       "mod_lists")
+            _lib.check(L_.vnx_expert_gemm_bf16_rows(
+                P_(xh), D, 0, P_(w1p), w1p.stride(0), M, 2 * He, D, PE, _lib.VNX_EPI_SWIGLU, P_(comb), PE, P_(rows),
+                P_(counts), total, P_(act), bf, He, M * He, self._st()), "expert_gemm w1")
+            _lib.check(L_.vnx_expert_gemm_bf16_rows(
+                P_(act), He, M * He, P_(w2p), w2p.stride(0), M, D, He, PE, _lib.VNX_EPI_NONE, None, 0, None,
+                P_(counts), total, P_(y), bf, D, M * D, self._st()), "expert_gemm w2")
+        _lib.check(L_.vnx_sum_expert_rows(P_(y), bf, D, M * D, P_(slots), M, PE, D, P_(out), out.stride(0),
+                                          int(accumulate), self._st()), "sum_expert_rows")
 
     def _mod(self, L: _Layer, h: torch.Tensor) -> torch.Tensor:
-        """MoD FFN on (M, D) fp32 normalized rows.  Verify-size forwards (bf16,
-        M <= 256): the routing weights (vnx_mod_route_x), each expert's
-        products on its routed rows only (vnx_expert_gemm_bf16) and the sum
-        over each row's experts (vnx_sum_expert_rows).  Otherwise fp32 routing
+        """MoD FFN on (M, D) fp32 normalized rows.  bf16 models with packed
+        experts: the routed products (_mod_routed).  Otherwise fp32 routing
         logits in one product and the routing weights (vnx_mod_route); every
         expert's gate|up and down as batched products over the P*E experts,
         with the weighted activations in between (vnx_mod_swiglu; zero for
@@ -891,35 +913,12 @@ class CometSparkGPU:
         M = h.shape[0]
         P_ = ctypes.c_void_p
         L_ = self.hip._L
+        out = torch.empty((M, D), dtype=torch.float32, device=self.dev)
+        if P + PE <= 32 and "w1p" in L.ffn:
+            self._mod_routed(L, h, None, out, False)
+            return out
         comb = torch.empty((M, PE), dtype=torch.float32, device=self.dev)
         wr = L.ffn["route"]                                                        # (P + PE, D) fp32
-        if P + PE <= 32 and "w1p" in L.ffn and M <= 256:
-            # routed products: router + routing rule (one bf16 copy of h),
-            # then each expert's gate|up with the SwiGLU and routing weight
-            # fused and its down product on its own rows only, then the sum
-            # over each row's experts
-            xh = torch.empty((M, D), dtype=torch.bfloat16, device=self.dev)
-            _lib.check(L_.vnx_mod_route_x(P_(h.data_ptr()), h.stride(0), None, 0.0, P_(wr.data_ptr()), wr.stride(0), M,
-                                          D, P, E, k, P_(comb.data_ptr()), PE, P_(xh.data_ptr()), D, 0, 1,
-                                          self._st()), "mod_route_x")
-            rows = torch.empty((PE, M), dtype=torch.int32, device=self.dev)
-            counts = torch.empty((PE,), dtype=torch.int32, device=self.dev)
-            slots = torch.empty((M, PE), dtype=torch.int32, device=self.dev)
-            w1p, w2p = L.ffn["w1p"], L.ffn["w2p"]
-            act = torch.empty((PE, M, He), dtype=torch.bfloat16, device=self.dev)
-            _lib.check(L_.vnx_expert_gemm_bf16(
-                P_(xh.data_ptr()), D, 0, P_(w1p.data_ptr()), w1p.stride(0), M, 2 * He, D, PE, _lib.VNX_EPI_SWIGLU,
-                P_(comb.data_ptr()), PE, 1, P_(rows.data_ptr()), P_(counts.data_ptr()), P_(slots.data_ptr()),
-                P_(act.data_ptr()), _lib.VNX_BF16, He, M * He, self._st()), "expert_gemm w1")
-            y = torch.empty((PE, M, D), dtype=torch.bfloat16, device=self.dev)
-            _lib.check(L_.vnx_expert_gemm_bf16(
-                P_(act.data_ptr()), He, M * He, P_(w2p.data_ptr()), w2p.stride(0), M, D, He, PE, _lib.VNX_EPI_NONE,
-                None, 0, 0, None, P_(counts.data_ptr()), None, P_(y.data_ptr()), _lib.VNX_BF16, D, M * D,
-                self._st()), "expert_gemm w2")
-            out = torch.empty((M, D), dtype=torch.float32, device=self.dev)
-            _lib.check(L_.vnx_sum_expert_rows(P_(y.data_ptr()), _lib.VNX_BF16, D, M * D, P_(slots.data_ptr()), M, PE,
-                                              D, P_(out.data_ptr()), D, 0, self._st()), "sum_expert_rows")
-            return out
         if P + PE <= 32 and self.dtype == torch.bfloat16:
             # router products and routing rule in one launch, which also
             # writes the experts' bf16 input rows (one copy per expert)
@@ -938,7 +937,6 @@ class CometSparkGPU:
                                      P_(comb.data_ptr()), PE, M, PE, He, P_(act.data_ptr()),
                                      _lib.DTYPE_CODES[act.dtype], He, M * He, self._st()), "mod_swiglu")
         y = torch.matmul(act, L.ffn["w2"])                                        # (PE, M, D)
-        out = torch.empty((M, D), dtype=torch.float32, device=self.dev)
         _lib.check(L_.vnx_sum_experts(P_(y.data_ptr()), _lib.DTYPE_CODES[y.dtype], M, PE, D, P_(out.data_ptr()),
                                       self._st()), "sum_experts")
         return out
@@ -1003,14 +1001,18 @@ class CometSparkGPU:
         chain = self.kernel_attention and not use_kernel
         pending = None
         for li, L in enumerate(self.layers):
-            # verify-size bf16 forwards: the norms and the residual adds live in
-            # the projections (vnx_gemm_bf16_norm / _residual) and in the MoD
-            # routing / expert sum, so x is the up-to-date residual stream
-            fused = (L.wqkv.wp is not None and L.proj.wp is not None and M <= _Linear.GEMM_MAX_M
-                     and self.dtype == torch.bfloat16 and D <= 2048
+            # bf16 forwards: the residual adds live in the projections
+            # (vnx_gemm_bf16_residual) and in the MoD expert sum, so x is the
+            # up-to-date residual stream; for verify-size rows the norms live
+            # in the projections and the MoD routing too (vnx_gemm_bf16_norm;
+            # staging fp32 rows for every 32 of them again would cost a
+            # prefill-size product more than the norm's own launch)
+            fused = (L.wqkv.wp is not None and L.proj.wp is not None
+                     and self.dtype == torch.bfloat16
                      and pending is None
-                     and ("w1p" in L.ffn if L.kind == "mod" else
+                     and ("w1p" in L.ffn and len(L.ffn["route"]) <= 32 if L.kind == "mod" else
                           (L.ffn["gu"].wp is not None and L.ffn["gu"].swiglu and L.ffn["down"].wp is not None)))
+            norm_in = fused and M <= _Linear.GEMM_MAX_M and D <= 2048
             # the INT4 draft's decode: the same fusions on its GEMVs
             qfused = (not fused and L.kind == "trisparse" and L.wqkv.wq_rope is not None and L.proj.int4
                       and L.ffn["gu"].int4 and L.ffn["gu"].swiglu and L.ffn["down"].int4 and M <= 64
@@ -1026,13 +1028,13 @@ class CometSparkGPU:
             if li == 0 and qfused and self.embed_fold and L.wqkv.rope_kv_embed(
                     tok, self.emb, self.emb_scale, x, rk, L.norm1, cfg.eps):
                 done = True                                # embedding, norm, q|k|v, RoPE, cache rows: one call
-            elif li == 0 and fused and self.embed_fold and (qkv := L.wqkv.gemm_norm_embed(
+            elif li == 0 and norm_in and self.embed_fold and (qkv := L.wqkv.gemm_norm_embed(
                     tok, self.emb, self.emb_scale, x, L.norm1, cfg.eps)) is not None:
                 pass                                       # embedding, norm and q|k|v: one call
             elif li == 0:
                 h = torch.empty((M, D), dtype=self.act_dtype, device=self.dev)
                 self._embed_rms(tok, L.norm1, x, h)        # token embedding folded into the first norm
-            elif fused:
+            elif norm_in:
                 qkv = L.wqkv.gemm_norm(x, L.norm1, cfg.eps)
             elif qfused:
                 done = L.wqkv.rope_kv(x, rk, L.norm1, cfg.eps)
@@ -1068,9 +1070,14 @@ class CometSparkGPU:
             if fused and L.proj.gemm_residual(o, x):
                 # x += proj(o); then the FFN of RMSNorm(x) * norm2, added into x
                 if L.kind == "mod":
-                    self._mod_fused(L, x)
+                    self._mod_routed(L, x, L.norm2, x, True)
                 else:
-                    act = L.ffn["gu"].gemm_norm(x, L.norm2, cfg.eps, epilogue=_lib.VNX_EPI_SWIGLU)
+                    if norm_in:
+                        act = L.ffn["gu"].gemm_norm(x, L.norm2, cfg.eps, epilogue=_lib.VNX_EPI_SWIGLU)
+                    else:
+                        h = torch.empty((M, D), dtype=torch.bfloat16, device=self.dev)
+                        self._rms(x, None, L.norm2, h)
+                        act = L.ffn["gu"].gemm(h, epilogue=_lib.VNX_EPI_SWIGLU)
                     if act is None or not L.ffn["down"].gemm_residual(act, x):
                         raise RuntimeError("fused FFN path unavailable for this layer")
                 continue
