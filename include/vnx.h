@@ -307,7 +307,7 @@ typedef struct vnx_rope_kv_args {
  * Weight-only quantized GEMV / skinny GEMM (draft decode, tied LM head):
  * y (B, N) fp32, row pitch ldy = x (B, K) fp16 (row pitch ldx) . W^T with W
  * the dequantized (N, K) weight.  Matrix-core kernels (MFMA f16 -> f32); any
- * B (processed 32 columns at a time).  K must be a multiple of 128; x and
+ * B (up to 32 at a time, a tiled GEMM beyond).  K must be a multiple of 128; x and
  * each weight row must start 16-byte aligned (ldx % 8 == 0, ldw % 16 == 0).
  * Small N splits K over workgroups: the fp32 partials go to the workspace
  * (vnx_gemv_workspace bytes; no initialisation needed) and are added in a
@@ -400,6 +400,16 @@ int vnx_gemv_w4_residual(const void* x, int64_t ldx, const uint8_t* wq, int64_t 
 int vnx_gemv_w8(const void* x, int64_t ldx, const int8_t* wq, int64_t ldw, const float* scale,
                 int64_t B, int64_t N, int64_t K, float* y, int64_t ldy, void* workspace,
                 size_t workspace_bytes, void* stream);
+
+/* QuantizedLinear.forward whole (quantize.py:506-582): the products above with
+ * x in x_dtype, VNX_F16 or VNX_F32 (fp32 rows are rounded to fp16, nearest
+ * even, as they are read; 16-byte aligned, ldx % 4 == 0), and bias (N) fp32
+ * added to the finished sums (NULL: none). */
+int vnx_linear_w4(const void* x, int x_dtype, int64_t ldx, const uint8_t* wq, int64_t ldw, const void* scales,
+                  int scale_dtype, int64_t lds, int64_t B, int64_t N, int64_t K, int group, const float* bias,
+                  float* y, int64_t ldy, void* stream);
+int vnx_linear_w8(const void* x, int x_dtype, int64_t ldx, const int8_t* wq, int64_t ldw, const float* scale,
+                  int64_t B, int64_t N, int64_t K, const float* bias, float* y, int64_t ldy, void* stream);
 
 /* INT4 group-128 quantization on the device (the writer of the format above;
  * quantize_int4_g of the product's quant.py, restating the group variant of

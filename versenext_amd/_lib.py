@@ -87,6 +87,9 @@ SIGNATURES = {
                                     _vp, _c_i64, _vp]),
     "vnx_gemv_w8": (_int, [_vp, _c_i64, _vp, _c_i64, _vp, _c_i64, _c_i64, _c_i64, _vp, _c_i64,
                            _vp, _c_sz, _vp]),
+    "vnx_linear_w4": (_int, [_vp, _int, _c_i64, _vp, _c_i64, _vp, _int, _c_i64, _c_i64, _c_i64, _c_i64, _int, _vp, _vp,
+                             _c_i64, _vp]),
+    "vnx_linear_w8": (_int, [_vp, _int, _c_i64, _vp, _c_i64, _vp, _c_i64, _c_i64, _c_i64, _vp, _vp, _c_i64, _vp]),
     "vnx_dequant_w4": (_int, [_vp, _c_i64, _vp, _int, _c_i64, _c_i64, _c_i64, _int, _vp, _c_i64, _vp]),
     "vnx_dequant_w8": (_int, [_vp, _c_i64, _vp, _c_i64, _c_i64, _vp, _c_i64, _vp]),
     "vnx_sample_workspace": (_c_sz, [_c_i64, _c_i64]),

@@ -64,6 +64,8 @@ struct QGemvParams {
   const float* nw;     // NX: RMSNorm weight (K)
   float eps;
   int64_t row_off;     // batch row of x's first row (the launch's 32-row chunks)
+  const float* x32;    // fp32 rows, row pitch ldx, rounded to fp16 as they are staged (x unused), or NULL
+  const float* bias;   // (N), added to the finished fp32 sums, or NULL
   // NX 2: x rows are the token embedding, xf unused: row b is
   // emb[ids[b]] * emb_scale (bf16 table, ids clamped to [0, vocab)), and the
   // workgroups write those fp32 rows to xout (pitch ldx)
@@ -158,6 +160,34 @@ __device__ __forceinline__ u32x4 stage_perm_w4(u32x4 v) {
   return o;
 }
 
+// Eight fp32 values rounded to fp16 (nearest even), as torch's and numpy's
+// casts do.
+__device__ __forceinline__ u32x4 half8_bits(u32x4 lo, u32x4 hi) {
+  half8 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    o[e] = (_Float16)__builtin_bit_cast(float, (uint32_t)lo[e]);
+    o[4 + e] = (_Float16)__builtin_bit_cast(float, (uint32_t)hi[e]);
+  }
+  return __builtin_bit_cast(u32x4, o);
+}
+
+// x[b, k .. k + 8) as fp16 (fp32 rows rounded).
+__device__ __forceinline__ u32x4 load_x8(const QGemvParams& p, int64_t b, int64_t k) {
+  if (p.x32) {
+    const u32x4* src = reinterpret_cast<const u32x4*>(p.x32 + b * p.ldx + k);
+    return half8_bits(src[0], src[1]);
+  }
+  return *reinterpret_cast<const u32x4*>(p.x + b * p.ldx + k);
+}
+
+// v += bias[n0 .. n0 + 4) (columns past N repeat the last: not stored).
+__device__ __forceinline__ void add_bias4(const QGemvParams& p, int64_t n0, f32x4& v) {
+  if (!p.bias) return;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] += p.bias[min(n0 + j, p.N - 1)];
+}
+
 template <int BITS, int NC, int TPW>
 __global__ __launch_bounds__(kQNT) void k_qgemv(QGemvParams p) {
   constexpr int KS = 1024 / NC;                 // k per slice
@@ -192,7 +222,7 @@ __global__ __launch_bounds__(kQNT) void k_qgemv(QGemvParams p) {
     for (int idx = tid; idx < brows * (KS / 8); idx += kQNT) {
       const int b = idx / (KS / 8), c8 = idx % (KS / 8);
       u32x4 v = {0u, 0u, 0u, 0u};
-      if (b < p.B && c8 * 8 < ks) v = *reinterpret_cast<const u32x4*>(p.x + b * p.ldx + k0 + c8 * 8);
+      if (b < p.B && c8 * 8 < ks) v = load_x8(p, b, k0 + c8 * 8);
       if constexpr (BITS == 4) v = stage_perm_w4(v);
       *reinterpret_cast<u32x4*>(&xs[b * XS + c8 * 8]) = v;
     }
@@ -299,6 +329,7 @@ __global__ __launch_bounds__(kQNT) void k_qgemv(QGemvParams p) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[j] *= load_scale(p, min(n0 + j, p.N - 1), 0);
       }
+      add_bias4(p, n0, v);
       float* dst = out + b * ldo + n0;
       if (n0 + 4 <= p.N && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
         *reinterpret_cast<f32x4*>(dst) = v;
@@ -333,6 +364,7 @@ __global__ __launch_bounds__(kQNT) void k_qgemv(QGemvParams p) {
 // pass of a wave (1 where K has at most one group per wave, or TP 2).
 template <int BITS, int NC, int NW, int QE, int NX, int TP, int GP, bool SF16>
 __device__ __forceinline__ void qgemv_tile_body(const QGemvParams& p, char* smem, float* ssp_flat) {
+  constexpr bool NRM = NX == 1 || NX == 2;  // NX 3: fp32 rows rounded to fp16, no norm
   constexpr int WBYTES = BITS == 4 ? 16 : 32;
   constexpr int XR = NC * 16;            // staged batch rows
   constexpr int XP = kGK + kXPad;        // LDS row pitch (fp16)
@@ -341,7 +373,7 @@ __device__ __forceinline__ void qgemv_tile_body(const QGemvParams& p, char* smem
   constexpr size_t kXBytes = size_t(NW) * XR * XP * 2, kRBytes = size_t(NW) * TP * NC * 64 * 16;
   auto xs_all = reinterpret_cast<uint16_t(*)[XR * XP]>(smem);
   auto red = reinterpret_cast<f32x4(*)[TP][NC][64]>(smem);
-  auto ssp = reinterpret_cast<float(*)[NX ? XR : 1]>(ssp_flat);  // NX: per-wave sums of squares per row
+  auto ssp = reinterpret_cast<float(*)[NRM ? XR : 1]>(ssp_flat);  // NRM: per-wave sums of squares per row
   const int tid = threadIdx.x;
   const int wave = tid / VNX_WAVE, lane = tid % VNX_WAVE;
   const int m = lane % 16, kq = lane / 16;
@@ -377,9 +409,9 @@ __device__ __forceinline__ void qgemv_tile_body(const QGemvParams& p, char* smem
       }
     }
   }
-  float ss[NX ? XL : 1];  // NX: this lane's sums of squares, row (i*64 + lane) / 16
+  float ss[NRM ? XL : 1];  // NRM: this lane's sums of squares, row (i*64 + lane) / 16
 #pragma unroll
-  for (int i = 0; i < (NX ? XL : 1); ++i) ss[i] = 0.0f;
+  for (int i = 0; i < (NRM ? XL : 1); ++i) ss[i] = 0.0f;
   const uint16_t* erow[NX == 2 ? XL : 1];  // NX 2: embedding row of row (i*64 + lane) / 16
   if constexpr (NX == 2) {
 #pragma unroll
@@ -397,7 +429,7 @@ __device__ __forceinline__ void qgemv_tile_body(const QGemvParams& p, char* smem
     const bool second = g0 + NW < ngroups;
     uint32_t wv[GP][TP][WBYTES / 4];
     u32x4 xv[GP][XL][NX ? 2 : 1];
-    u32x4 nwv[GP][NX ? 2 : 1];
+    u32x4 nwv[GP][NRM ? 2 : 1];
     float sc[GP][TP][4];
 #pragma unroll
     for (int u = 0; u < GP; ++u) {
@@ -419,14 +451,14 @@ __device__ __forceinline__ void qgemv_tile_body(const QGemvParams& p, char* smem
         if constexpr (NX == 2) {
           xv[u][i][0] = *reinterpret_cast<const u32x4*>(erow[i] + k0 + m * 8);
         } else if constexpr (NX) {
-          const float* src = p.xf + (int64_t)min(b, (int)p.B - 1) * p.ldx + k0 + m * 8;
+          const float* src = (NX == 3 ? p.x32 : p.xf) + (int64_t)min(b, (int)p.B - 1) * p.ldx + k0 + m * 8;
           xv[u][i][0] = *reinterpret_cast<const u32x4*>(src);
           xv[u][i][1] = *reinterpret_cast<const u32x4*>(src + 4);
         } else {
           xv[u][i][0] = *reinterpret_cast<const u32x4*>(p.x + (int64_t)min(b, (int)p.B - 1) * p.ldx + k0 + m * 8);
         }
       }
-      if constexpr (NX) {
+      if constexpr (NRM) {
         nwv[u][0] = *reinterpret_cast<const u32x4*>(p.nw + k0 + m * 8);
         nwv[u][1] = *reinterpret_cast<const u32x4*>(p.nw + k0 + m * 8 + 4);
       }
@@ -446,7 +478,9 @@ __device__ __forceinline__ void qgemv_tile_body(const QGemvParams& p, char* smem
       for (int i = 0; i < XL; ++i) {
         const int b = (i * 64 + lane) / 16;
         u32x4 v;
-        if constexpr (NX) {
+        if constexpr (NX == 3) {
+          v = half8_bits(xv[u][i][0], xv[u][i][1]);
+        } else if constexpr (NX) {
           // fp16(x * w) of 8 columns; their squares into ss (counted once)
           f32x4 xa, xb;
           if constexpr (NX == 2) {
@@ -520,7 +554,7 @@ __device__ __forceinline__ void qgemv_tile_body(const QGemvParams& p, char* smem
     }
   }
 
-  if constexpr (NX) {
+  if constexpr (NRM) {
     // each row's sum over its 16 lanes (consecutive), one partial per wave
 #pragma unroll
     for (int i = 0; i < XL; ++i) {
@@ -555,7 +589,7 @@ __device__ __forceinline__ void qgemv_tile_body(const QGemvParams& p, char* smem
 #pragma unroll
     for (int j = 0; j < 4; ++j) v[j] *= load_scale_t<SF16>(p, min(n0 + j, p.N - 1), 0);
   }
-  if constexpr (NX) {
+  if constexpr (NRM) {
     float t = 0.0f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) t += ssp[w][b];
@@ -631,6 +665,7 @@ __device__ __forceinline__ void qgemv_tile_body(const QGemvParams& p, char* smem
     }
     return;
   }
+  add_bias4(p, n0, v);
   float* dst = p.y + b * p.ldy + n0;
   if (n0 + 4 <= p.N && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
     *reinterpret_cast<f32x4*>(dst) = v;
@@ -673,7 +708,7 @@ __global__ __launch_bounds__(kQNT) void k_qgemv_stream(QGemvParams p, int tiles_
   for (int idx = tid; idx < NC * 16 * KG * 16; idx += kQNT) {
     const int b = idx / (KG * 16), c8 = idx % (KG * 16);
     u32x4 v = {0u, 0u, 0u, 0u};
-    if (b < p.B) v = *reinterpret_cast<const u32x4*>(p.x + b * p.ldx + c8 * 8);
+    if (b < p.B) v = load_x8(p, b, c8 * 8);
     *reinterpret_cast<u32x4*>(&xs[b * XS + c8 * 8]) = stage_perm_w4(v);
   }
   __syncthreads();
@@ -740,12 +775,13 @@ __global__ __launch_bounds__(kQNT) void k_qgemv_stream(QGemvParams p, int tiles_
     if (tile >= t_hi) return;
     const int64_t n = tile * 16 + m;
     if (n >= p.N) return;
+    const float bv = p.bias ? p.bias[n] : 0.0f;
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int64_t b = c * 16 + 4 * kq + j;
-        if (b < p.B) p.y[b * p.ldy + n] = yacc[c][j];
+        if (b < p.B) p.y[b * p.ldy + n] = p.bias ? yacc[c][j] + bv : yacc[c][j];
       }
   };
   // RS slots: slot j holds tile ta + 4j; each slot is reloaded (tiles past
@@ -971,6 +1007,204 @@ __global__ void k_dequant(QGemvParams p, int bits, float* out, int64_t ldo) {
   out[n * ldo + k] = (float)q * s;
 }
 
+// ---------------------------------------------------------------------------
+// Many rows (a prompt through a quantized layer; qgemv_launch says from
+// where): the same product as a tiled
+// GEMM, the weight read and converted once per RT 32-row tiles of x instead
+// of once per 32 rows.  A workgroup (4 waves) owns 32 RT rows and WN 32-column
+// tiles; its waves are WN (one column tile each) x WK = 4 / WN (K splits,
+// 128-k chunks kw, kw + WK, ..., summed through LDS in split order).  x goes
+// through LDS (double-buffered, 16-byte units XOR-swizzled by row); a lane's
+// weights (column r = lane % 32, k = h * 64 + [0, 64) of the chunk, h = lane /
+// 32) go from memory to registers PD passes ahead and become fp16 operands
+// there, so v_mfma_f32_32x32x16_f16 has x as A and the weights as B and a
+// lane's 16 results share one weight row: its scale is one register.  SC 0:
+// one scale per row, applied to the finished sums; 1 / 2: fp16 / fp32 group
+// scales, applied per 128-k chunk.  XF: x is fp32, rounded to fp16 as it is
+// staged.  What bounds it: at 1,024 x 2,048 x 2,048 the weights' conversion and
+// the group scaling cost the vector units about as much as the products cost
+// the matrix cores, at two workgroups per CU; 21 us (32 passes of the narrow
+// kernel: 162 us).
+// ---------------------------------------------------------------------------
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+template <int BITS, int SC, int RT, int WN, bool XF>
+__global__ __launch_bounds__(256, 2) void k_qwgemm(QGemvParams p, int mt, int ng) {
+  constexpr int WK = 4 / WN;
+  constexpr int ROWS = 32 * RT;
+  constexpr int SLAB = ROWS * 256;               // one staged chunk: ROWS x 128 fp16
+  constexpr int PASS = WK * SLAB;
+  constexpr int RED = (WK - 1) * WN * RT * 4096; // K-split partial tiles
+  constexpr int SM = 2 * PASS > RED ? 2 * PASS : RED;
+  constexpr int NW = BITS == 4 ? 2 : 4;          // 16-byte weight loads per chunk
+  constexpr int NX = 2 * RT * WK;                // 16-byte x loads per thread and pass
+  constexpr int PD = 2;
+  __shared__ __attribute__((aligned(16))) char smem[SM];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wn = wave % WN, wk = wave / WN;
+  // tiles numbered (N group, row tile), cut into eight runs, one per XCD
+  const int total = mt * ng, run = (total + 7) / 8, at = blockIdx.x >> 3;
+  const int idx = (blockIdx.x & 7) * run + at;
+  if (at >= run || idx >= total) return;         // uniform over the workgroup
+  const int gi = idx / mt;
+  const int64_t m0 = (int64_t)(idx - gi * mt) * ROWS;
+  const int r = lane & 31, h = lane >> 5;
+  const int nch = (int)(p.K / kGK), npass = (nch + WK - 1) / WK;
+  const int64_t n = ((int64_t)gi * WN + wn) * 32 + r;
+  const int64_t nc = min(n, p.N - 1);            // columns past N re-read the last (not stored)
+
+  // x: thread tid takes rows tid / 16 + 16 q, 16-byte unit tid % 16
+  const int xr = tid >> 4, xu = tid & 15;
+  using XT = typename std::conditional<XF, float, uint16_t>::type;
+  const XT* xp[2 * RT];
+#pragma unroll
+  for (int q = 0; q < 2 * RT; ++q) {
+    const int64_t off = min(m0 + xr + 16 * q, p.B - 1) * p.ldx + xu * 8;
+    if constexpr (XF) xp[q] = p.x32 + off;
+    else xp[q] = p.x + off;
+  }
+  const uint8_t* wp = p.w + nc * p.ldw + h * (BITS == 4 ? 32 : 64);
+  constexpr int XW = XF ? 2 : 1;
+  auto load_x = [&](int ps, u32x4 (&v)[NX][XW]) {
+#pragma unroll
+    for (int j = 0; j < WK; ++j) {
+      const int c = min(ps * WK + j, nch - 1);
+#pragma unroll
+      for (int q = 0; q < 2 * RT; ++q)
+#pragma unroll
+        for (int e = 0; e < XW; ++e)
+          v[j * 2 * RT + q][e] = *reinterpret_cast<const u32x4*>(xp[q] + c * kGK + 4 * e);
+    }
+  };
+  auto stage_x = [&](int ps, const u32x4 (&v)[NX][XW]) {
+    char* buf = smem + (ps & 1) * PASS;
+#pragma unroll
+    for (int j = 0; j < WK; ++j)
+#pragma unroll
+      for (int q = 0; q < 2 * RT; ++q) {
+        const int row = xr + 16 * q;
+        u32x4 t;
+        if constexpr (XF) t = half8_bits(v[j * 2 * RT + q][0], v[j * 2 * RT + q][1]);
+        else t = v[j * 2 * RT + q][0];
+        if constexpr (BITS == 4) t = stage_perm_w4(t);
+        *reinterpret_cast<u32x4*>(buf + j * SLAB + row * 256 + ((xu ^ (row & 15)) << 4)) = t;
+      }
+  };
+  float sc[PD];
+  auto load_w = [&](int ps, u32x4 (&v)[NW], float& s) {
+    const int c = min(ps * WK + wk, nch - 1);
+#pragma unroll
+    for (int j = 0; j < NW; ++j)
+      v[j] = *reinterpret_cast<const u32x4*>(wp + (int64_t)c * (BITS == 4 ? 64 : 128) + 16 * j);
+    if constexpr (SC) s = load_scale_t<SC == 1>(p, nc, (unsigned)(c / p.gpg));
+  };
+
+  // Sums in three levels, a chunk's products, kMid chunks, the rest, so that
+  // a long K rounds no more than the narrow kernels' K split does.
+  constexpr int kMid = WK == 1 ? 8 : 4;
+  f32x16 acc[RT], mid[RT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[i][e] = mid[i][e] = 0.0f;
+  u32x4 xv[NX][XW], wv[PD][NW];
+  load_x(0, xv);
+  stage_x(0, xv);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int d = 0; d < PD; ++d) load_w(d, wv[d], sc[d]);
+  __builtin_amdgcn_sched_barrier(0);
+  load_x(1, xv);
+  __syncthreads();
+  for (int p0 = 0; p0 < npass; p0 += PD) {
+#pragma unroll
+    for (int d = 0; d < PD; ++d) {
+      const int ps = p0 + d;
+      const char* xb = smem + (ps & 1) * PASS + wk * SLAB;
+      // this chunk's x operands and, under their latency, its weights' fp16
+      u32x4 a[8][RT];
+      half8 b[8];
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+          const int row = 32 * i + r;
+          a[s][i] = *reinterpret_cast<const u32x4*>(xb + row * 256 + (((h * 8 + s) ^ (row & 15)) << 4));
+        }
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        if constexpr (BITS == 4) b[s] = a_w4(wv[d][s >> 2][s & 3]);
+        else b[s] = a_w8(wv[d][s >> 1][2 * (s & 1)], wv[d][s >> 1][2 * (s & 1) + 1]);
+      }
+      const float sd = sc[d];
+      __builtin_amdgcn_sched_barrier(0);
+      load_w(ps + PD, wv[d], sc[d]);
+      __builtin_amdgcn_sched_barrier(0);
+      stage_x(ps + 1, xv);                       // past the end: the last chunk again, never read
+      __builtin_amdgcn_sched_barrier(0);
+      load_x(ps + 2, xv);
+      __builtin_amdgcn_sched_barrier(0);
+      if (ps * WK + wk < nch) {                  // uniform per wave
+        f32x16 t[RT];
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) t[i][e] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+#pragma unroll
+          for (int i = 0; i < RT; ++i)
+            t[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a[s][i]), b[s], t[i], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) mid[i][e] = SC ? __builtin_fmaf(sd, t[i][e], mid[i][e]) : mid[i][e] + t[i][e];
+        if (ps % kMid == kMid - 1) {             // uniform
+#pragma unroll
+          for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+              acc[i][e] += mid[i][e];
+              mid[i][e] = 0.0f;
+            }
+        }
+      }
+      __syncthreads();
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < RT; ++i) acc[i] += mid[i];
+  if constexpr (WK > 1) {
+    f32x16* red = reinterpret_cast<f32x16*>(smem);
+    if (wk > 0)
+#pragma unroll
+      for (int i = 0; i < RT; ++i) red[(((wk - 1) * WN + wn) * RT + i) * 64 + lane] = acc[i];
+    __syncthreads();
+    if (wk > 0) return;
+#pragma unroll
+    for (int k = 1; k < WK; ++k)
+#pragma unroll
+      for (int i = 0; i < RT; ++i) acc[i] += red[(((k - 1) * WN + wn) * RT + i) * 64 + lane];
+  }
+  if (n >= p.N) return;
+  if constexpr (SC == 0) {
+    const float s = load_scale(p, n, 0);
+#pragma unroll
+    for (int i = 0; i < RT; ++i) acc[i] *= s;
+  }
+  const float bv = p.bias ? p.bias[n] : 0.0f;
+  // lane holds rows 8ii + 4h + e of column n: 32 lanes store 128 bytes of a row
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int64_t m = m0 + 32 * i + 8 * ii + 4 * h + e;
+        if (m < p.B) p.y[m * p.ldy + n] = p.bias ? acc[i][4 * ii + e] + bv : acc[i][4 * ii + e];
+      }
+}
+
 constexpr int64_t kQTargetWgs = 512;
 constexpr int64_t kQTileMaxN = 64 * kQTargetWgs;
 
@@ -990,7 +1224,7 @@ static int qgemv_check(const QGemvParams& p, int bits) {
   if (p.ldw < (bits == 4 ? p.K / 2 : p.K)) return VNX_ERR_INVALID_ARG;
   if (p.lds < (bits == 4 ? p.K / p.G : 1)) return VNX_ERR_INVALID_ARG;
   // 16-byte vector loads of x (fp16, or fp32 rows to normalize) and of every row's weights.
-  if (!aligned16(p.x) || p.ldx % (p.xf ? 4 : 8) || !aligned16(p.w) || p.ldw % 16) return VNX_ERR_UNSUPPORTED;
+  if (!aligned16(p.x) || p.ldx % (p.xf || p.x32 ? 4 : 8) || !aligned16(p.w) || p.ldw % 16) return VNX_ERR_UNSUPPORTED;
   if (p.xf && !aligned16(p.nw)) return VNX_ERR_UNSUPPORTED;
   return VNX_OK;
 }
@@ -1000,12 +1234,50 @@ static int qgemv_check(const QGemvParams& p, int bits) {
 // columns, and N fills the GPU anyway, else 1), whole K.  Smaller N: the
 // tile kernel, one 16-row tile per workgroup with K split over its waves.
 
+template <int RT, int WN>
+static int qwgemm_launch(const QGemvParams& p, int bits, hipStream_t s) {
+  const int64_t mt = (p.B + 32 * RT - 1) / (32 * RT), ng = (p.N + 32 * WN - 1) / (32 * WN);
+  if (mt * ng >= INT32_MAX - 8) return VNX_ERR_UNSUPPORTED;
+  const dim3 grid((unsigned)((mt * ng + 7) / 8 * 8));
+  // one scale per row: applied once at the end
+  const int sc = bits == 8 || p.G == p.K ? 0 : p.sc_f16 ? 1 : 2;
+#define VNX_QW(BITS, SC) \
+  do { \
+    if (p.x32) hipLaunchKernelGGL((k_qwgemm<BITS, SC, RT, WN, true>), grid, dim3(256), 0, s, p, (int)mt, (int)ng); \
+    else hipLaunchKernelGGL((k_qwgemm<BITS, SC, RT, WN, false>), grid, dim3(256), 0, s, p, (int)mt, (int)ng); \
+  } while (0)
+  if (bits == 8) VNX_QW(8, 0);
+  else if (sc == 0) VNX_QW(4, 0);
+  else if (sc == 1) VNX_QW(4, 1);
+  else VNX_QW(4, 2);
+#undef VNX_QW
+  VNX_LAUNCH_CHECK();
+  return VNX_OK;
+}
+
 static int qgemv_launch(QGemvParams p, int bits, hipStream_t s) {
   if (p.B == 0 || p.N == 0) return VNX_OK;
+  // The tiled GEMM from 33 rows on (a second 32-row pass of the narrow
+  // kernels: 40 rows x 2,048 x 2,048 9.2 us there, 8.6 here; 1,024 rows 162
+  // and 21), except for the many weight rows of an LM head, whose streaming
+  // kernels take up to two passes.  The widest tile that leaves a workgroup
+  // per CU, else the K split of four waves (us, 64 x 128 / 32 x 128 / 32 x 64 /
+  // 32 x 32): 1,024 rows x 2,048 x 2,048 21 / 22 / 28 / 43, 512 rows 19 / 14 /
+  // 15 / 22, 256 rows 18 / 13 / 10 / 12, 128 rows 18 / 13 / 9.8 / 8.9.
+  const bool plain = !p.yh && !p.rope_on && !p.resid && !p.xf;
+  if (plain && p.B > 32 && (p.N < kQTileMaxN || p.B > 64)) {
+    auto tiles = [&](int64_t rt, int64_t ct) { return ((p.B + rt - 1) / rt) * ((p.N + ct - 1) / ct); };
+    const int64_t cus = device_cus();
+    if (tiles(64, 128) >= cus) return qwgemm_launch<2, 4>(p, bits, s);
+    if (tiles(32, 128) >= cus) return qwgemm_launch<1, 4>(p, bits, s);
+    if (tiles(32, 64) >= cus) return qwgemm_launch<1, 2>(p, bits, s);
+    return qwgemm_launch<1, 1>(p, bits, s);
+  }
   // Batch columns in chunks of 32 (two MFMA column blocks) or one of 16.
   for (int64_t b0 = 0; b0 < p.B; b0 += 32) {
     QGemvParams c = p;
     c.x = p.x + b0 * p.ldx;
+    if (p.x32) c.x32 = p.x32 + b0 * p.ldx;
     if (p.xf) c.xf = p.xf + b0 * p.ldx;
     if (p.emb) {
       c.ids = p.ids + b0;
@@ -1023,7 +1295,10 @@ static int qgemv_launch(QGemvParams p, int bits, hipStream_t s) {
       const bool wide = tiles <= device_cus();
       const dim3 grid((unsigned)tiles);
 #define VNX_QTILE(BITS, NC, NW) \
-  hipLaunchKernelGGL((k_qgemv_tile<BITS, NC, NW>), grid, dim3(NW * 64), 0, s, c)
+  do { \
+    if (c.x32) hipLaunchKernelGGL((k_qgemv_tile<BITS, NC, NW, 0, 3>), grid, dim3(NW * 64), 0, s, c); \
+    else hipLaunchKernelGGL((k_qgemv_tile<BITS, NC, NW>), grid, dim3(NW * 64), 0, s, c); \
+  } while (0)
 #define VNX_QTILE_E(NC, NW, QE, NX) \
   hipLaunchKernelGGL((k_qgemv_tile<4, NC, NW, QE, NX>), grid, dim3(NW * 64), 0, s, c)
 #define VNX_QTILE_E1(NC, QE, NX) \
@@ -1170,6 +1445,36 @@ int vnx_gemv_w4(const void* x, int64_t ldx, const uint8_t* wq, int64_t ldw, cons
   if (st) return st;
   (void)workspace; (void)workspace_bytes;
   return qgemv_launch(p, 4, static_cast<hipStream_t>(stream));
+}
+
+int vnx_linear_w4(const void* x, int x_dtype, int64_t ldx, const uint8_t* wq, int64_t ldw, const void* scales,
+                  int scale_dtype, int64_t lds, int64_t B, int64_t N, int64_t K, int group, const float* bias, float* y,
+                  int64_t ldy, void* stream) {
+  if (x_dtype != VNX_F16 && x_dtype != VNX_F32) return VNX_ERR_UNSUPPORTED;
+  if (scale_dtype != VNX_F16 && scale_dtype != VNX_F32) return VNX_ERR_UNSUPPORTED;
+  if (reinterpret_cast<uintptr_t>(bias) & 3u) return VNX_ERR_INVALID_ARG;
+  QGemvParams p{};
+  p.x = static_cast<const uint16_t*>(x); p.ldx = ldx; p.w = wq; p.ldw = ldw; p.sc = scales; p.lds = lds;
+  if (x_dtype == VNX_F32) p.x32 = static_cast<const float*>(x);
+  p.sc_f16 = scale_dtype == VNX_F16; p.B = B; p.N = N; p.K = K; p.G = group; p.y = y; p.ldy = ldy;
+  p.gpg = group / kGK; p.bias = bias;
+  const int st = qgemv_check(p, 4);
+  if (st) return st;
+  return qgemv_launch(p, 4, static_cast<hipStream_t>(stream));
+}
+
+int vnx_linear_w8(const void* x, int x_dtype, int64_t ldx, const int8_t* wq, int64_t ldw, const float* scale, int64_t B,
+                  int64_t N, int64_t K, const float* bias, float* y, int64_t ldy, void* stream) {
+  if (x_dtype != VNX_F16 && x_dtype != VNX_F32) return VNX_ERR_UNSUPPORTED;
+  if (reinterpret_cast<uintptr_t>(bias) & 3u) return VNX_ERR_INVALID_ARG;
+  QGemvParams p{};
+  p.x = static_cast<const uint16_t*>(x); p.ldx = ldx; p.w = reinterpret_cast<const uint8_t*>(wq); p.ldw = ldw;
+  if (x_dtype == VNX_F32) p.x32 = static_cast<const float*>(x);
+  p.sc = scale; p.lds = 1; p.sc_f16 = 0; p.B = B; p.N = N; p.K = K; p.G = (int)K; p.y = y; p.ldy = ldy;
+  p.gpg = 1; p.bias = bias;
+  const int st = qgemv_check(p, 8);
+  if (st) return st;
+  return qgemv_launch(p, 8, static_cast<hipStream_t>(stream));
 }
 
 int vnx_gemv_w4_swiglu(const void* x, int64_t ldx, const float* norm_w, float eps, const uint8_t* wq, int64_t ldw,

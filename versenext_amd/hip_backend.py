@@ -396,9 +396,33 @@ class HipBackend(DeviceBackend):
         out[:, :w.shape[1]] = w
         return out[:, :w.shape[1]]
 
-    def gemv_w4(self, x, wq, scales, group: int) -> torch.Tensor:
-        """y = x @ (q * s)^T for packed int4 wq (N, K/2) and scales (N, K/group)
-        (fp16 or fp32); returns (..., N) fp32 (vnx_gemv_w4)."""
+    def _linear_x(self, x, K: int, N: int):
+        """(lead shape, rows, dtype code): the activations as the GEMV
+        entries read them, fp16 (B, K) or fp32 rows (rounded to fp16 in the
+        kernel).  Where many row tiles times many weight rows would round
+        each value again and again, one cast first is cheaper (1,024 x 8,192
+        outputs of K = 5,120: 120 + 10 us against 152)."""
+        t = _to_tensor(x, self._torch_device)
+        if t.shape[-1] != K:
+            raise ValueError(f"activations have {t.shape[-1]} features, the weight expects {K}")
+        if t.dtype == torch.float32:
+            t2 = t.reshape(-1, K)
+            if (t2.shape[0] * N < 1 << 22 and t2.stride(1) == 1 and t2.stride(0) % 4 == 0 and t2.stride(0) >= K
+                    and t2.data_ptr() % 16 == 0):
+                return t.shape[:-1], t2, _lib.VNX_F32
+        return t.shape[:-1], self._acts(t, K), _lib.VNX_F16
+
+    def _bias(self, bias, N: int):
+        if bias is None:
+            return None
+        b = _to_tensor(bias, self._torch_device, torch.float32).reshape(-1).contiguous()
+        if b.numel() != N:
+            raise ValueError(f"bias must have {N} entries")
+        return b
+
+    def gemv_w4(self, x, wq, scales, group: int, bias=None) -> torch.Tensor:
+        """y = x @ (q * s)^T (+ bias) for packed int4 wq (N, K/2) and scales
+        (N, K/group) (fp16 or fp32); returns (..., N) fp32 (vnx_linear_w4)."""
         dev = self._torch_device
         w = self._rows16(_to_tensor(wq, dev, torch.uint8))
         sc = _to_tensor(scales, dev)
@@ -406,15 +430,13 @@ class HipBackend(DeviceBackend):
             sc = sc.to(torch.float32)
         sc = sc.reshape(w.shape[0], -1).contiguous()
         N, K = w.shape[0], 2 * w.shape[1]
-        lead = _to_tensor(x, dev).shape[:-1]
-        x2 = self._acts(x, K)
+        lead, x2, xdt = self._linear_x(x, K, N)
         B = x2.shape[0]
         y = torch.empty((B, N), dtype=torch.float32, device=dev)
         sdt = _lib.VNX_F16 if sc.dtype == torch.float16 else _lib.VNX_F32
-        ws = self._workspace(self._L.vnx_gemv_workspace(B, N, K))
-        _lib.check(self._L.vnx_gemv_w4(_ptr(x2), K, _ptr(w), w.stride(0), _ptr(sc), sdt, sc.stride(0), B, N, K,
-                                       int(group), _ptr(y), N, _ptr(ws), ws.numel(),
-                                       ctypes.c_void_p(self._stream().cuda_stream)), "gemv_w4")
+        _lib.check(self._L.vnx_linear_w4(_ptr(x2), xdt, x2.stride(0), _ptr(w), w.stride(0), _ptr(sc), sdt, sc.stride(0),
+                                         B, N, K, int(group), _ptr(self._bias(bias, N)), _ptr(y), N,
+                                         ctypes.c_void_p(self._stream().cuda_stream)), "gemv_w4")
         return y.reshape(*lead, N)
 
     def pack_w4_tiles(self, wq, K: int) -> torch.Tensor:
@@ -446,20 +468,19 @@ class HipBackend(DeviceBackend):
                                                  ctypes.c_void_p(self._stream().cuda_stream)), "gemv_w4_tiles")
         return y.reshape(*lead, N)
 
-    def gemv_w8(self, x, wq, scale) -> torch.Tensor:
-        """y = x @ (q * s)^T for int8 wq (N, K) and per-row fp32 scale (N,)."""
+    def gemv_w8(self, x, wq, scale, bias=None) -> torch.Tensor:
+        """y = x @ (q * s)^T (+ bias) for int8 wq (N, K) and per-row fp32 scale
+        (N,) (vnx_linear_w8)."""
         dev = self._torch_device
         w = self._rows16(_to_tensor(wq, dev, torch.int8))
         sc = _to_tensor(scale, dev, torch.float32).reshape(-1).contiguous()
         N, K = w.shape
-        lead = _to_tensor(x, dev).shape[:-1]
-        x2 = self._acts(x, K)
+        lead, x2, xdt = self._linear_x(x, K, N)
         B = x2.shape[0]
         y = torch.empty((B, N), dtype=torch.float32, device=dev)
-        ws = self._workspace(self._L.vnx_gemv_workspace(B, N, K))
-        _lib.check(self._L.vnx_gemv_w8(_ptr(x2), K, _ptr(w), w.stride(0), _ptr(sc), B, N, K, _ptr(y), N,
-                                       _ptr(ws), ws.numel(), ctypes.c_void_p(self._stream().cuda_stream)),
-                   "gemv_w8")
+        _lib.check(self._L.vnx_linear_w8(_ptr(x2), xdt, x2.stride(0), _ptr(w), w.stride(0), _ptr(sc), B, N, K,
+                                         _ptr(self._bias(bias, N)), _ptr(y), N,
+                                         ctypes.c_void_p(self._stream().cuda_stream)), "gemv_w8")
         return y.reshape(*lead, N)
 
     def dequant_w4(self, wq, scales, K: int, group: int) -> torch.Tensor:

@@ -12,7 +12,7 @@ device) follow packages/verse_torch/verse_torch/quantize.py:
 
 `QuantizedLinear` mirrors the reference class (quantize.py:382-582): it holds
 the packed weight and scales on the GPU and runs `forward` on the gfx950
-dequant-GEMV kernels (vnx_gemv_w4 / vnx_gemv_w8), y = x @ W^T (+ bias).
+dequant-GEMV kernels (vnx_linear_w4 / vnx_linear_w8), y = x @ W^T (+ bias).
 """
 from __future__ import annotations
 
@@ -115,7 +115,7 @@ class QuantizedLinear:
 
     qtype "int8": per-channel int8; "int4": per-channel int4 with fp32 scales
     (the reference's format); "int4_g128": group-128 int4 with fp16 scales.
-    forward(x) takes (..., in) activations (cast to fp16, as the kernels read)
+    forward(x) takes (..., in) activations (rounded to fp16, as the kernels read)
     and returns (..., out) fp32."""
 
     QTYPES = ("int8", "int4", "int4_g128")
@@ -149,12 +149,18 @@ class QuantizedLinear:
         return self.backend.dequant_w4(self.wq, self.scale, self.in_features, group)
 
     def forward(self, x) -> torch.Tensor:
+        # a plain (out,) bias is added by the kernel; one that a gradient flows
+        # to, or of another shape, by PyTorch
+        b = self.bias
+        fuse = b is not None and b.shape == (self.out_features,) and not (b.requires_grad and torch.is_grad_enabled())
+        y = self._product(x, b if fuse else None)
+        return y if b is None or fuse else y + b
+
+    def _product(self, x, bias) -> torch.Tensor:
         if self.qtype == "int8":
-            y = self.backend.gemv_w8(x, self.wq, self.scale)
-        else:
-            group = self.in_features if self.qtype == "int4" else 128
-            y = self.backend.gemv_w4(x, self.wq, self.scale, group)
-        return y if self.bias is None else y + self.bias
+            return self.backend.gemv_w8(x, self.wq, self.scale, bias=bias)
+        group = self.in_features if self.qtype == "int4" else 128
+        return self.backend.gemv_w4(x, self.wq, self.scale, group, bias=bias)
 
     __call__ = forward
 
