@@ -546,6 +546,11 @@ typedef struct vnx_tree_attn_args {
    * then any N >= 1 (prefill chunks); the window may be shorter than N.
    * Zero: the bf16 rows above. */
   int f32_rows;
+  /* The ancestor words in host memory (N, shared by all batch rows), read
+   * during the call and passed to the kernel by value: used when anc is NULL
+   * (bf16 rows), so that a caller whose tree lives on the host needs no
+   * transfer.  NULL (or zero-initialised trailing fields): anc as above. */
+  const uint64_t* anc_host;
 } vnx_tree_attn_args;
 
 /* Workspace bytes of the automatic plan without a window (an upper bound for
@@ -611,6 +616,16 @@ size_t vnx_row_topk_workspace(int64_t rows, int64_t V, int b);
 int vnx_row_topk(const void* logits, int dtype, int64_t rows, int64_t V, int64_t ld, int b,
                  int64_t* ids, float* vals, int64_t ldo, void* workspace, size_t workspace_bytes,
                  void* stream);
+
+/* Tree expansion whole: node n of every batch row takes the r-th best id (the
+ * order above) of its parent's draft row (draft + b*sb + i*ld, i = parent[n] +
+ * 1 < R), r = the number of earlier nodes with that parent (at most 15, < V).
+ * parent (N): host memory, -1 or a node index < n, 1 <= N <= 64.  Only the rows
+ * with children are read.  tokens (B, N) int64.  Rows as vnx_greedy_verify's;
+ * workspace: vnx_row_topk_workspace(B * (rows with children), V, most
+ * children). */
+int vnx_tree_expand(const void* draft, int dtype, int64_t B, int R, int N, int64_t V, int64_t ld, int64_t sb,
+                    const int32_t* parent, int64_t* tokens, void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---------------------------------------------------------------------------
  * Verify-pass LM head on the matrix cores: out (M, V) = x (M, K) . w (V, K)^T,

@@ -115,7 +115,7 @@ class TreeAttnArgs(ctypes.Structure):
         ("qkv", _vp), ("qkv_ld", _c_i64), ("cos_table", _vp), ("sin_table", _vp), ("table_rows", _c_i64),
         ("rope", _int), ("cap", _c_i64),
         ("window", _int), ("alibi_slopes", _vp), ("alibi_max_keys", _int),
-        ("force_splits", _int), ("force_waves", _int), ("f32_rows", _int),
+        ("force_splits", _int), ("force_waves", _int), ("f32_rows", _int), ("anc_host", _vp),
     ]
 
 
@@ -145,6 +145,7 @@ SIGNATURES.update({
                                _vp, _vp, _vp, _vp, _vp, _c_sz, _vp]),
     "vnx_row_topk_workspace": (_c_sz, [_c_i64, _c_i64, _int]),
     "vnx_row_topk": (_int, [_vp, _int, _c_i64, _c_i64, _c_i64, _int, _vp, _vp, _c_i64, _vp, _c_sz, _vp]),
+    "vnx_tree_expand": (_int, [_vp, _int, _c_i64, _int, _int, _c_i64, _c_i64, _c_i64, _vp, _vp, _vp, _c_sz, _vp]),
     "vnx_lm_head": (_int, [_vp, _c_i64, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp, _int, _c_i64, _vp]),
     "vnx_rmsnorm": (_int, [_vp, _c_i64, _vp, _int, _c_i64, _vp, _f32, _c_i64, _c_i64, _vp, _c_i64, _vp, _int,
                            _c_i64, _vp]),

@@ -1,5 +1,7 @@
 // Row top-b: the b best ids of each vocab row (tree expansion: a node's
-// children take the best ids of its parent's draft row).
+// children take the best ids of its parent's draft row; vnx_tree_expand reads
+// only the rows that have children and writes the nodes' tokens from the merge:
+// 17 of the 41 rows of a (4, 3, 2) tree).
 //
 // Order: value descending, ties to the lower id, NaN above every number (the
 // numpy.argmax order, so b = 1 is argmax); -inf ranks below every number.
@@ -8,6 +10,8 @@
 // k_topk_chunk (longer rows) reduces one chunk of one row per workgroup and
 // writes its best KB (b rounded up to a power of two) to the workspace;
 // k_topk_merge merges a row's chunk lists in one wave.
+#include <type_traits>
+
 #include "rowred.h"
 #include "vnx_internal.h"
 
@@ -18,6 +22,7 @@ constexpr int kTNT = 256;
 constexpr int kTNB = 4;
 constexpr int kTopMaxChunks = 64;
 constexpr int kTopMaxB = 16;
+constexpr int kTopMaxNodes = 64;  // tree nodes per sequence
 
 // Order key of (value, id): the value's bits made unsigned-monotone (NaN
 // above +inf, -inf above an empty slot, -0 equal to +0), the id inverted
@@ -97,13 +102,35 @@ struct TopkParams {
   int64_t ldo;
 };
 
-template <typename Tin, int KB>
-__global__ __launch_bounds__(kTNT) void k_topk_chunk(TopkParams p) {
+// Tree expansion: of each batch row's R draft rows only the `inner` ones with
+// children are read (row j of the launch's rows is draft row row[j % inner] of
+// batch row j / inner), and node n takes the rank[n]-th best id of launch row
+// at[n].
+struct TreeMap {
+  int64_t sb;         // elements between batch rows
+  int inner, N;
+  uint8_t row[kTopMaxNodes + 1], at[kTopMaxNodes], rank[kTopMaxNodes];
+  int64_t* tokens;    // (B, N)
+};
+struct NoMap {};
+
+template <typename Tin>
+__device__ __forceinline__ const Tin* topk_row(const TopkParams& p, const NoMap&, int64_t r) {
+  return static_cast<const Tin*>(p.x) + r * p.ld;
+}
+template <typename Tin>
+__device__ __forceinline__ const Tin* topk_row(const TopkParams& p, const TreeMap& m, int64_t r) {
+  const int b = (int)r / m.inner, j = (int)r - b * m.inner;  // launch rows < 2^31
+  return static_cast<const Tin*>(p.x) + b * m.sb + (int64_t)m.row[j] * p.ld;
+}
+
+template <typename Tin, int KB, typename Map>
+__global__ __launch_bounds__(kTNT) void k_topk_chunk(TopkParams p, Map map) {
   constexpr int VE = Vec<Tin>::N;
   __shared__ uint64_t sk[kTNT / VNX_WAVE];
   const int64_t r = blockIdx.x / p.chunks;
   const int c = blockIdx.x % p.chunks;
-  const Tin* row = static_cast<const Tin*>(p.x) + r * p.ld;
+  const Tin* row = topk_row<Tin>(p, map, r);
   const int64_t c0 = (int64_t)c * p.chunk_len;
   const int64_t c1 = c0 + p.chunk_len < p.V ? c0 + p.chunk_len : p.V;
   const int tid = threadIdx.x;
@@ -164,15 +191,15 @@ __global__ __launch_bounds__(kTNT) void k_topk_chunk(TopkParams p) {
 constexpr int kFiltPer = 32;                    // elements per thread
 constexpr int64_t kFiltLen = (int64_t)kTNT * kFiltPer;
 
-template <typename Tin, int KB>
-__global__ __launch_bounds__(kTNT) void k_topk_filter(TopkParams p) {
+template <typename Tin, int KB, typename Map>
+__global__ __launch_bounds__(kTNT) void k_topk_filter(TopkParams p, Map map) {
   constexpr int VE = Vec<Tin>::N;
   constexpr int NV = kFiltPer / VE;             // vectors per thread
   __shared__ uint64_t sk[kTNT / VNX_WAVE];
   __shared__ uint32_t st[kTNT / VNX_WAVE];
   const int64_t r = blockIdx.x / p.chunks;
   const int c = blockIdx.x % p.chunks;
-  const Tin* row = static_cast<const Tin*>(p.x) + r * p.ld;
+  const Tin* row = topk_row<Tin>(p, map, r);
   const int64_t c0 = (int64_t)c * p.chunk_len;
   const int64_t c1 = c0 + p.chunk_len < p.V ? c0 + p.chunk_len : p.V;
   const int64_t n = c1 - c0;
@@ -252,9 +279,10 @@ __global__ __launch_bounds__(kTNT) void k_topk_filter(TopkParams p) {
   }
 }
 
-// One wave per row: lane c holds chunk c's sorted list.
-template <int KB>
-__global__ __launch_bounds__(kTNT) void k_topk_merge(TopkParams p) {
+// One wave per row: lane c holds chunk c's sorted list (tree expansion: lane n
+// writes node n's token when its rank comes up).
+template <int KB, typename Map>
+__global__ __launch_bounds__(kTNT) void k_topk_merge(TopkParams p, Map map) {
   const int lane = threadIdx.x % VNX_WAVE;
   const int64_t r = (int64_t)blockIdx.x * (kTNT / VNX_WAVE) + threadIdx.x / VNX_WAVE;
   if (r >= p.rows) return;
@@ -265,20 +293,41 @@ __global__ __launch_bounds__(kTNT) void k_topk_merge(TopkParams p) {
   for (int q = 0; q < KB; ++q) {
     const uint64_t best = wave_max_u64(K.k[0]);
     if (K.k[0] == best && best != 0ull) K.pop();
-    if (lane == 0 && q < p.b) {
+    if constexpr (std::is_same<Map, TreeMap>::value) {
+      const int b = (int)r / map.inner, j = (int)r - b * map.inner;
+      if (lane < map.N && map.at[lane] == j && map.rank[lane] == q)
+        map.tokens[(int64_t)b * map.N + lane] = (int64_t)(uint32_t)~(uint32_t)best;
+    } else if (lane == 0 && q < p.b) {
       p.ids[r * p.ldo + q] = (int64_t)(uint32_t)~(uint32_t)best;
       if (p.vals) p.vals[r * p.ldo + q] = vkey_value((uint32_t)(best >> 32));
     }
   }
 }
 
-template <typename Tin, int KB>
-void launch_topk(const TopkParams& p, hipStream_t s) {
+template <typename Tin, int KB, typename Map>
+void launch_topk(const TopkParams& p, const Map& map, hipStream_t s) {
+  const dim3 grid((unsigned)(p.rows * p.chunks));
   if (p.chunk_len == kFiltLen)
-    hipLaunchKernelGGL((k_topk_filter<Tin, KB>), dim3((unsigned)(p.rows * p.chunks)), dim3(kTNT), 0, s, p);
+    hipLaunchKernelGGL((k_topk_filter<Tin, KB, Map>), grid, dim3(kTNT), 0, s, p, map);
   else
-    hipLaunchKernelGGL((k_topk_chunk<Tin, KB>), dim3((unsigned)(p.rows * p.chunks)), dim3(kTNT), 0, s, p);
-  hipLaunchKernelGGL(k_topk_merge<KB>, dim3((unsigned)((p.rows + 3) / 4)), dim3(kTNT), 0, s, p);
+    hipLaunchKernelGGL((k_topk_chunk<Tin, KB, Map>), grid, dim3(kTNT), 0, s, p, map);
+  hipLaunchKernelGGL((k_topk_merge<KB, Map>), dim3((unsigned)((p.rows + 3) / 4)), dim3(kTNT), 0, s, p, map);
+}
+
+template <typename Map>
+void launch_topk_kb(int dtype, int kb, const TopkParams& p, const Map& map, hipStream_t s) {
+  auto go = [&](auto tin) {
+    using Tin = decltype(tin);
+    switch (kb) {
+      case 1: launch_topk<Tin, 1>(p, map, s); break;
+      case 2: launch_topk<Tin, 2>(p, map, s); break;
+      case 4: launch_topk<Tin, 4>(p, map, s); break;
+      case 8: launch_topk<Tin, 8>(p, map, s); break;
+      default: launch_topk<Tin, 16>(p, map, s); break;
+    }
+  };
+  if (dtype == VNX_F32) go(float{});
+  else go(__hip_bfloat16{});
 }
 
 int kb_of(int b) {
@@ -343,19 +392,50 @@ int vnx_row_topk(const void* logits, int dtype, int64_t rows, int64_t V, int64_t
   if (!workspace || workspace_bytes < cv.bytes()) return VNX_ERR_WORKSPACE;
   p.x = logits; p.rows = rows; p.V = V; p.ld = ld; p.chunks = c; p.chunk_len = len;
   p.b = b; p.ids = ids; p.vals = vals; p.ldo = ldo;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  auto go = [&](auto tin) {
-    using Tin = decltype(tin);
-    switch (kb) {
-      case 1: launch_topk<Tin, 1>(p, s); break;
-      case 2: launch_topk<Tin, 2>(p, s); break;
-      case 4: launch_topk<Tin, 4>(p, s); break;
-      case 8: launch_topk<Tin, 8>(p, s); break;
-      default: launch_topk<Tin, 16>(p, s); break;
+  launch_topk_kb(dtype, kb, p, NoMap{}, static_cast<hipStream_t>(stream));
+  VNX_LAUNCH_CHECK();
+  return VNX_OK;
+}
+
+int vnx_tree_expand(const void* draft, int dtype, int64_t B, int R, int N, int64_t V, int64_t ld, int64_t sb,
+                    const int32_t* parent, int64_t* tokens, void* workspace, size_t workspace_bytes, void* stream) {
+  if (dtype != VNX_F32 && dtype != VNX_BF16) return VNX_ERR_UNSUPPORTED;
+  if (B < 0 || R < 1 || N < 1 || N > kTopMaxNodes || V <= 0 || !parent) return VNX_ERR_INVALID_ARG;
+  TreeMap m{};
+  int at[kTopMaxNodes + 1], kids[kTopMaxNodes + 1] = {0};  // launch row and children so far of a draft row
+  for (int q = 0; q <= N; ++q) at[q] = -1;
+  int most = 0;
+  for (int i = 0; i < N; ++i) {
+    if (parent[i] < -1 || parent[i] >= i) return VNX_ERR_INVALID_ARG;
+    const int row = parent[i] + 1;
+    if (row >= R) return VNX_ERR_INVALID_ARG;
+    if (at[row] < 0) {
+      at[row] = m.inner;
+      m.row[m.inner++] = (uint8_t)row;
     }
-  };
-  if (dtype == VNX_F32) go(float{});
-  else go(__hip_bfloat16{});
+    m.at[i] = (uint8_t)at[row];
+    m.rank[i] = (uint8_t)kids[row]++;
+    if (kids[row] > most) most = kids[row];
+  }
+  if (most > kTopMaxB || most > V) return VNX_ERR_INVALID_ARG;
+  if (B == 0) return VNX_OK;
+  if (!tokens) return VNX_ERR_INVALID_ARG;
+  const int st = check_rows(draft, dtype, ld, sb, R, V);
+  if (st) return st;
+  const int64_t rows = B * m.inner;
+  if (B > (1 << 24) || rows > (1 << 24) || V >= ((int64_t)1 << 31)) return VNX_ERR_UNSUPPORTED;
+  int c;
+  int64_t len;
+  topk_plan(rows, V, dtype, &c, &len);
+  if (rows * (int64_t)c >= INT32_MAX) return VNX_ERR_UNSUPPORTED;
+  const int kb = kb_of(most);
+  Carve cv(workspace);
+  TopkParams p{};
+  p.part = cv.take<uint64_t>((size_t)rows * c * kb);
+  if (!workspace || workspace_bytes < cv.bytes()) return VNX_ERR_WORKSPACE;
+  p.x = draft; p.rows = rows; p.V = V; p.ld = ld; p.chunks = c; p.chunk_len = len; p.b = most;
+  m.sb = sb; m.N = N; m.tokens = tokens;
+  launch_topk_kb(dtype, kb, p, m, static_cast<hipStream_t>(stream));
   VNX_LAUNCH_CHECK();
   return VNX_OK;
 }

@@ -90,6 +90,7 @@ struct TreeAttnParams {
   const float* sin;
   int rope;
   int64_t cap;                      // rows at or past it are not written (and not rotated past the table)
+  uint64_t anc_in[kTaMaxN];         // the shared ancestor words, when anc is NULL
 };
 
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
@@ -272,6 +273,7 @@ __global__ __launch_bounds__(NW * 64, (PF == 2 && D == 64 && NW == 4) ? 2 : 1) v
     }
   }
   // Ancestor words of this lane's query columns.
+  auto word = [&](int node) -> uint64_t { return p.anc ? p.anc[b * p.anc_sb + node] : p.anc_in[node]; };
   uint64_t anc[QT];
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
@@ -279,7 +281,7 @@ __global__ __launch_bounds__(NW * 64, (PF == 2 && D == 64 && NW == 4) ? 2 : 1) v
     anc[qt] = ~0ull;
     if (r < nrows) {
       const int rr = row0 + r, node = rr % p.N;
-      anc[qt] = p.anc[b * p.anc_sb + node];
+      anc[qt] = word(node);
     }
   }
   __syncthreads();
@@ -438,7 +440,7 @@ __global__ __launch_bounds__(NW * 64, (PF == 2 && D == 64 && NW == 4) ? 2 : 1) v
           const int key = base + (e < 4 ? 0 : 16) + grp * 4 + (e & 3);
           const int j = key - Tpe;
           kpos[e] = key < Tpe ? key
-                              : (j < p.N ? Tp + __builtin_popcountll(p.anc[b * p.anc_sb + j]) - 1 : Tp);
+                              : (j < p.N ? Tp + __builtin_popcountll(word(j)) - 1 : Tp);
         }
       }
     }
@@ -1128,7 +1130,8 @@ int vnx_tree_attn(const vnx_tree_attn_args* a, void* workspace, size_t workspace
   if (N > kTaMaxN || (d != 64 && d != 128)) return VNX_ERR_UNSUPPORTED;
   if (a->T2 < 0) return VNX_ERR_INVALID_ARG;
   if (B == 0) return VNX_OK;
-  if ((!a->q && !a->qkv) || !a->k_tree || !a->v_tree || !a->anc || !a->out) return VNX_ERR_INVALID_ARG;
+  if ((!a->q && !a->qkv) || !a->k_tree || !a->v_tree || (!a->anc && !a->anc_host) || !a->out)
+    return VNX_ERR_INVALID_ARG;
   if (a->qkv) {
     // the projection rows: RoPE and the tree rows' cache write here
     if (!a->tree_follows_prefix || !a->tp_batch || a->cap < 1) return VNX_ERR_INVALID_ARG;
@@ -1179,6 +1182,8 @@ int vnx_tree_attn(const vnx_tree_attn_args* a, void* workspace, size_t workspace
   p.kt = static_cast<const uint16_t*>(a->k_tree);
   p.vt = static_cast<const uint16_t*>(a->v_tree);
   p.anc = a->anc;
+  if (!a->anc)
+    for (int i = 0; i < N; ++i) p.anc_in[i] = a->anc_host[i];
   p.out = a->out;
   p.q_sb = a->q_strides[0]; p.q_sh = a->q_strides[1]; p.q_sr = a->q_strides[2];
   p.c_sb = a->cache_strides[0]; p.c_sh = a->cache_strides[1]; p.c_sr = a->cache_strides[2];

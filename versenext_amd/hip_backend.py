@@ -578,7 +578,9 @@ class HipBackend(DeviceBackend):
             a = np.ascontiguousarray(a.astype(np.uint64) if a.dtype != np.uint64 else a)
             if a.shape not in ((N,), (B, N)):
                 raise ValueError(f"anc must be ({N},) or ({B}, {N}), got {a.shape}")
-            anc_t = torch.from_numpy(a.view(np.int64)).to(dev)
+            # one tree for all rows: by value with the launch (no transfer);
+            # a tree per batch row, or the fp32-rows path: on the device
+            anc_t = None if a.ndim == 1 and not fp32_rows else torch.from_numpy(a.view(np.int64)).to(dev)
         if out_dtype not in (torch.float32, torch.bfloat16, torch.float16):
             raise ValueError("out_dtype must be torch.float32, torch.bfloat16 or torch.float16")
         out = torch.empty((B, H, N, d), dtype=out_dtype, device=dev)
@@ -593,6 +595,8 @@ class HipBackend(DeviceBackend):
         args.v_tree = vt.data_ptr()
         args.tree_strides[:] = list(kt.stride()[:3])
         args.anc = anc_t.data_ptr() if anc_t is not None else None
+        if a is not None and anc_t is None:
+            args.anc_host = a.ctypes.data
         args.anc_batch_stride = N if a is not None and a.ndim == 2 else 0
         args.f32_rows = int(fp32_rows)
         args.out = out.data_ptr()
@@ -697,7 +701,7 @@ class HipBackend(DeviceBackend):
             _ptr(tg), _LOGIT_DTYPES[tg.dtype], B, k, rows_t, V, tg.stride(1), tg.stride(0), _ptr(ids),
             _ptr(acc), _ptr(pred), _ptr(alen), _ptr(out), _ptr(ws), ws.numel(),
             ctypes.c_void_p(self._stream().cuda_stream)), "greedy_verify")
-        return acc.bool(), pred, alen, out
+        return acc.view(torch.bool), pred, alen, out   # the kernel writes 0 / 1
 
     def lm_head(self, x, weight, out=None, out_dtype=torch.float32) -> torch.Tensor:
         """Verify-pass LM head (vnx_lm_head): x (..., K) . weight (V, K)^T on the
@@ -782,18 +786,26 @@ class HipBackend(DeviceBackend):
     def expand_tree(self, draft, parent):
         """Node tokens (B, N) of a token tree: node n takes the r-th best id
         of its parent's draft row (row 0 for the root, 1 + parent otherwise),
-        r = the number of earlier siblings of n.  draft (B, R, V)."""
+        r = the number of earlier siblings of n.  draft (B, R, V)
+        (vnx_tree_expand: only the rows with children are read)."""
         from . import tree as _tree
-        par = _tree.check_parents(parent)
-        rows = np.where(par < 0, 0, par + 1)
-        rank = np.zeros(par.size, np.int64)
-        seen: dict = {}
-        for i, p in enumerate(par):
-            rank[i] = seen.get(int(p), 0)
-            seen[int(p)] = rank[i] + 1
-        ids, _ = self.topk(draft, int(rank.max()) + 1)
-        dev = self._torch_device
-        return ids[:, torch.from_numpy(rows).to(dev), torch.from_numpy(rank).to(dev)]
+        par = np.ascontiguousarray(_tree.check_parents(parent), dtype=np.int32)
+        t = _to_tensor(draft, self._torch_device)
+        if t.dim() != 3:
+            raise IndexError(f"draft must be (B, R, V), got shape {tuple(t.shape)}")
+        R, used = t.shape[1], np.unique(par + 1)
+        if R <= used[-1]:
+            raise IndexError(f"draft has {R} rows, the tree reads row {used[-1]}")
+        t = self._rows3d(t, R)
+        B, _, V = t.shape
+        most = int(np.bincount(par + 1).max())
+        tokens = torch.empty((B, par.size), dtype=torch.int64, device=self._torch_device)
+        ws = self._workspace(self._L.vnx_row_topk_workspace(B * used.size, V, most))
+        _lib.check(self._L.vnx_tree_expand(
+            _ptr(t), _LOGIT_DTYPES[t.dtype], B, R, par.size, V, t.stride(1), t.stride(0),
+            par.ctypes.data_as(ctypes.c_void_p), _ptr(tokens), _ptr(ws), ws.numel(),
+            ctypes.c_void_p(self._stream().cuda_stream)), "tree_expand")
+        return tokens
 
 
 __all__ = ["HipBackend"]
