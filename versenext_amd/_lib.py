@@ -178,6 +178,14 @@ SIGNATURES.update({
                                     _c_i64, _int, _vp, _vp, _vp, _vp, _int, _c_i64, _c_i64, _vp]),
 })
 
+def stream_handle(index: int) -> int:
+    """The current PyTorch stream of GPU `index` as the void* the entries take.
+    PyTorch's own raw getter where it has one (0.1 us); torch.cuda.current_stream
+    builds a Stream object for the same value (3.5 us, twice per operator)."""
+    get = getattr(_torch._C, "_cuda_getCurrentRawStream", None)
+    return get(index) if get is not None else _torch.cuda.current_stream(index).cuda_stream
+
+
 _lib = None
 _lock = threading.Lock()
 

@@ -176,7 +176,7 @@ class SpecDecodeEngine:
             P(alen.data_ptr()), P(ids.data_ptr()), ids.stride(0), B, k, P(self.out.data_ptr()), self.out.stride(0),
             self.out.shape[1] - 1, P(self.count.data_ptr()), P(self.c.data_ptr()), P(self.lens_t.data_ptr()),
             P(self.lens_d.data_ptr()), P(self.info.data_ptr()),
-            ctypes.c_void_p(torch.cuda.current_stream(self.dev).cuda_stream)), "spec_commit")
+            _lib.stream_handle(self.hip._index)), "spec_commit")
 
     # ---- driver ---------------------------------------------------------
     @torch.no_grad()

@@ -41,8 +41,8 @@ def _to_tensor(x, device, dtype=None) -> torch.Tensor:
     return t
 
 
-def _ptr(t) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+def _ptr(t):
+    return t.data_ptr() if t is not None else None
 
 
 _LOGIT_DTYPES = {torch.float32: _lib.VNX_F32, torch.bfloat16: _lib.VNX_BF16}
@@ -86,12 +86,12 @@ class HipBackend(DeviceBackend):
         return t.detach().cpu().numpy() if isinstance(t, torch.Tensor) else np.asarray(t)
 
     # ---- plumbing -------------------------------------------------------
-    def _stream(self):
-        return torch.cuda.current_stream(self._torch_device)
+    def _stream(self) -> int:
+        return _lib.stream_handle(self._index)
 
     def _workspace(self, nbytes: int) -> torch.Tensor:
         """Zeroed scratch for the current stream, grown on demand."""
-        st = self._stream().cuda_stream
+        st = self._stream()
         with self._ws_lock:
             buf = self._ws.get(st)
             if buf is None or buf.numel() < nbytes:
@@ -132,9 +132,10 @@ class HipBackend(DeviceBackend):
         t = self._logits(x)
         if t.dim() != 3 or t.shape[1] != nrows:
             raise ValueError(f"expected logits of shape (B, {nrows}, V), got {tuple(t.shape)}")
-        V = t.shape[-1]
-        ok = self._vec_ok(t) and t.stride(1) >= V and t.stride(0) >= (nrows - 1) * t.stride(1) + V
-        if not ok:
+        V = t.shape[2]
+        sb, ld, s1 = t.stride()
+        ve = 4 if t.dtype == torch.float32 else 8
+        if s1 != 1 or t.data_ptr() % 16 or sb % ve or ld % ve or ld < V or sb < (nrows - 1) * ld + V:
             t = t.contiguous()
             if not self._vec_ok(t):
                 ve = 4 if t.dtype == torch.float32 else 8
@@ -167,7 +168,7 @@ class HipBackend(DeviceBackend):
         ws = self._workspace(self._L.vnx_softmax_workspace(R, V))
         _lib.check(self._L.vnx_softmax(_ptr(x2), _LOGIT_DTYPES[x2.dtype], R, V, x2.stride(0), float(temperature),
                                        _ptr(thr), _ptr(out), V, _ptr(ws), ws.numel(),
-                                       ctypes.c_void_p(self._stream().cuda_stream)), "softmax")
+                                       self._stream()), "softmax")
         out = out.reshape(shape)
         return out.movedim(-1, dim) if moved else out
 
@@ -209,7 +210,7 @@ class HipBackend(DeviceBackend):
         ws = self._workspace(self._L.vnx_row_lse_workspace(R, V))
         _lib.check(self._L.vnx_row_lse(_ptr(x2), _LOGIT_DTYPES[x2.dtype], R, V, x2.stride(0), float(temperature),
                                        _ptr(thr), _ptr(lse), _ptr(mx), _ptr(am), _ptr(ws), ws.numel(),
-                                       ctypes.c_void_p(self._stream().cuda_stream)), "row_lse")
+                                       self._stream()), "row_lse")
         return lse, mx, am
 
     def argmax(self, x) -> torch.Tensor:
@@ -221,7 +222,7 @@ class HipBackend(DeviceBackend):
         am = torch.empty(R, dtype=torch.int64, device=self._torch_device)
         ws = self._workspace(self._L.vnx_row_lse_workspace(R, V))
         _lib.check(self._L.vnx_row_argmax(_ptr(x2), _LOGIT_DTYPES[x2.dtype], R, V, x2.stride(0), _ptr(am),
-                                          _ptr(ws), ws.numel(), ctypes.c_void_p(self._stream().cuda_stream)),
+                                          _ptr(ws), ws.numel(), self._stream()),
                    "argmax")
         return am.reshape(lead)
 
@@ -273,14 +274,14 @@ class HipBackend(DeviceBackend):
                 tg.stride(1), tg.stride(0), df.stride(1), df.stride(0),
                 _ptr(ids), _ptr(u), float(temperature), _ptr(ld), _ptr(fd), ld.stride(0),
                 _ptr(alen), _ptr(out), _ptr(flags), _ptr(lse_t),
-                _ptr(ws), ws.numel(), ctypes.c_void_p(self._stream().cuda_stream)), "spec_accept_draft_lse")
+                _ptr(ws), ws.numel(), self._stream()), "spec_accept_draft_lse")
             return dict(accept_len=alen, out_ids=out, flags=flags, lse_t=lse_t, lse_d=ld.t())
         _lib.check(self._L.vnx_spec_accept(
             _ptr(tg), _ptr(df), _LOGIT_DTYPES[tg.dtype], B, k, V,
             tg.stride(1), tg.stride(0), df.stride(1), df.stride(0),
             _ptr(ids), _ptr(u), float(temperature), _ptr(tt), _ptr(td),
             _ptr(alen), _ptr(out), _ptr(flags), _ptr(lse_t), _ptr(lse_d),
-            _ptr(ws), ws.numel(), ctypes.c_void_p(self._stream().cuda_stream)), "spec_accept")
+            _ptr(ws), ws.numel(), self._stream()), "spec_accept")
         return dict(accept_len=alen, out_ids=out, flags=flags, lse_t=lse_t, lse_d=lse_d)
 
     def sample(self, logits, uniforms, temperature: float = 1.0, thresholds=None, out=None,
@@ -310,7 +311,7 @@ class HipBackend(DeviceBackend):
         _lib.check(self._L.vnx_sample(
             _ptr(lg), _LOGIT_DTYPES[lg.dtype], B, V, lg.stride(0), _ptr(u), float(temperature), _ptr(thr),
             _ptr(ids), _ptr(flags), _ptr(lse), _ptr(ws), ws.numel(),
-            ctypes.c_void_p(self._stream().cuda_stream)), "sample")
+            self._stream()), "sample")
         if return_all:
             return dict(ids=ids, flags=flags, lse=lse)
         return ids
@@ -357,7 +358,7 @@ class HipBackend(DeviceBackend):
             _ptr(lg), dt, B, V, lg.stride(0), float(temperature), int(top_k), float(top_p),
             mode, float(calib_factor if calib_factor is not None else 1.0), float(calib_eps),
             _ptr(u), _ptr(ids), g("flags"), g("lse"), g("kth"), g("p_star"), g("j_star"), g("k_star"),
-            _ptr(ws), ws.numel(), ctypes.c_void_p(self._stream().cuda_stream)), "sampler_sample")
+            _ptr(ws), ws.numel(), self._stream()), "sampler_sample")
         if return_all:
             return dict(ids=ids, **extra)
         return ids
@@ -373,7 +374,7 @@ class HipBackend(DeviceBackend):
         var = torch.empty(R, dtype=torch.float64, device=self._torch_device)
         _lib.check(self._L.vnx_logit_calibrate(_ptr(x2), _LOGIT_DTYPES[x2.dtype], R, V, x2.stride(0),
                                                float(calib_factor), float(eps), _ptr(out), V, _ptr(var),
-                                               ctypes.c_void_p(self._stream().cuda_stream)), "logit_calibrate")
+                                               self._stream()), "logit_calibrate")
         out = out.reshape(shape)
         return (out, var) if return_var else out
 
@@ -436,7 +437,7 @@ class HipBackend(DeviceBackend):
         sdt = _lib.VNX_F16 if sc.dtype == torch.float16 else _lib.VNX_F32
         _lib.check(self._L.vnx_linear_w4(_ptr(x2), xdt, x2.stride(0), _ptr(w), w.stride(0), _ptr(sc), sdt, sc.stride(0),
                                          B, N, K, int(group), _ptr(self._bias(bias, N)), _ptr(y), N,
-                                         ctypes.c_void_p(self._stream().cuda_stream)), "gemv_w4")
+                                         self._stream()), "gemv_w4")
         return y.reshape(*lead, N)
 
     def pack_w4_tiles(self, wq, K: int) -> torch.Tensor:
@@ -448,7 +449,7 @@ class HipBackend(DeviceBackend):
         N = w.shape[0]
         out = torch.empty(self._L.vnx_w4_tiles_bytes(N, K), dtype=torch.uint8, device=dev)
         _lib.check(self._L.vnx_pack_w4_tiles(_ptr(w), w.stride(0), N, K, _ptr(out),
-                                             ctypes.c_void_p(self._stream().cuda_stream)), "pack_w4_tiles")
+                                             self._stream()), "pack_w4_tiles")
         return out
 
     def gemv_w4_tiles(self, x, wt, scales, N: int, K: int, out_dtype=torch.float32) -> torch.Tensor:
@@ -465,7 +466,7 @@ class HipBackend(DeviceBackend):
         y = torch.empty((B, N), dtype=out_dtype, device=dev)
         _lib.check(self._L.vnx_gemv_w4_tiles_out(_ptr(x2), K, _ptr(wt), _ptr(sc), sc.stride(0), B, N, K, _ptr(y),
                                                  _LOGIT_DTYPES[out_dtype], N,
-                                                 ctypes.c_void_p(self._stream().cuda_stream)), "gemv_w4_tiles")
+                                                 self._stream()), "gemv_w4_tiles")
         return y.reshape(*lead, N)
 
     def gemv_w8(self, x, wq, scale, bias=None) -> torch.Tensor:
@@ -480,7 +481,7 @@ class HipBackend(DeviceBackend):
         y = torch.empty((B, N), dtype=torch.float32, device=dev)
         _lib.check(self._L.vnx_linear_w8(_ptr(x2), xdt, x2.stride(0), _ptr(w), w.stride(0), _ptr(sc), B, N, K,
                                          _ptr(self._bias(bias, N)), _ptr(y), N,
-                                         ctypes.c_void_p(self._stream().cuda_stream)), "gemv_w8")
+                                         self._stream()), "gemv_w8")
         return y.reshape(*lead, N)
 
     def dequant_w4(self, wq, scales, K: int, group: int) -> torch.Tensor:
@@ -494,7 +495,7 @@ class HipBackend(DeviceBackend):
         out = torch.empty((N, K), dtype=torch.float32, device=dev)
         sdt = _lib.VNX_F16 if sc.dtype == torch.float16 else _lib.VNX_F32
         _lib.check(self._L.vnx_dequant_w4(_ptr(w), w.stride(0), _ptr(sc), sdt, sc.stride(0), N, K, int(group),
-                                          _ptr(out), K, ctypes.c_void_p(self._stream().cuda_stream)),
+                                          _ptr(out), K, self._stream()),
                    "dequant_w4")
         return out
 
@@ -505,7 +506,7 @@ class HipBackend(DeviceBackend):
         N, K = w.shape
         out = torch.empty((N, K), dtype=torch.float32, device=dev)
         _lib.check(self._L.vnx_dequant_w8(_ptr(w), w.stride(0), _ptr(sc), N, K, _ptr(out), K,
-                                          ctypes.c_void_p(self._stream().cuda_stream)), "dequant_w8")
+                                          self._stream()), "dequant_w8")
         return out
 
     # ---- tree-verify attention ------------------------------------------------
@@ -645,7 +646,7 @@ class HipBackend(DeviceBackend):
             args.gates = g.data_ptr()
         ws = self._workspace(self._L.vnx_tree_attn_workspace_args(ctypes.byref(args)))
         _lib.check(self._L.vnx_tree_attn(ctypes.byref(args), _ptr(ws), ws.numel(),
-                                         ctypes.c_void_p(self._stream().cuda_stream)), "tree_attn")
+                                         self._stream()), "tree_attn")
         del keep
         return out
 
@@ -700,7 +701,7 @@ class HipBackend(DeviceBackend):
         _lib.check(self._L.vnx_greedy_verify(
             _ptr(tg), _LOGIT_DTYPES[tg.dtype], B, k, rows_t, V, tg.stride(1), tg.stride(0), _ptr(ids),
             _ptr(acc), _ptr(pred), _ptr(alen), _ptr(out), _ptr(ws), ws.numel(),
-            ctypes.c_void_p(self._stream().cuda_stream)), "greedy_verify")
+            self._stream()), "greedy_verify")
         return acc.view(torch.bool), pred, alen, out   # the kernel writes 0 / 1
 
     def lm_head(self, x, weight, out=None, out_dtype=torch.float32) -> torch.Tensor:
@@ -732,7 +733,7 @@ class HipBackend(DeviceBackend):
                 raise ValueError(f"out must be a ({M}, {V}) view with unit last stride")
         _lib.check(self._L.vnx_lm_head(
             _ptr(x2), x2.stride(0), _ptr(wt), wt.stride(0), M, K, V, _ptr(o),
-            _LOGIT_DTYPES[o.dtype], o.stride(0), ctypes.c_void_p(self._stream().cuda_stream)), "lm_head")
+            _LOGIT_DTYPES[o.dtype], o.stride(0), self._stream()), "lm_head")
         return o.reshape(*lead, V) if out is None else o
 
     def tree_greedy(self, target, tokens, parent):
@@ -766,7 +767,7 @@ class HipBackend(DeviceBackend):
         _lib.check(self._L.vnx_tree_greedy(
             _ptr(tg), _LOGIT_DTYPES[tg.dtype], B, N, V, tg.stride(1), tg.stride(0), _ptr(tok),
             tok.stride(0), par.ctypes.data_as(ctypes.c_void_p), _ptr(alen), _ptr(best), _ptr(out),
-            _ptr(pred), _ptr(ws), ws.numel(), ctypes.c_void_p(self._stream().cuda_stream)), "tree_greedy")
+            _ptr(pred), _ptr(ws), ws.numel(), self._stream()), "tree_greedy")
         return alen, best, out, pred
 
     def topk(self, x, b: int):
@@ -780,7 +781,7 @@ class HipBackend(DeviceBackend):
         ws = self._workspace(self._L.vnx_row_topk_workspace(rows, V, b))
         _lib.check(self._L.vnx_row_topk(
             _ptr(t), _LOGIT_DTYPES[t.dtype], rows, V, t.stride(0), int(b), _ptr(ids),
-            _ptr(vals), b, _ptr(ws), ws.numel(), ctypes.c_void_p(self._stream().cuda_stream)), "row_topk")
+            _ptr(vals), b, _ptr(ws), ws.numel(), self._stream()), "row_topk")
         return ids.reshape(*lead, b), vals.reshape(*lead, b)
 
     def expand_tree(self, draft, parent):
@@ -804,7 +805,7 @@ class HipBackend(DeviceBackend):
         _lib.check(self._L.vnx_tree_expand(
             _ptr(t), _LOGIT_DTYPES[t.dtype], B, R, par.size, V, t.stride(1), t.stride(0),
             par.ctypes.data_as(ctypes.c_void_p), _ptr(tokens), _ptr(ws), ws.numel(),
-            ctypes.c_void_p(self._stream().cuda_stream)), "tree_expand")
+            self._stream()), "tree_expand")
         return tokens
 
 

@@ -305,7 +305,7 @@ def _pack(w: torch.Tensor, hip) -> torch.Tensor:
     L = hip._L
     out = torch.empty(L.vnx_pack_bf16_size(N, K) // 2, dtype=torch.bfloat16, device=hip.torch_device)
     _lib.check(L.vnx_pack_bf16(ctypes.c_void_p(w.data_ptr()), K, N, K, ctypes.c_void_p(out.data_ptr()),
-                               ctypes.c_void_p(torch.cuda.current_stream(hip.torch_device).cuda_stream)), "pack_bf16")
+                               _lib.stream_handle(hip._index)), "pack_bf16")
     return out
 
 
@@ -356,8 +356,7 @@ class _Linear:
                                       device=hip.torch_device)
                 _lib.check(L.vnx_pack_w4_tiles(ctypes.c_void_p(self.wq.data_ptr()), self.wq.stride(0), self.N,
                                                self.K, ctypes.c_void_p(self.wt.data_ptr()),
-                                               ctypes.c_void_p(torch.cuda.current_stream(hip.torch_device)
-                                                               .cuda_stream)), "pack_w4_tiles")
+                                               _lib.stream_handle(hip._index)), "pack_w4_tiles")
         else:
             self.wd = w.to(dtype).contiguous()
             # the products run vnx_gemm_bf16 on a packed copy; for a fused [gate; up] weight its rows are
@@ -373,7 +372,7 @@ class _Linear:
                                       device=hip.torch_device)
                 _lib.check(L.vnx_pack_bf16(ctypes.c_void_p(src.data_ptr()), self.K, self.N, self.K,
                                            ctypes.c_void_p(self.wp.data_ptr()),
-                                           ctypes.c_void_p(torch.cuda.current_stream(hip.torch_device).cuda_stream)),
+                                           _lib.stream_handle(hip._index)),
                            "pack_bf16")
 
 
@@ -396,7 +395,7 @@ class _Linear:
         _lib.check(self.hip._L.vnx_gemm_bf16(
             ctypes.c_void_p(x.data_ptr()), x.stride(0), 0, ctypes.c_void_p(self.wp.data_ptr()), 0, M, self.N, self.K,
             1, int(epilogue), None, 1, ctypes.c_void_p(y.data_ptr()), _lib.DTYPE_CODES[y.dtype], ncols, 0,
-            ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)), "gemm_bf16")
+            _lib.stream_handle(x.device.index)), "gemm_bf16")
         return y
 
     def gemm_norm(self, x: torch.Tensor, norm_w: torch.Tensor, eps: float, epilogue: int = 0) -> Optional[torch.Tensor]:
@@ -412,7 +411,7 @@ class _Linear:
         _lib.check(self.hip._L.vnx_gemm_bf16_norm(
             ctypes.c_void_p(x.data_ptr()), x.stride(0), ctypes.c_void_p(norm_w.data_ptr()), float(eps),
             ctypes.c_void_p(self.wp.data_ptr()), M, self.N, self.K, int(epilogue), ctypes.c_void_p(y.data_ptr()),
-            ncols, ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)), "gemm_bf16_norm")
+            ncols, _lib.stream_handle(x.device.index)), "gemm_bf16_norm")
         return y
 
     def gemm_norm_embed(self, tokens: torch.Tensor, emb: torch.Tensor, scale: float, x: torch.Tensor,
@@ -431,7 +430,7 @@ class _Linear:
         _lib.check(self.hip._L.vnx_gemm_bf16_norm_embed(
             P(tokens.data_ptr()), P(emb.data_ptr()), _lib.VNX_BF16, emb.stride(0), emb.shape[0], float(scale),
             P(x.data_ptr()), x.stride(0), P(norm_w.data_ptr()), float(eps), P(self.wp.data_ptr()), M, self.N,
-            self.K, P(y.data_ptr()), self.N, P(torch.cuda.current_stream(x.device).cuda_stream)),
+            self.K, P(y.data_ptr()), self.N, _lib.stream_handle(x.device.index)),
             "gemm_bf16_norm_embed")
         return y
 
@@ -444,7 +443,7 @@ class _Linear:
         _lib.check(self.hip._L.vnx_gemm_bf16_residual(
             ctypes.c_void_p(x.data_ptr()), x.stride(0), ctypes.c_void_p(self.wp.data_ptr()), M, self.N, self.K,
             ctypes.c_void_p(res.data_ptr()), res.stride(0),
-            ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)), "gemm_bf16_residual")
+            _lib.stream_handle(x.device.index)), "gemm_bf16_residual")
         return True
 
     def _gemv_x(self, x: torch.Tensor, norm_w):
@@ -469,7 +468,7 @@ class _Linear:
         _lib.check(self.hip._L.vnx_gemv_w4_rope_kv(
             xp, ldx, nwp, float(eps), ctypes.c_void_p(self.wq_rope.data_ptr()), self.wq_rope.stride(0),
             ctypes.c_void_p(self.sc_rope.data_ptr()), _lib.VNX_F16, self.sc_rope.stride(0), M, self.N, self.K, 128,
-            ctypes.byref(rk), ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)), "gemv_w4_rope_kv")
+            ctypes.byref(rk), _lib.stream_handle(x.device.index)), "gemv_w4_rope_kv")
         return True
 
     def rope_kv_embed(self, tokens: torch.Tensor, emb: torch.Tensor, scale: float, x: torch.Tensor, rk,
@@ -487,7 +486,7 @@ class _Linear:
             P(tokens.data_ptr()), P(emb.data_ptr()), _lib.VNX_BF16, emb.stride(0), emb.shape[0], float(scale),
             P(x.data_ptr()), x.stride(0), P(norm_w.data_ptr()), float(eps), P(self.wq_rope.data_ptr()),
             self.wq_rope.stride(0), P(self.sc_rope.data_ptr()), _lib.VNX_F16, self.sc_rope.stride(0), M, self.N,
-            self.K, 128, ctypes.byref(rk), P(torch.cuda.current_stream(x.device).cuda_stream)),
+            self.K, 128, ctypes.byref(rk), _lib.stream_handle(x.device.index)),
             "gemv_w4_rope_kv_embed")
         return True
 
@@ -505,7 +504,7 @@ class _Linear:
         _lib.check(self.hip._L.vnx_gemv_w4_swiglu(
             xp, ldx, nwp, float(eps), ctypes.c_void_p(self.wq_sw.data_ptr()), self.wq_sw.stride(0),
             ctypes.c_void_p(self.sc_sw.data_ptr()), _lib.VNX_F16, self.sc_sw.stride(0), M, self.N, self.K, 128,
-            ctypes.c_void_p(y.data_ptr()), H, ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)),
+            ctypes.c_void_p(y.data_ptr()), H, _lib.stream_handle(x.device.index)),
             "gemv_w4_swiglu")
         return y
 
@@ -520,7 +519,7 @@ class _Linear:
             ctypes.c_void_p(x16.data_ptr()), self.K, ctypes.c_void_p(self.wq.data_ptr()), self.wq.stride(0),
             ctypes.c_void_p(self.sc.data_ptr()), _lib.VNX_F16, self.sc.stride(0), M, self.N, self.K, 128,
             ctypes.c_void_p(res.data_ptr()), res.stride(0),
-            ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)), "gemv_w4_residual")
+            _lib.stream_handle(x.device.index)), "gemv_w4_residual")
         return True
 
     def __call__(self, x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -539,7 +538,7 @@ class _Linear:
                     ctypes.c_void_p(x16.data_ptr()), self.K, ctypes.c_void_p(self.wt.data_ptr()),
                     ctypes.c_void_p(self.sc.data_ptr()), self.sc.stride(0), M, self.N, self.K,
                     ctypes.c_void_p(y.data_ptr()), _lib.VNX_BF16 if y.dtype == torch.bfloat16 else _lib.VNX_F32,
-                    y.stride(0), ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)), "gemv_w4_tiles")
+                    y.stride(0), _lib.stream_handle(x.device.index)), "gemv_w4_tiles")
                 return y
             if y.dtype != torch.float32:
                 raise ValueError("the INT4 GEMV writes fp32")
@@ -547,7 +546,7 @@ class _Linear:
                 ctypes.c_void_p(x16.data_ptr()), self.K, ctypes.c_void_p(self.wq.data_ptr()), self.wq.stride(0),
                 ctypes.c_void_p(self.sc.data_ptr()), _lib.VNX_F16, self.sc.stride(0), M, self.N, self.K, 128,
                 ctypes.c_void_p(y.data_ptr()), y.stride(0), ctypes.c_void_p(self._ws.data_ptr()),
-                self._ws.numel(), ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)), "gemv_w4")
+                self._ws.numel(), _lib.stream_handle(x.device.index)), "gemv_w4")
             return y
         y = self.gemm(x) if out is None else None
         if y is not None:
@@ -700,8 +699,8 @@ class CometSparkGPU:
         return cls(cfg, W, hip, batch, capacity, dtype, int4)
 
     # ---- pieces ---------------------------------------------------------
-    def _st(self) -> ctypes.c_void_p:
-        return ctypes.c_void_p(torch.cuda.current_stream(self.dev).cuda_stream)
+    def _st(self) -> int:
+        return _lib.stream_handle(self.hip._index)
 
     def _rms(self, x: torch.Tensor, res: Optional[torch.Tensor], w: torch.Tensor, y: torch.Tensor) -> None:
         """x += res (in place, res may be None); y = RMSNorm(x) * w (vnx_rmsnorm)."""
