@@ -90,7 +90,13 @@ struct TreeAttnParams {
   const float* sin;
   int rope;
   int64_t cap;                      // rows at or past it are not written (and not rotated past the table)
-  uint64_t anc_in[kTaMaxN];         // the shared ancestor words, when anc is NULL
+};
+
+// The shared ancestor words by value, read when anc is NULL.  An argument of
+// its own: indexed by lane, it would keep the compiler from loading the other
+// arguments once at entry.
+struct TreeWords {
+  uint64_t w[kTaMaxN];
 };
 
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
@@ -163,7 +169,7 @@ constexpr bool ta_variant_ok(int D, int QT, int NW, int PF) {
 // keep every wave resident; deeper rings take one workgroup per CU (up to
 // 512 registers a lane, VGPRs and AGPRs) and keep more bytes in flight.
 template <int D, int QT, int OT, int NW, int PF, bool EXT>
-__global__ __launch_bounds__(NW * 64, (PF == 2 && D == 64 && NW == 4) ? 2 : 1) void k_tree_attn(TreeAttnParams p) {
+__global__ __launch_bounds__(NW * 64, (PF == 2 && D == 64 && NW == 4) ? 2 : 1) void k_tree_attn(TreeAttnParams p, TreeWords tw) {
   constexpr int KS = D / 32;          // MFMA k-steps over the head dimension
   constexpr int DT = D / 16;          // 16-wide dimension tiles of O
   constexpr int R = TaSmem<D, QT, NW>::R;
@@ -273,7 +279,14 @@ __global__ __launch_bounds__(NW * 64, (PF == 2 && D == 64 && NW == 4) ? 2 : 1) v
     }
   }
   // Ancestor words of this lane's query columns.
-  auto word = [&](int node) -> uint64_t { return p.anc ? p.anc[b * p.anc_sb + node] : p.anc_in[node]; };
+  // (Two loads of two address spaces under a uniform branch: one load through
+  // a selected pointer would be a flat one, which also counts against the LDS
+  // counter; it cost the verify calls 1 us.)
+  auto word = [&](int node) -> uint64_t {
+    typedef const __attribute__((address_space(1))) uint64_t* gptr;
+    if (p.anc) return *(gptr)(p.anc + b * p.anc_sb + node);
+    return tw.w[node];
+  };
   uint64_t anc[QT];
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
@@ -752,30 +765,30 @@ static int ta_waves(int D, int QT, int64_t nwg, int force, bool ext) {
 }
 
 template <int D, int OT, int NW, int PF, bool EXT>
-static void ta_launch_qt(const TreeAttnParams& p, int QT, dim3 grid, hipStream_t st) {
+static void ta_launch_qt(const TreeAttnParams& p, const TreeWords& tw, int QT, dim3 grid, hipStream_t st) {
   const dim3 block(NW * 64);
   switch (QT) {
     case 1:
       if constexpr (ta_variant_ok(D, 1, NW, PF))
-        hipLaunchKernelGGL((k_tree_attn<D, 1, OT, NW, PF, EXT>), grid, block, 0, st, p);
+        hipLaunchKernelGGL((k_tree_attn<D, 1, OT, NW, PF, EXT>), grid, block, 0, st, p, tw);
       break;
     case 2:
       if constexpr (ta_variant_ok(D, 2, NW, PF))
-        hipLaunchKernelGGL((k_tree_attn<D, 2, OT, NW, PF, EXT>), grid, block, 0, st, p);
+        hipLaunchKernelGGL((k_tree_attn<D, 2, OT, NW, PF, EXT>), grid, block, 0, st, p, tw);
       break;
     case 3:
       if constexpr (ta_variant_ok(D, 3, NW, PF))
-        hipLaunchKernelGGL((k_tree_attn<D, 3, OT, NW, PF, EXT>), grid, block, 0, st, p);
+        hipLaunchKernelGGL((k_tree_attn<D, 3, OT, NW, PF, EXT>), grid, block, 0, st, p, tw);
       break;
     default:
       if constexpr (ta_variant_ok(D, 4, NW, PF))
-        hipLaunchKernelGGL((k_tree_attn<D, 4, OT, NW, PF, EXT>), grid, block, 0, st, p);
+        hipLaunchKernelGGL((k_tree_attn<D, 4, OT, NW, PF, EXT>), grid, block, 0, st, p, tw);
       break;
   }
 }
 
 template <int D, int OT>
-static int ta_launch_d(TreeAttnParams p, int QT, bool ext, int force_waves, hipStream_t st, hipEvent_t* ev) {
+static int ta_launch_d(TreeAttnParams p, const TreeWords& tw, int QT, bool ext, int force_waves, hipStream_t st, hipEvent_t* ev) {
   const int64_t nwg = (int64_t)p.B * p.Hkv * p.G * p.S;
   const dim3 grid((unsigned)nwg);
   const int nw = ta_waves(D, QT, nwg, force_waves, ext);
@@ -794,15 +807,15 @@ static int ta_launch_d(TreeAttnParams p, int QT, bool ext, int force_waves, hipS
   }
   if (ev) VNX_HIP_CHECK(hipEventRecord(ev[0], st));
   if (ext) {
-    if (nw == 8) ta_launch_qt<D, OT, 8, 0, true>(p, QT, grid, st);
-    else ta_launch_qt<D, OT, 4, 0, true>(p, QT, grid, st);
+    if (nw == 8) ta_launch_qt<D, OT, 8, 0, true>(p, tw, QT, grid, st);
+    else ta_launch_qt<D, OT, 4, 0, true>(p, tw, QT, grid, st);
   } else {
     switch (nw) {
-      case 16: ta_launch_qt<D, OT, 16, 0, false>(p, QT, grid, st); break;
-      case 8: ta_launch_qt<D, OT, 8, 0, false>(p, QT, grid, st); break;
-      case 5: ta_launch_qt<D, OT, 4, 2, false>(p, QT, grid, st); break;
-      case 9: ta_launch_qt<D, OT, 8, 2, false>(p, QT, grid, st); break;
-      default: ta_launch_qt<D, OT, 4, 0, false>(p, QT, grid, st); break;
+      case 16: ta_launch_qt<D, OT, 16, 0, false>(p, tw, QT, grid, st); break;
+      case 8: ta_launch_qt<D, OT, 8, 0, false>(p, tw, QT, grid, st); break;
+      case 5: ta_launch_qt<D, OT, 4, 2, false>(p, tw, QT, grid, st); break;
+      case 9: ta_launch_qt<D, OT, 8, 2, false>(p, tw, QT, grid, st); break;
+      default: ta_launch_qt<D, OT, 4, 0, false>(p, tw, QT, grid, st); break;
     }
   }
   VNX_LAUNCH_CHECK();
@@ -1182,8 +1195,9 @@ int vnx_tree_attn(const vnx_tree_attn_args* a, void* workspace, size_t workspace
   p.kt = static_cast<const uint16_t*>(a->k_tree);
   p.vt = static_cast<const uint16_t*>(a->v_tree);
   p.anc = a->anc;
+  TreeWords tw{};
   if (!a->anc)
-    for (int i = 0; i < N; ++i) p.anc_in[i] = a->anc_host[i];
+    for (int i = 0; i < N; ++i) tw.w[i] = a->anc_host[i];
   p.out = a->out;
   p.q_sb = a->q_strides[0]; p.q_sh = a->q_strides[1]; p.q_sr = a->q_strides[2];
   p.c_sb = a->cache_strides[0]; p.c_sh = a->cache_strides[1]; p.c_sr = a->cache_strides[2];
@@ -1225,12 +1239,12 @@ int vnx_tree_attn(const vnx_tree_attn_args* a, void* workspace, size_t workspace
   const int ot = a->out_dtype == VNX_F32 ? 0 : a->out_dtype == VNX_BF16 ? 1 : 2;
   const int fw = a->force_waves;
   if (d == 64)
-    return ot == 0   ? ta_launch_d<64, 0>(p, pl.QT, ext, fw, st, ev)
-           : ot == 1 ? ta_launch_d<64, 1>(p, pl.QT, ext, fw, st, ev)
-                     : ta_launch_d<64, 2>(p, pl.QT, ext, fw, st, ev);
-  return ot == 0   ? ta_launch_d<128, 0>(p, pl.QT, ext, fw, st, ev)
-         : ot == 1 ? ta_launch_d<128, 1>(p, pl.QT, ext, fw, st, ev)
-                   : ta_launch_d<128, 2>(p, pl.QT, ext, fw, st, ev);
+    return ot == 0   ? ta_launch_d<64, 0>(p, tw, pl.QT, ext, fw, st, ev)
+           : ot == 1 ? ta_launch_d<64, 1>(p, tw, pl.QT, ext, fw, st, ev)
+                     : ta_launch_d<64, 2>(p, tw, pl.QT, ext, fw, st, ev);
+  return ot == 0   ? ta_launch_d<128, 0>(p, tw, pl.QT, ext, fw, st, ev)
+         : ot == 1 ? ta_launch_d<128, 1>(p, tw, pl.QT, ext, fw, st, ev)
+                   : ta_launch_d<128, 2>(p, tw, pl.QT, ext, fw, st, ev);
 }
 
 int vnx_tree_attn_plan(int B, int H, int Hkv, int N, int Tp, int d, int* splits, int* groups, int* chunk) {
