@@ -60,11 +60,13 @@ def _check(y, x, w, epi, cw=None):
 
 # the three tile shapes (128 x 256, 64 x 256, 64 x 128), remainders of rows,
 # columns (element stores past N % 32) and chunks (odd and a single one), the
-# line of the dispatch (2,048 tiles) from both sides
+# line of the dispatch (2,048 tiles) from both sides, one row tile of a W past
+# 64 MB (read past the caches)
 @pytest.mark.parametrize("M,N,K,epi,dtype", [
     (4099, 2080, 192, 0, torch.bfloat16), (16384, 1024, 64, 1, torch.bfloat16),
     (2048, 2048, 128, 0, torch.float32), (2017, 2080, 320, 1, torch.float16), (1000, 2053, 64, 0, torch.bfloat16),
-    (1030, 1985, 448, 0, torch.float32), (1024, 2048, 1024, 0, torch.bfloat16), (1024, 2016, 1024, 0, torch.bfloat16)])
+    (1030, 1985, 448, 0, torch.float32), (1024, 2048, 1024, 0, torch.bfloat16), (1024, 2016, 1024, 0, torch.bfloat16),
+    (97, 131105, 320, 0, torch.float32), (128, 131072, 320, 0, torch.bfloat16)])
 def test_wide_gemm(hip, M, N, K, epi, dtype):
     print("wide gemm", M, N, K, epi, dtype, flush=True)
     x, w = _inputs(hip, M, N, K, 1, seed=M + N)

@@ -29,10 +29,18 @@
 namespace vnx {
 namespace {
 
+// 16 bytes of W; NT: past the caches.
+template <bool NT>
+__device__ __forceinline__ u32x4 ld_w(const uint16_t* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+  else return *reinterpret_cast<const u32x4*>(p);
+}
+
 // RT x CT tiles per wave; PD register sets of W and X (PD 1: one set, each W
 // register reloaded as soon as its products are issued); LA: A operands of LA
-// 16-k steps read ahead (PD 1; else the whole chunk's); OCC workgroups per CU.
-template <int OT, int EPI, int RT, int CT, int PD, int LA, int OCC>
+// 16-k steps read ahead (PD 1; else the whole chunk's); OCC workgroups per CU; NT: W
+// is read past the caches (wg_run's rule).
+template <int OT, int EPI, int RT, int CT, int PD, int LA, int OCC, bool NT = false>
 __global__ __launch_bounds__(256, OCC) void k_wgemm(WgParams p) {
   constexpr int ROWS = 32 * RT;
   constexpr int UN = PD;
@@ -120,7 +128,7 @@ __global__ __launch_bounds__(256, OCC) void k_wgemm(WgParams p) {
 #pragma unroll
     for (int t = 0; t < CT; ++t)
 #pragma unroll
-      for (int s = 0; s < 4; ++s) v[t][s] = *reinterpret_cast<const u32x4*>(wt[t] + (cc * 4 + s) * 512);
+      for (int s = 0; s < 4; ++s) v[t][s] = ld_w<NT>(wt[t] + (cc * 4 + s) * 512);
   };
   // Every load in the order of the loop, X(c + 1) before W(c): the waits the
   // compiler derives for the loop's first chunk then leave as many loads in
@@ -167,7 +175,7 @@ __global__ __launch_bounds__(256, OCC) void k_wgemm(WgParams p) {
               acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_b8(a[s][i]), as_b8(wv[0][t][s]), acc[i][t], 0, 0, 0);
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int t = 0; t < CT; ++t) wv[0][t][s] = *reinterpret_cast<const u32x4*>(wt[t] + (cw * 4 + s) * 512);
+          for (int t = 0; t < CT; ++t) wv[0][t][s] = ld_w<NT>(wt[t] + (cw * 4 + s) * 512);
           __builtin_amdgcn_sched_barrier(0);
         }
       } else {
@@ -338,8 +346,22 @@ int wg_run(WgParams p, int epi, int y_dtype, hipStream_t s) {
   const int64_t wgs = (tiles + kVgXcds - 1) / kVgXcds * kVgXcds;
   if (wgs >= INT_MAX) return VNX_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)wgs);
+  // One row tile reads each byte of W once.  A W past 64 MB then leaves nothing
+  // in the caches that this launch would read again, and pushes out the layers
+  // the next launches read, so it streams past them: the 248,320 x 512 head at
+  // 4-128 rows 89-110 -> 87-103 us, and a 4-layer verify of 8 x 7 tokens around
+  // it 344 -> 330 us.  From two row tiles on the second read has to hit: at 224
+  // rows 143 us cached, 181 us streamed.
+  const bool nt = p.M <= 128 && (int64_t)p.N * p.K * 2 > ((int64_t)64 << 20);
   auto shape = [&](auto ot, auto ep) -> int {
     constexpr int OT = decltype(ot)::value, EP = decltype(ep)::value;
+    if constexpr (EP == 0) {
+      if (sh == 0 && nt) {
+        hipLaunchKernelGGL((k_wgemm<OT, EP, 4, 2, 1, 2, 2, true>), grid, dim3(256), 0, s, p);
+        VNX_LAUNCH_CHECK();
+        return VNX_OK;
+      }
+    }
     if (sh == 0) hipLaunchKernelGGL((k_wgemm<OT, EP, 4, 2, 1, 2, 2>), grid, dim3(256), 0, s, p);
     else if (sh == 1) hipLaunchKernelGGL((k_wgemm<OT, EP, 2, 2, 1, 1, 3>), grid, dim3(256), 0, s, p);
     else hipLaunchKernelGGL((k_wgemm<OT, EP, 2, 1, 2, 4, 2>), grid, dim3(256), 0, s, p);
