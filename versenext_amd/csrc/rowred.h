@@ -270,4 +270,136 @@ __device__ __forceinline__ T ld_agent(const T* p) {
   return __hip_atomic_load(const_cast<T*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// ---------------------------------------------------------------------------
+// The inverse-CDF walk over a row's sub-block masses, by one workgroup of NT
+// threads: thread t owns sub-blocks [t*q, (t+1)*q), q = ceil(nsb/NT); the
+// total is sum_t (sum_i m[t*q + i]) in that nested order, and the walk to the
+// target follows the same order: thread, sub-block, then (walk_pick) lane and
+// element.  The workgroup that runs it is alone on the critical path of its
+// launch and runs most of this code once, so what it costs is the fetch of
+// the instructions: loops stay rolled and reductions go through ballots.
+// ---------------------------------------------------------------------------
+template <int NT>
+struct WalkLds {
+  double E[NT];            // inclusive scan of the threads' sums
+  double scan[NT / VNX_WAVE];
+  int first[NT / VNX_WAVE], last[NT / VNX_WAVE];
+  double base;             // cumulative mass before the sub-block found
+  int sb;                  // that sub-block (-1: no mass at all)
+};
+
+// The masses the other workgroups published, into LDS (four loads a thread in
+// flight).
+template <int NT>
+__device__ __forceinline__ void walk_load(const double* sbm, int nsb, double* sh_m) {
+#pragma unroll 1
+  for (int i0 = threadIdx.x; i0 < nsb; i0 += 4 * NT) {
+    double v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = ld_agent(sbm + min(i0 + j * NT, nsb - 1));
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (i0 + j * NT < nsb) sh_m[i0 + j * NT] = v[j];
+  }
+}
+
+// The total of the row's masses; L.E holds every thread's end, *own this
+// thread's sum.
+template <int NT>
+__device__ __forceinline__ double walk_total(const double* sh_m, int nsb, WalkLds<NT>& L, double* own) {
+  const int tid = threadIdx.x, q = (nsb + NT - 1) / NT;
+  __syncthreads();
+  double t = 0.0;
+#pragma unroll 1
+  for (int i = tid * q; i < min((tid + 1) * q, nsb); ++i) t += sh_m[i];
+  const double incl = block_inclusive_scan<NT>(t, L.scan);
+  L.E[tid] = incl;
+  *own = t;
+  // each wave's last thread with mass
+  const uint64_t pos = __ballot(t > 0.0);
+  if (tid % VNX_WAVE == 0) L.last[tid / VNX_WAVE] = pos ? tid + 63 - __builtin_clzll(pos) : -1;
+  __syncthreads();
+  return L.E[NT - 1];
+}
+
+// The first thread whose range [start, end) holds the target (ranges of zero
+// mass are empty; the last thread with mass if rounding leaves none), then
+// its sub-blocks in order: L.sb, L.base.
+template <int NT>
+__device__ __forceinline__ void walk_find(const double* sh_m, int nsb, double own, double target,
+                                          WalkLds<NT>& L) {
+  const int tid = threadIdx.x, q = (nsb + NT - 1) / NT;
+  const int w = tid / VNX_WAVE;
+  const double start = tid ? L.E[tid - 1] : 0.0, end = L.E[tid];
+  const uint64_t hit = __ballot(own > 0.0 && start <= target && target < end);
+  if (tid % VNX_WAVE == 0) {
+    L.first[w] = hit ? tid + (int)__builtin_ctzll(hit) : NT;
+    if (w == 0) L.sb = -1;
+  }
+  __syncthreads();
+  int ts = NT, tl = -1;
+#pragma unroll
+  for (int j = 0; j < NT / VNX_WAVE; ++j) {
+    ts = min(ts, L.first[j]);
+    tl = max(tl, L.last[j]);
+  }
+  if (ts == NT) ts = tl;
+  if (tid == ts) {
+    int sstar = -1, slast = -1;
+    double run = start, base = start, blast = start;
+#pragma unroll 1
+    for (int i = tid * q; i < min((tid + 1) * q, nsb); ++i) {
+      const double m = sh_m[i];
+      if (m > 0.0) {
+        if (sstar < 0 && run + m > target) { sstar = i; base = run; }
+        slast = i;
+        blast = run;
+      }
+      run += m;
+    }
+    L.sb = sstar < 0 ? slast : sstar;
+    L.base = sstar < 0 ? blast : base;
+  }
+  __syncthreads();
+}
+
+// One wave: the element of its sub-block that holds the target.  w: this
+// lane's weights in element order, lm their sum, e0 its first element;
+// base = the mass before the sub-block.  *edge: the target within 1e-12 of
+// the total of the element's bounds, or past every one (the last positive
+// weight then; the sub-block's first element if there is none).
+template <int VE>
+__device__ __forceinline__ int64_t walk_pick(const float (&w)[VE], double lm, int64_t e0, double base, double tgt,
+                                             double total, bool* edge_out) {
+  const int lane = threadIdx.x % VNX_WAVE;
+  const double incl = wave_inclusive_scan(lm);
+  const double start = base + (incl - lm), end = base + incl;
+  const uint64_t hits = __ballot(lm > 0.0 && start <= tgt && tgt < end);
+  const uint64_t pos = __ballot(lm > 0.0);
+  bool edge = hits == 0;
+  const int lstar = hits ? (int)__builtin_ctzll(hits) : pos ? 63 - (int)__builtin_clzll(pos) : 0;
+  int64_t token = e0;
+  if (pos && lane == lstar) {
+    double run = start, before = start, after = end;
+    int pick = -1, lastpos = -1;
+#pragma unroll
+    for (int i = 0; i < VE; ++i) {
+      if (w[i] > 0.0f) {
+        lastpos = i;
+        if (pick < 0) {
+          const double nr = run + (double)w[i];
+          if (nr > tgt) { pick = i; before = run; after = nr; }
+          run = nr;
+        }
+      }
+    }
+    if (pick < 0) { pick = lastpos; edge = true; }
+    token = e0 + pick;
+    const double tol = 1e-12 * total;
+    if (tgt - before < tol || after - tgt < tol) edge = true;
+  }
+  *edge_out = __shfl((int)edge, lstar, VNX_WAVE) != 0;
+  return __shfl(token, lstar, VNX_WAVE);
+}
+
 }  // namespace vnx

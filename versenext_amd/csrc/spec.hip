@@ -83,7 +83,8 @@ struct SpecParams {
   float* part_m;   // [B*(2k+1)][chunks]
   double* part_s;  // [B*(2k+1)][chunks]
   double* sbm;     // [B][nsb] sub-block draw masses
-  unsigned* cnt;   // [B] arrival counters of launch B
+  unsigned* cnt;   // [B] arrival counters of launch B, cnt_ld apart
+  int64_t cnt_ld;
   float* gath;     // [B][2k] scaled target / draft logits at the draft ids
   // Draft rows' LSEs supplied by the caller (the draws that produced the
   // draft ids computed them): lse_din[i * ld_din + b] = RN32(LSE of q_i / T),
@@ -301,20 +302,9 @@ __device__ __forceinline__ Job accept_row(const SpecParams& p, int64_t b, bool w
 }
 
 // ---------------------------------------------------------------------------
-// Draw weights.  W_RESID: max(0, p - q); W_P: p.  p = E(a - Lp), q = E(b - Lq),
-// E = vnx_exp_canon, a / b the exact scaled logits.
+// Draw weights: max(0, p - q) (residual draw) or p.  p = E(a - Lp),
+// q = E(b - Lq), E = vnx_exp_canon, a / b the exact scaled logits.
 // ---------------------------------------------------------------------------
-enum { W_RESID = 0, W_P = 1 };
-
-template <int SM, bool THR>
-__device__ __forceinline__ float draw_weight(float lp, float lq, int wsel, const TScale& sc, float thr_p,
-                                             float thr_q, float Lp, float Lq) {
-  const float pp = vnx_exp_canon(scaled<SM, THR>(lp, sc, thr_p) - Lp);
-  if (wsel == W_P) return pp;
-  const float d = pp - vnx_exp_canon(scaled<SM, THR>(lq, sc, thr_q) - Lq);
-  return d > 0.0f ? d : 0.0f;
-}
-
 // Rows drawn from for batch row b (p_n / q_n, or p_k for the bonus draw).
 struct DrawRows {
   int64_t poff, qoff;
@@ -336,23 +326,8 @@ __device__ __forceinline__ DrawRows draw_rows(const SpecParams& p, int64_t b, co
   return d;
 }
 
-// Raw logits of this lane's vector of sub-block sbi (elements
-// sbi*64*VE + lane*VE + [0, VE)); elements past V read as -inf, whose weight is 0.
-template <typename Tin>
-__device__ __forceinline__ void lane_vec(const Tin* row, int64_t sbi, int64_t V, float (&x)[Vec<Tin>::N]) {
-  constexpr int VE = Vec<Tin>::N;
-  const int64_t e = (sbi * VNX_WAVE + (threadIdx.x % VNX_WAVE)) * VE;
-  if (e + VE <= V) {
-    Vec<Tin>::load(row + e, x);
-  } else {
-#pragma unroll
-    for (int i = 0; i < VE; ++i) x[i] = e + i < V ? Vec<Tin>::load1(row + e + i) : kNegInf;
-  }
-}
-
-// The same vector as raw bits (elements past V carry -inf bits), converted
-// later: a conversion beside the load would wait for it there, and with it for
-// every load issued before it.
+// Raw bits of this lane's vector of sub-block sbi (elements sbi*64*VE +
+// lane*VE + [0, VE)); elements past V carry -inf bits, whose weight is 0.
 template <typename Tin>
 __device__ __forceinline__ u32x4 lane_raw(const Tin* row, int64_t sbi, int64_t V) {
   constexpr int VE = Vec<Tin>::N;
@@ -374,245 +349,6 @@ __device__ __forceinline__ u32x4 lane_raw(const Tin* row, int64_t sbi, int64_t V
   return u32x4{w[0], w[1], w[2], w[3]};
 }
 
-// Draw mass of this lane's vector of sub-block sbi (sequential fp64 sum in
-// element order), and its weights.
-template <typename Tin, int SM, bool THR>
-__device__ __forceinline__ double lane_weights(const Tin* P, const Tin* Q, int64_t sbi, int64_t V, int wsel,
-                                               const TScale& sc, const DrawRows& d, const Job& jb,
-                                               float (&w)[Vec<Tin>::N]) {
-  constexpr int VE = Vec<Tin>::N;
-  float xp[VE], xq[VE];
-  lane_vec<Tin>(P, sbi, V, xp);
-  if (wsel == W_RESID) lane_vec<Tin>(Q, sbi, V, xq);
-  double m = 0.0;
-#pragma unroll
-  for (int i = 0; i < VE; ++i) {
-    w[i] = draw_weight<SM, THR>(xp[i], wsel == W_RESID ? xq[i] : 0.0f, wsel, sc, d.thr_p, d.thr_q, jb.Lp, jb.Lq);
-    m += (double)w[i];
-  }
-  return m;
-}
-
-// ---------------------------------------------------------------------------
-// mass: chunk c of batch row b = sub-blocks [c*spc, (c+1)*spc); wave w takes
-// sub-blocks c*spc + w + kNW*j, so the workgroup's loads are contiguous.
-// ---------------------------------------------------------------------------
-template <typename Tin, int SM, bool THR, int WSEL>
-__device__ __forceinline__ void mass_chunk(const SpecParams& p, int64_t b, int c, int spc, const Tin* P,
-                                           const Tin* Q, const DrawRows& d, const Job& jb) {
-  constexpr int VE = Vec<Tin>::N;
-  const int wave = threadIdx.x / VNX_WAVE;
-  const int64_t s0 = (int64_t)c * spc;
-  const int64_t s1 = min(s0 + spc, p.nsb);
-  for (int64_t sb = s0 + wave; sb < s1; sb += (int64_t)kNW * kNB2) {
-    // every load of the batch in flight first (raw bits), then the weights
-    u32x4 rp[kNB2], rq[kNB2];
-#pragma unroll
-    for (int j = 0; j < kNB2; ++j) {
-      const int64_t sbi = sb + (int64_t)kNW * j;
-      rp[j] = rq[j] = u32x4{0u, 0u, 0u, 0u};
-      if (sbi < s1) {
-        rp[j] = lane_raw<Tin>(P, sbi, p.V);
-        if constexpr (WSEL == W_RESID) rq[j] = lane_raw<Tin>(Q, sbi, p.V);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < kNB2; ++j) {
-      const int64_t sbi = sb + (int64_t)kNW * j;
-      if (sbi < s1) {
-        float xp[VE], xq[VE];
-        Vec<Tin>::cvt_raw(rp[j], xp);
-        if constexpr (WSEL == W_RESID) Vec<Tin>::cvt_raw(rq[j], xq);
-        double m = 0.0;
-#pragma unroll
-        for (int i = 0; i < VE; ++i)
-          m += (double)draw_weight<SM, THR>(xp[i], WSEL == W_RESID ? xq[i] : 0.0f, WSEL, p.sc, d.thr_p,
-                                            d.thr_q, jb.Lp, jb.Lq);
-        m = wave_sum(m);
-        if (threadIdx.x % VNX_WAVE == 0) st_agent(&p.sbm[b * p.nsb + sbi], m);
-      }
-    }
-  }
-  // every wave's published masses complete before the workgroup arrives
-  __builtin_amdgcn_s_waitcnt(0);
-}
-
-// ---------------------------------------------------------------------------
-// draw: thread t owns sub-blocks [t*q, (t+1)*q) (q = ceil(nsb/kNT)); the
-// total is sum_t (sum_i sbm[t*q+i]) in that nested sequential order, and the
-// walk to the target follows the same order: thread, then sub-block, then
-// (one wave, lane-order inclusive scan) lane, then element.  sh_m holds the
-// row's nsb sub-block masses (dynamic LDS), published by the other
-// workgroups of launch B (coherent loads).
-// ---------------------------------------------------------------------------
-struct DrawLds {
-  double T[kNT], E[kNT];
-  double scan[kNW];
-  double total, target, base;
-  int64_t sb;
-  int tstar, tlast;
-};
-
-template <typename Tin, int SM, bool THR>
-__device__ __forceinline__ void draw_work(const SpecParams& p, int64_t b, const Job& jb, DrawLds& L, double* sh_m) {
-  constexpr int VE = Vec<Tin>::N;
-  const int k = p.k;
-  const int tid = threadIdx.x;
-  const DrawRows d = draw_rows<THR>(p, b, jb);
-  const Tin* P = static_cast<const Tin*>(p.tgt) + d.poff;
-  const Tin* Q = static_cast<const Tin*>(p.dft) + d.qoff;
-  double* sbm = p.sbm + b * p.nsb;
-  const int64_t q = (p.nsb + kNT - 1) / kNT;  // <= kDrawLds / kNT (host check)
-  int wsel = jb.mode == 0 ? W_RESID : W_P;
-  uint8_t fl = 0;
-
-  // All sub-block masses into LDS (one load per element, all in flight);
-  // thread t sums its q consecutive sub-blocks in order (T_t); an inclusive
-  // block scan of T_t in thread order gives every thread its range
-  // [start_t, end_t), and the total is the scan's last value, so the total
-  // and the ranges come from the same sums.
-  auto scan_totals = [&]() {
-    __syncthreads();
-    double t = 0.0;
-    for (int64_t i = (int64_t)tid * q; i < min((int64_t)(tid + 1) * q, p.nsb); ++i) t += sh_m[i];
-    const double incl = block_inclusive_scan<kNT>(t, L.scan);
-    L.T[tid] = t;
-    L.E[tid] = incl;
-    __syncthreads();
-    if (tid == kNT - 1) L.total = incl;
-    __syncthreads();
-  };
-  {
-    // every load in flight first (at most kDrawLds / kNT per thread), then
-    // the LDS stores
-    double v[kDrawLds / kNT];
-#pragma unroll
-    for (int j = 0; j < kDrawLds / kNT; ++j) {
-      const int64_t i = tid + (int64_t)j * kNT;
-      v[j] = i < p.nsb ? ld_agent(&sbm[i]) : 0.0;
-    }
-#pragma unroll
-    for (int j = 0; j < kDrawLds / kNT; ++j) {
-      const int64_t i = tid + (int64_t)j * kNT;
-      if (i < p.nsb) sh_m[i] = v[j];
-    }
-  }
-  scan_totals();
-  if (!(L.total > 0.0) && wsel == W_RESID) {
-    // max(0, p_n - q_n) has no mass (p_n == q_n after rounding): draw from
-    // p_n.  This workgroup recomputes the sub-block masses of p_n (rare path).
-    fl |= VNX_FLAG_ZERO_RESIDUAL;
-    wsel = W_P;
-    for (int64_t sbi = tid / VNX_WAVE; sbi < p.nsb; sbi += kNW) {
-      float w[VE];
-      const double m = wave_sum(lane_weights<Tin, SM, THR>(P, Q, sbi, p.V, wsel, p.sc, d, jb, w));
-      if (tid % VNX_WAVE == 0) sh_m[sbi] = m;
-    }
-    scan_totals();
-  }
-  // The thread whose range holds target = u * total (ranges of zero mass are
-  // empty); if rounding leaves none, the last thread with positive mass.
-  if (tid == 0) {
-    L.tstar = kNT;  // atomicMin sentinel: no thread
-    L.tlast = -1;
-  }
-  __syncthreads();
-  const double total = L.total;
-  const double target = (double)jb.u * total;
-  {
-    const double T = L.T[tid], end = L.E[tid];
-    const double start = tid ? L.E[tid - 1] : 0.0;
-    if (T > 0.0 && start <= target && target < end) atomicMin(&L.tstar, tid);
-    if (T > 0.0) atomicMax(&L.tlast, tid);
-  }
-  __syncthreads();
-  if (tid == 0) {
-    int tstar = L.tstar;
-    if (tstar == kNT) tstar = L.tlast;
-    int64_t sstar = -1;
-    double base = 0.0;
-    if (tstar >= 0) {
-      // Sub-blocks of that thread, in order, from the thread's start.
-      const double b0 = tstar ? L.E[tstar - 1] : 0.0;
-      double r2 = b0, b_last = b0;
-      int64_t slast = -1;
-      for (int64_t i = (int64_t)tstar * q; i < min((int64_t)(tstar + 1) * q, p.nsb); ++i) {
-        const double m = sh_m[i];
-        if (m > 0.0) {
-          if (sstar < 0 && r2 + m > target) { sstar = i; base = r2; }
-          slast = i;
-          b_last = r2;
-        }
-        r2 += m;
-      }
-      if (sstar < 0) { sstar = slast; base = b_last; }
-    }
-    L.sb = sstar;
-    L.target = target;
-    L.base = base;
-  }
-  __syncthreads();
-  const int64_t sstar = L.sb;
-  if (tid >= VNX_WAVE) return;
-  // Wave 0: the sub-block's weights, lane-order inclusive scan, element walk.
-  int64_t token = 0;
-  if (sstar < 0) {
-    fl |= VNX_FLAG_ZERO_RESIDUAL;
-  } else {
-    float w[VE];
-    const double lm = lane_weights<Tin, SM, THR>(P, Q, sstar, p.V, wsel, p.sc, d, jb, w);
-    const double incl = wave_inclusive_scan(lm);
-    const double start = L.base + (incl - lm);
-    const double end = L.base + incl;
-    const double tgt = L.target;
-    // The lane whose [start, end) holds the target; if rounding leaves the
-    // target past every lane, the last lane with positive mass.
-    const bool hit = lm > 0.0 && start <= tgt && tgt < end;
-    const uint64_t hits = __ballot(hit);
-    const uint64_t pos = __ballot(lm > 0.0);
-    const int lane = tid;
-    int lstar;
-    bool edge = false;
-    if (hits) {
-      lstar = __builtin_ctzll(hits);
-    } else {
-      lstar = pos ? 63 - __builtin_clzll(pos) : -1;
-      edge = true;
-    }
-    if (lstar < 0) {
-      token = (sstar * VNX_WAVE) * VE;
-      edge = true;
-    } else if (lane == lstar) {
-      double run = start, before = start, after = end;
-      int pick = -1, lastpos = -1;
-#pragma unroll
-      for (int i = 0; i < VE; ++i) {
-        if (w[i] > 0.0f) {
-          lastpos = i;
-          if (pick < 0) {
-            const double nr = run + (double)w[i];
-            if (nr > tgt) { pick = i; before = run; after = nr; }
-            run = nr;
-          }
-        }
-      }
-      if (pick < 0) { pick = lastpos; edge = true; }
-      token = (sstar * VNX_WAVE + lane) * VE + pick;
-      const double tol = 1e-12 * L.total;
-      if (tgt - before < tol || after - tgt < tol) edge = true;
-    }
-    if (lstar >= 0) {
-      token = __shfl(token, lstar, VNX_WAVE);
-      edge = __shfl((int)edge, lstar, VNX_WAVE) != 0;
-    }
-    if (edge) fl |= VNX_FLAG_CDF_EDGE;
-  }
-  if (tid == 0) {
-    p.out_ids[b * (k + 1) + jb.n] = token;
-    if (p.flags) p.flags[b * (k + 1) + jb.n] = (uint8_t)(jb.fln | fl);
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Launch A: chunk partials of every row; the first workgroups also clear the
 // arrival counters of launch B.
@@ -621,39 +357,178 @@ template <typename Tin, int SM, bool THR>
 __global__ __launch_bounds__(kNT) void k_spec_lse(SpecParams p) {
   __shared__ ReduceLds lds;
   const int64_t zc = (int64_t)blockIdx.x * kNT + threadIdx.x;
-  if (zc < p.B) p.cnt[zc] = 0u;
+  if (zc < p.B) p.cnt[zc * p.cnt_ld] = 0u;
   const int64_t w = blockIdx.x;
   if (w < p.B * p.rows_a * p.chunks) lse_work<Tin, SM, THR>(p, w / p.chunks, (int)(w % p.chunks), lds);
 }
 
 // ---------------------------------------------------------------------------
-// Launch B: accept of the row, draw masses of one chunk; the workgroup
-// completing batch row b draws its token.  Dynamic LDS: the row's partials
-// during the accept, then its sub-block masses if it draws.
+// Launch B: accept of the row, then the draw masses of one chunk: sub-blocks
+// [c*spc, (c+1)*spc), wave w the sub-blocks w + kNW*j of them, so the
+// workgroup's loads are contiguous.  The workgroup completing batch row b
+// walks the row's masses to u * total (rowred.h) and draws the token from the
+// sub-block there.  Dynamic LDS: the row's partials during the accept, then
+// its sub-block masses if it draws.
+//
+// Small batches are bound by latencies and, above all, by instruction fetch:
+// every phase runs once on a workgroup, and its code comes from a cache that
+// the kernels before swept.  So one rolled loop holds the only copy of the
+// weights' code, for the mass of each sub-block, for the recomputed masses of
+// a row without residual mass and for the sub-block drawn from (14 KB;
+// 40 KB with each form inlined and unrolled).  Launch B of a draw of 8 rows of
+// 248,320 in the engine's rounds: 18.6 -> 12.0 us; of one row's acceptance
+// (k = 4) 12.2 -> 10.1; both launches of 8 rows' (k = 6, bf16) 40 -> 30.5, of
+// 64 rows' (k = 8) 154 -> 151 in bf16, 202 -> 203 in fp32.
 // ---------------------------------------------------------------------------
 union MassDrawLds {
   AcceptLds acc;
-  DrawLds draw;
+  WalkLds<kNT> walk;
 };
 
 template <typename Tin, int SM, bool THR>
-__global__ __launch_bounds__(kNT) void k_spec_mass_draw(SpecParams p) {
+__global__ __launch_bounds__(kNT, 4) void k_spec_mass_draw(SpecParams p) {
+  constexpr int VE = Vec<Tin>::N;
+  constexpr int U = 8 / VE;  // sub-blocks per turn of the loop
   __shared__ MassDrawLds lds;
   __shared__ int last_flag;
   extern __shared__ double dyn[];
   const int c = blockIdx.x % p.chunks2;
   const int64_t b = blockIdx.x / p.chunks2;
-  const int total = p.rows_a * p.chunks;  // the partials' LDS, sized by the host for rows_a rows
-  const Job jb = accept_row<Tin, SM, THR>(p, b, c == 0, lds.acc, reinterpret_cast<float*>(dyn + total), dyn);
+  const int parts = p.rows_a * p.chunks;  // the partials' LDS, sized by the host for rows_a rows
+  Job jb = accept_row<Tin, SM, THR>(p, b, c == 0, lds.acc, reinterpret_cast<float*>(dyn + parts), dyn);
+  // one job for the workgroup: in scalar registers, so the loop below is
+  // scalar control over scalar row bases
+  jb.n = __builtin_amdgcn_readfirstlane(jb.n);
+  jb.mode = __builtin_amdgcn_readfirstlane(jb.mode);
+  jb.Lp = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(jb.Lp)));
+  jb.Lq = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(jb.Lq)));
   const DrawRows d = draw_rows<THR>(p, b, jb);
   const Tin* P = static_cast<const Tin*>(p.tgt) + d.poff;
   const Tin* Q = static_cast<const Tin*>(p.dft) + d.qoff;
-  if (jb.mode == 0)
-    mass_chunk<Tin, SM, THR, W_RESID>(p, b, c, p.spc, P, Q, d, jb);
-  else
-    mass_chunk<Tin, SM, THR, W_P>(p, b, c, p.spc, P, Q, d, jb);
-  if (!arrive_last(&p.cnt[b], (unsigned)p.chunks2, &last_flag)) return;
-  draw_work<Tin, SM, THR>(p, b, jb, lds.draw, dyn);
+  const int lane = threadIdx.x % VNX_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / VNX_WAVE);
+  const int nsb = (int)p.nsb;                              // <= kDrawLds
+  const int whole = (int)(p.V / (VNX_WAVE * VE));          // sub-blocks without an element past V
+  int s1 = min((c + 1) * p.spc, nsb);
+  int sb = c * p.spc + wave, j = 0;
+  bool resid = jb.mode == 0, redo = false, draw = false;   // uniform
+  int fl = 0;
+  double total = 0.0;
+  u32x4 rp[kNB2], rq[kNB2];
+  float w[U][VE];
+  double lm[U];
+  // the batch of this wave's sub-blocks from at, every load in flight first
+  auto load = [&](int at) {
+    const Tin* bp = P + ((int64_t)at * VNX_WAVE + lane) * VE;
+    const Tin* bq = Q + ((int64_t)at * VNX_WAVE + lane) * VE;
+    const int e1 = min(s1, whole);
+#pragma unroll
+    for (int t = 0; t < kNB2; ++t)
+      if (at + kNW * t < e1) rp[t] = Vec<Tin>::load_raw(bp + kNW * VNX_WAVE * VE * t);
+    if (resid)
+#pragma unroll
+      for (int t = 0; t < kNB2; ++t)
+        if (at + kNW * t < e1) rq[t] = Vec<Tin>::load_raw(bq + kNW * VNX_WAVE * VE * t);
+    j = 0;
+  };
+  load(sb);
+#pragma unroll 1
+  for (;;) {
+    if (sb >= s1) {  // this wave's masses are out (never while drawing)
+      if (!redo) {
+        // every wave's published masses complete before the workgroup arrives
+        __builtin_amdgcn_s_waitcnt(0);
+        if (!arrive_last(&p.cnt[b * p.cnt_ld], (unsigned)p.chunks2, &last_flag)) return;
+        walk_load<kNT>(p.sbm + b * nsb, nsb, dyn);
+      }
+      double own;
+      total = walk_total<kNT>(dyn, nsb, lds.walk, &own);
+      if (resid && __ballot(total > 0.0) == 0) {
+        // max(0, p_n - q_n) has no mass (p_n == q_n after rounding): draw
+        // from p_n, whose masses this workgroup computes (rare)
+        fl |= VNX_FLAG_ZERO_RESIDUAL;
+        resid = false;
+        redo = true;
+        s1 = nsb;
+        sb = wave;
+        load(sb);
+        continue;
+      }
+      walk_find<kNT>(dyn, nsb, own, (double)jb.u * total, lds.walk);
+      if (wave) return;
+      draw = true;
+      sb = __builtin_amdgcn_readfirstlane(lds.walk.sb);
+      if (sb < 0) break;
+      s1 = nsb;
+    }
+    // one sub-block (past the whole ones, or the one drawn from), or U
+    const bool one = draw || sb + kNW * (U - 1) >= whole;
+    u32x4 ap[U], aq[U];
+    if (one) {
+      ap[0] = aq[0] = lane_raw<Tin>(P, sb, p.V);
+      if (resid) aq[0] = lane_raw<Tin>(Q, sb, p.V);
+#pragma unroll
+      for (int q = 1; q < U; ++q) { ap[q] = ap[0]; aq[q] = aq[0]; }
+    } else {
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        ap[q] = rp[q];
+        aq[q] = rq[q];
+#pragma unroll
+        for (int t = U; t < kNB2; t += U)
+          if (j == t) { ap[q] = rp[t + q]; aq[q] = rq[t + q]; }
+      }
+      j += U;
+      if (j == kNB2) load(sb + kNW * U);  // under this turn's weights
+    }
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      float xp[VE];
+      Vec<Tin>::cvt_raw(ap[q], xp);
+#pragma unroll
+      for (int i = 0; i < VE; ++i) w[q][i] = vnx_exp_canon(scaled<SM, THR>(xp[i], p.sc, d.thr_p) - jb.Lp);
+    }
+    if (resid)
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        float xq[VE];
+        Vec<Tin>::cvt_raw(aq[q], xq);
+#pragma unroll
+        for (int i = 0; i < VE; ++i) {
+          const float r = w[q][i] - vnx_exp_canon(scaled<SM, THR>(xq[i], p.sc, d.thr_q) - jb.Lq);
+          w[q][i] = r > 0.0f ? r : 0.0f;
+        }
+      }
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      lm[q] = 0.0;
+#pragma unroll
+      for (int i = 0; i < VE; ++i) lm[q] += (double)w[q][i];
+    }
+    if (draw) break;
+    // lane 0 holds the first sub-block's mass, lane 32 the second's
+    static_assert(U <= 2, "");
+    const double m = U == 1 ? wave_sum(lm[0]) : wave_sum2(lm[0], lm[U - 1]);
+    const int at = sb + (lane >> 5) * kNW;
+    if ((lane & 31) == 0 && (lane == 0 || (U == 2 && !one && at < s1))) {
+      if (redo) dyn[at] = m;
+      else st_agent(&p.sbm[b * nsb + at], m);
+    }
+    sb += one ? kNW : kNW * U;
+  }
+  // wave 0 of the workgroup that draws
+  int64_t token = 0;
+  if (sb < 0) {
+    fl |= VNX_FLAG_ZERO_RESIDUAL;
+  } else {
+    bool edge;
+    token = walk_pick<VE>(w[0], lm[0], ((int64_t)sb * VNX_WAVE + lane) * VE, lds.walk.base, (double)jb.u * total, total,
+                          &edge);
+    if (edge) fl |= VNX_FLAG_CDF_EDGE;
+  }
+  if (lane == 0) {
+    p.out_ids[b * (p.k + 1) + jb.n] = token;
+    if (p.flags) p.flags[b * (p.k + 1) + jb.n] = (uint8_t)(jb.fln | fl);
+  }
 }
 
 struct SpecPlan {
@@ -703,26 +578,34 @@ static SpecPlan spec_plan(int64_t B, int k, int64_t V, int dtype, int rows_a = -
   return pl;
 }
 
-static size_t spec_carve(void* ws, int64_t B, int k, const SpecPlan& pl, SpecParams* p) {
+// Row b's arrival counter lies kCntLd counters after row b - 1's, a cache line
+// of its own: the last arrival of 8 rows on one line took 3.5 us, that of a
+// single row 1 (atomics on a line run one after the other).  A workspace that has no room for that (the
+// fixed scratch near its limit) keeps them next to each other.
+constexpr int64_t kCntLd = 32;
+
+static size_t spec_carve(void* ws, int64_t B, int k, const SpecPlan& pl, SpecParams* p, int64_t cnt_ld) {
   Carve cv(ws);
   const size_t n1 = (size_t)B * (2 * k + 1) * pl.chunks;
   float* pm = cv.take<float>(n1);
   double* ps = cv.take<double>(n1);
   double* sbm = cv.take<double>((size_t)B * pl.nsb);
-  unsigned* cnt = cv.take<unsigned>((size_t)B);
+  unsigned* cnt = cv.take<unsigned>((size_t)(B * cnt_ld));
   float* gath = cv.take<float>((size_t)B * 2 * k);
   if (p) {
     p->part_m = pm; p->part_s = ps; p->sbm = sbm; p->cnt = cnt; p->gath = gath;
+    p->cnt_ld = cnt_ld;
   }
   return cv.bytes();
 }
 
 // Workspace bound over both dtypes, with and without caller-supplied draft
 // LSEs (whose plan may cut the rows into more chunks).
-static size_t spec_ws_bytes(int64_t B, int k, int64_t V) {
+static size_t spec_ws_bytes(int64_t B, int k, int64_t V, int64_t cnt_ld) {
   size_t m = 0;
   for (int dt : {VNX_F32, VNX_BF16})
-    for (int ra : {2 * k + 1, k + 1}) m = std::max(m, spec_carve(nullptr, B, k, spec_plan(B, k, V, dt, ra), nullptr));
+    for (int ra : {2 * k + 1, k + 1})
+      m = std::max(m, spec_carve(nullptr, B, k, spec_plan(B, k, V, dt, ra), nullptr, cnt_ld));
   return m;
 }
 
@@ -822,7 +705,7 @@ extern "C" {
 
 size_t vnx_spec_accept_workspace(int64_t B, int k, int64_t V) {
   if (B <= 0 || k <= 0 || V <= 0) return 256;
-  return spec_ws_bytes(B, k, V);
+  return spec_ws_bytes(B, k, V, kCntLd);
 }
 
 // The two launches for k >= 0 draft positions (k = 0: the draw from p_0
@@ -853,7 +736,8 @@ static int spec_run(const void* target, const void* draft, int dtype, int64_t B,
       pl.nsb > kDrawLds || rows_a * pl.chunks > kAccParts)
     return VNX_ERR_UNSUPPORTED;
   // (the partials are carved for 2k + 1 rows of this plan's chunks: enough)
-  if (!workspace || workspace_bytes < spec_carve(nullptr, B, k, pl, nullptr)) return VNX_ERR_WORKSPACE;
+  if (!workspace || workspace_bytes < spec_carve(nullptr, B, k, pl, nullptr, 1)) return VNX_ERR_WORKSPACE;
+  const int64_t cnt_ld = workspace_bytes < spec_carve(nullptr, B, k, pl, nullptr, kCntLd) ? 1 : kCntLd;
   SpecParams p{};
   p.tgt = target; p.dft = draft; p.B = B; p.k = k; p.V = V;
   p.ld_t = ld_t; p.ld_d = ld_d; p.sb_t = sb_t; p.sb_d = sb_d;
@@ -862,7 +746,7 @@ static int spec_run(const void* target, const void* draft, int dtype, int64_t B,
   p.thr_t = thr_t; p.thr_d = thr_d; p.ids = draft_ids; p.u = uniforms;
   p.accept_len = accept_len; p.out_ids = out_ids; p.flags = flags; p.lse_t = lse_t; p.lse_d = lse_d;
   p.lse_din = lse_din; p.fl_din = fl_din; p.ld_din = ld_din; p.rows_a = rows_a;
-  spec_carve(workspace, B, k, pl, &p);
+  spec_carve(workspace, B, k, pl, &p, cnt_ld);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t na = B * rows_a * pl.chunks;
   const dim3 ga((unsigned)std::max<int64_t>(na, (B + kNT - 1) / kNT)), gb((unsigned)(B * pl.chunks2));
@@ -919,7 +803,7 @@ int vnx_spec_accept_noalloc(const void* target, const void* draft, int dtype, in
                             int64_t* out_ids, uint8_t* flags, float* lse_t, float* lse_d, void* stream) {
   if (k < 1) return VNX_ERR_INVALID_ARG;
   if (B < 0 || k > kMaxK || V <= 0) return VNX_ERR_INVALID_ARG;
-  if (B > 0 && spec_ws_bytes(B, k, V) > kSpecScratchBytes) return VNX_ERR_TOO_LARGE;
+  if (B > 0 && spec_ws_bytes(B, k, V, 1) > kSpecScratchBytes) return VNX_ERR_TOO_LARGE;
   int dev = 0;
   const hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return hip_fail(e);
@@ -932,7 +816,7 @@ int vnx_spec_accept_noalloc(const void* target, const void* draft, int dtype, in
 
 size_t vnx_sample_workspace(int64_t B, int64_t V) {
   if (B <= 0 || V <= 0) return 256;
-  return spec_ws_bytes(B, 0, V) + (((size_t)B * 4 + 255) & ~(size_t)255);
+  return spec_ws_bytes(B, 0, V, kCntLd) + (((size_t)B * 4 + 255) & ~(size_t)255);
 }
 
 int vnx_sample(const void* logits, int dtype, int64_t B, int64_t V, int64_t ld, const float* uniforms,
