@@ -1,10 +1,12 @@
-"""GPU parity of the draws' inverse-CDF walk where its loop can go wrong: rows
-shorter than a sub-block, partial last sub-blocks, odd numbers of sub-blocks
-per wave, rows without residual mass (recomputed by the drawing workgroup),
-and arrival counters packed for want of room.
+"""GPU parity of the draws' inverse-CDF walk and of the nucleus passes where
+their loops can go wrong: rows shorter than a sub-block, partial last
+sub-blocks, odd numbers of sub-blocks per wave, rows without residual mass
+(recomputed by the drawing workgroup), arrival counters packed for want of
+room, nucleus cuts inside long runs of ties, rows that nothing is drawn from.
 
-Bar as in tests/test_gpu_spec_accept.py: ids and accept_len bit-exact against
-the CPU oracle, save rows that a flag marks on either side."""
+Bar as in tests/test_gpu_spec_accept.py and tests/test_gpu_sampler.py: ids,
+accept_len and the nucleus bit-exact against the CPU oracle, save rows that a
+flag marks on either side."""
 import ctypes
 
 import numpy as np
@@ -13,6 +15,7 @@ import torch
 
 from oracle.speculative import spec_accept
 from spec_inputs import make_inputs
+from test_gpu_sampler import _check
 from test_gpu_spec_accept import compare, run_gpu
 from versenext_amd import _lib
 
@@ -63,3 +66,26 @@ def test_packed_counters(hip):
         outs.append((acc, out))
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
     assert int(outs[0][1].min()) >= -1 and int(outs[0][1].max()) < V
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("V", [3, 256, 1025, 33 * 512 + 8, 151936])
+def test_nucleus_edges(hip, V, dtype):
+    """Rows: one value (every cut is a tie), a few values, spread values, one
+    dominant value, NaN, +inf, all -inf, all but one -inf."""
+    rng = np.random.default_rng(V)
+    x = rng.normal(0, 3.0, (8, V)).astype(np.float32)
+    x[0] = 0.5
+    x[1] = np.round(x[1])
+    x[3, V // 2] = 60.0
+    x[4, V - 1] = np.nan
+    x[5, [0, V // 2]] = np.inf
+    x[6] = -np.inf
+    x[7] = -np.inf
+    x[7, V // 3] = -2.0
+    x = torch.from_numpy(x).to(dtype).float().numpy()
+    u = rng.random(8).astype(np.float32)
+    for T, p in ((1.0, 0.9), (0.7, 0.35), (1.0, 1e-4), (1.0, 0.99999), (0.8, 1.0), (0.0, 1.0)):
+        print("nucleus", V, dtype, T, p, flush=True)
+        _, _, bad = _check(hip, x, T, 0, p, u, dtype=dtype)
+        assert bad <= 1, (T, p)

@@ -7,7 +7,6 @@
 // workgroups per CU over the batch, at most 8192 elements each), and the
 // reference's steps run as a short chain of launches; kernel boundaries carry
 // the row state between them (no fences, no grid barrier):
-//   init       (without top-k) zero the row's histograms and counters;
 //   calib 0,1  (VNX_SAMPLE_CALIBRATE) chunk sums of x, then of (x - mean)^2,
 //              in fp64; later launches merge the C partials in chunk order
 //              into var, s = RN(sqrt(RN32(var) + eps)), l -> RN(RN(l/s) * f).
@@ -34,21 +33,27 @@
 //              a larger k or a longer row runs the whole algorithm over the
 //              row in the same workgroup instead (single-workgroup form).
 // Without top-k:
-//   lse        per chunk the max of a (NaN -> +inf), the fp64 sum of
-//              2^(a*log2e - mt), and numpy.argmax of the row;
-//   ppass 0..3 (top-p) every workgroup merges the C LSE partials (one wave,
+//   lse        per chunk the max of a (NaN -> +inf) and the fp64 sum of
+//              2^(a*log2e - mt); numpy.argmax of the chunk where the row may
+//              need it (T == 0, or a maximum that is not finite); zeroes the
+//              row's histograms and counter for the launches below;
+//   ppass 0..2 (top-p) every workgroup merges the C LSE partials (one wave,
 //              fixed order) into L32 and radix-selects the nucleus value p*
-//              over the keys of p with fixed-point mass histograms (the last
-//              pass also counts per chunk, for ranking the ties),
-//              one 8-bit digit per launch: per-wave LDS histograms, nonzero
-//              bins added to the row's global histogram, the digit derived by
-//              the next launch (a block scan) and recorded by its chunk 0;
+//              over the 30 bits that p in [0, 1] has, with fixed-point mass
+//              histograms, one 10-bit digit per launch: LDS histograms,
+//              nonzero bins added to the row's global histogram, the digit
+//              derived by the next launch (a block scan) and recorded by its
+//              chunk 0 (the last pass also counts per chunk, for ranking the
+//              ties).  The launches read the rows from the caches and are
+//              bound by the exps and their prologues, so they are few: four
+//              passes of 8 bits took 47 us for 32 rows of 248,320 in fp32,
+//              three of 10 35;
 //   mass       draw weights (p, or p masked by the nucleus: p > p*, or
 //              p == p* and id <= j*, j* ranked by the one chunk holding it),
 //              fp64 masses per 64-vector sub-block published with agent-scope
 //              stores; the workgroup that completes the row walks them to
-//              u * total and writes every output.
-// T == 0 runs init, an argmax-only lse and the mass launch's final step.
+//              u * total (rowred.h) and writes every output.
+// T == 0 runs an argmax-only lse and the mass launch's final step.
 // The CPU checker oracle/sampler.py restates the same rules.  The exactly-k
 // draw runs over the kept tokens in id order: argpartition's output order,
 // which the reference draws over, is implementation-defined.
@@ -64,7 +69,11 @@ constexpr int kSNW = kSNT / VNX_WAVE;
 constexpr int kST = 1024;              // threads per workgroup (per-row kernels)
 constexpr int kSW = kST / VNX_WAVE;
 constexpr int kSNB = 4;                // vectors in flight per thread
-constexpr int kBins = 256;             // 8-bit digits
+constexpr int kBins = 256;             // 8-bit digits (the per-row kernel)
+constexpr int kPBits = 10;             // digits of the nucleus passes
+constexpr int kPBins = 1 << kPBits;
+constexpr int kPPass = 3;              // p <= 1 has 30 significant bits
+constexpr int kCntLd = 32;             // arrival counters a cache line apart
 constexpr int kSMaxC = 64;             // chunks per row (one wave merges their partials)
 constexpr int64_t kChunkMax = 8192;    // elements per chunk (the local kernel's LDS keys)
 constexpr int kSampDraw = 4096;        // sub-blocks of 64 vectors per row (the draw walk in LDS)
@@ -102,9 +111,9 @@ struct SampParams {
   int64_t* j_star;
   int64_t* k_star;
   // workspace
-  unsigned long long* phm;    // [B][4][256]
-  uint32_t* lp;               // [B][C][256] the last p pass's per-chunk counts
-  RadixState* stp;            // [B][5] top-p state before pass i
+  unsigned long long* phm;    // [B][kPPass][kPBins]
+  uint32_t* lp;               // [B][C][kPBins] the last p pass's per-chunk counts
+  RadixState* stp;            // [B][kPPass] top-p state before pass i
   double* cs1;                // [B][C] calibration partials
   double* cs2;
   float* pm;                  // [B][C] LSE / argmax partials
@@ -113,7 +122,7 @@ struct SampParams {
   int64_t* pai;
   int64_t* jstar;             // [B] the last kept tie of the nucleus (agent-scope)
   double* sbm;                // [B][nsb]
-  unsigned* cnt;              // [B]
+  unsigned* cnt;              // [B], kCntLd apart
   unsigned long long* cand;   // [B][C][kSegCap] candidates (key << 32 | ~id)
   unsigned* nct;              // [B][C] candidates per chunk
   uint32_t* tc;               // [B][C] the chunk's threshold key
@@ -145,8 +154,12 @@ __device__ __forceinline__ float okey_value(uint32_t k) {
 }
 
 __device__ __forceinline__ unsigned long long fix60(float p) {
-  // floor(p * 2^60) for 0 <= p <= 2 (exact: scaling by a power of two)
-  return (unsigned long long)((double)p * 1152921504606846976.0);
+  // floor(p * 2^60) for 0 <= p <= 2: the 24-bit significand shifted (2^-90
+  // and less become 0, subnormals among them)
+  const uint32_t u = __float_as_uint(p);
+  const int sh = (int)(u >> 23) - 90;
+  const unsigned long long m = (u & 0x7FFFFFu) | 0x800000u;
+  return sh >= 0 ? m << sh : m >> min(-sh, 63);
 }
 
 // Calls f(j, raw) for every element of [j0, j1) (j0 a multiple of the vector
@@ -277,90 +290,160 @@ __device__ __forceinline__ int pick_digit(const T* h, unsigned long long rem, un
 // ===========================================================================
 // Chunk kernels (kSNT threads).
 // ===========================================================================
-struct SampLds {
-  unsigned hc[kSNW][kBins];            // per-wave histogram copies
-  unsigned long long hm[kSNW][kBins];
-  unsigned long long scan[kSW];
-  double dd[kSW];
-  float f[kSW];
-  int64_t i[kSW];
-  unsigned long long seg[kSNT];
+__device__ __forceinline__ unsigned lane_rank(uint64_t m) {
+  // set bits of m below this lane
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+struct ChunkLds {
+  unsigned long long scan[kSNW];
+  double dd[kSNW];
+  float f[kSNW];
+  int64_t i[kSNW];
   int sel, flag;
   unsigned long long rank, above;
   int64_t found;
-  // the draw walk
-  double T[kSNT], E[kSNT];
-  double total, target, base;
-  int64_t sb;
-  int tstar, tlast;
+};
+struct PassLds : ChunkLds {
+  unsigned long long hm[2][kPBins];  // a copy for every other wave
+  unsigned hc[kPBins];
+};
+struct MassLds : ChunkLds {
+  WalkLds<kSNT> walk;
 };
 
-// The id of the m-th element (1-based, id order) of [j0, j1) for which
-// pred(j, raw) holds, -1 if there are fewer: contiguous per-thread ranges,
-// counts, a scan in thread order, then the owner of the m-th match walks.
-template <typename Tin, int NT, typename P>
-__device__ __forceinline__ int64_t nth_in_range(const Tin* row, int64_t j0, int64_t j1, unsigned long long m,
-                                                SampLds& L, P&& pred) {
+// This lane's vector of sub-block sbi (elements past V read as NaN, whose
+// probability is 0).
+template <typename Tin>
+__device__ __forceinline__ void sub_block(const Tin* row, int sbi, int64_t V, float (&x)[Vec<Tin>::N]) {
   constexpr int VE = Vec<Tin>::N;
-  const int tid = threadIdx.x;
-  const int64_t seg = ((j1 - j0 + NT - 1) / NT + VE - 1) / VE * VE;
-  const int64_t a0 = min(j0 + (int64_t)tid * seg, j1), a1 = min(a0 + seg, j1);
-  unsigned long long c = 0;
-  seg_visit<Tin>(row, a0, a1, [&](int64_t j, float x) { c += pred(j, x) ? 1ull : 0ull; });
-  __syncthreads();
-  L.seg[tid] = c;
-  __syncthreads();
-  if (tid == 0) {
-    unsigned long long run = 0;
-    int owner = -1;
-    for (int t = 0; t < NT; ++t) {
-      if (run + L.seg[t] >= m) { owner = t; break; }
-      run += L.seg[t];
-    }
-    L.sel = owner;
-    L.rank = m - run;
-    L.found = -1;
+  const int64_t e0 = ((int64_t)sbi * VNX_WAVE + threadIdx.x % VNX_WAVE) * VE;
+  if (e0 + VE <= V) {
+    Vec<Tin>::load(row + e0, x);
+  } else {
+#pragma unroll
+    for (int i = 0; i < VE; ++i) x[i] = e0 + i < V ? Vec<Tin>::load1(row + e0 + i) : __builtin_nanf("");
   }
-  __syncthreads();
-  if (tid == L.sel) {
-    const unsigned long long want = L.rank;
-    unsigned long long r = 0;
-    int64_t found = -1;
-    seg_visit<Tin>(row, a0, a1, [&](int64_t j, float x) {
-      if (found < 0 && pred(j, x) && ++r == want) found = j;
-    });
-    L.found = found;
-  }
-  __syncthreads();
-  const int64_t res = L.found;
-  __syncthreads();
-  return res;
 }
 
-// One step of the nucleus radix select from the state before a pass and
-// that pass's global (count, mass) histogram.
-__device__ __forceinline__ RadixState p_step(RadixState s, int pass, const unsigned long long* hm, SampLds& L) {
+// The id of the m-th element (1-based, id order) of sub-blocks [s0, s1) for
+// which pred(raw) holds (-1 if there are fewer): matches per sub-block (n, LDS),
+// a scan over them, then one wave inside the sub-block.
+template <typename Tin, typename P>
+__device__ __forceinline__ int64_t nth_match(const Tin* row, int s0, int s1, int64_t V, unsigned m, unsigned* n,
+                                             ChunkLds& L, P&& pred) {
+  constexpr int VE = Vec<Tin>::N;
+  const int tid = threadIdx.x, lane = tid % VNX_WAVE;
+  const int whole = min(s1, (int)(V / (VNX_WAVE * VE)));
+#pragma unroll 1
+  for (int sbi = s0 + tid / VNX_WAVE; sbi < s1; sbi += kSNW * kSNB) {
+    u32x4 raw[kSNB];
+#pragma unroll
+    for (int t = 0; t < kSNB; ++t)
+      if (sbi + kSNW * t < whole)
+        raw[t] = Vec<Tin>::load_raw(row + ((int64_t)(sbi + kSNW * t) * VNX_WAVE + lane) * VE);
+#pragma unroll
+    for (int t = 0; t < kSNB; ++t) {
+      const int at = sbi + kSNW * t;
+      if (at >= s1) break;
+      float x[VE];
+      Vec<Tin>::cvt_raw(raw[t], x);
+      if (at >= whole) sub_block<Tin>(row, at, V, x);
+      unsigned c = 0;
+#pragma unroll
+      for (int i = 0; i < VE; ++i) c += (unsigned)__builtin_popcountll(__ballot(pred(x[i])));
+      if (lane == 0) n[at - s0] = c;
+    }
+  }
+  if (tid == 0) L.sel = -1;
+  __syncthreads();
+  const int ns = s1 - s0, q = (ns + kSNT - 1) / kSNT;
+  unsigned long long t = 0;
+#pragma unroll 1
+  for (int i = tid * q; i < min((tid + 1) * q, ns); ++i) t += n[i];
+  const unsigned long long incl = block_scan_u64<kSNT>(t, L.scan);
+  if (incl >= m && incl - t < m) {
+    unsigned long long run = incl - t;
+    int i = tid * q;
+#pragma unroll 1
+    for (; run + n[i] < m; ++i) run += n[i];
+    L.sel = s0 + i;
+    L.rank = m - run;
+  }
+  __syncthreads();
+  if (tid < VNX_WAVE) {
+    int64_t id = -1;
+    if (L.sel >= 0) {
+      float x[VE];
+      sub_block<Tin>(row, L.sel, V, x);
+      const unsigned want = (unsigned)L.rank;
+      unsigned c = 0;
+#pragma unroll
+      for (int i = 0; i < VE; ++i) c += pred(x[i]) ? 1u : 0u;
+      unsigned before = 0;  // matches of the lanes below
+#pragma unroll
+      for (int b = 0; b < 4; ++b)  // c <= VE <= 8 < 2^4
+        before += lane_rank(__ballot((c >> b) & 1u)) << b;
+      int pick = -1;
+      unsigned r = before;
+#pragma unroll
+      for (int i = 0; i < VE; ++i)
+        if (pred(x[i]) && ++r == want) pick = i;
+      const uint64_t hit = __ballot(pick >= 0);
+      const int owner = hit ? (int)__builtin_ctzll(hit) : 0;
+      id = ((int64_t)L.sel * VNX_WAVE + owner) * VE + __shfl(pick, owner, VNX_WAVE);
+    }
+    if (lane == 0) L.found = id;
+  }
+  __syncthreads();
+  return L.found;
+}
+
+// One step of the nucleus radix select, from the state before a pass and this
+// thread's four bins of that pass's global mass histogram, counted from the
+// top: bin kPBins - 1 - (4 tid + q).
+__device__ __forceinline__ RadixState p_step(RadixState s, int pass, const unsigned long long (&v)[4], ChunkLds& L) {
+  static_assert(kPBins == 4 * kSNT, "");
   if (s.done) return s;
-  unsigned long long above;
-  const int d = pick_digit(hm, s.rem, &above, &L.sel, &L.above);
+  if (threadIdx.x == 0) L.sel = kPBins;
+  const unsigned long long t = (v[0] + v[1]) + (v[2] + v[3]);
+  const unsigned long long incl = block_scan_u64<kSNT>(t, L.scan);
+  if (incl >= s.rem && incl - t < s.rem) {
+    unsigned long long run = incl - t;
+    int q = 0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      if (q == i && run + v[i] < s.rem) { run += v[i]; q = i + 1; }
+    L.sel = kPBins - 1 - (4 * (int)threadIdx.x + q);
+    L.above = run;
+  }
+  __syncthreads();
+  const int d = L.sel;
+  const unsigned long long above = L.above;
+  __syncthreads();
   RadixState o = s;
-  if (d == kBins) {
+  if (d == kPBins) {
     o.done = 1;  // the whole mass stays below top_p: every token is kept
   } else {
-    const int shift = 24 - 8 * pass;
+    const int shift = kPBits * (kPPass - 1 - pass);
     o.rem = s.rem - above;
     o.prefix = s.prefix | ((uint32_t)d << shift);
-    o.pmask = s.pmask | (0xFFu << shift);
+    o.pmask = s.pmask | ((uint32_t)(kPBins - 1) << shift);
   }
   return o;
 }
 
+__device__ __forceinline__ void p_bins(const unsigned long long* h, unsigned long long (&v)[4]) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) v[q] = h[kPBins - 1 - (4 * (int)threadIdx.x + q)];
+}
+
 // After the last pass: the chunk holding the rem-th tie of the cut key (from
 // every chunk's count of the last digit's bin) and the rank inside it.
-__device__ __forceinline__ RadixState locate_cut(RadixState s, const uint32_t* local, int C, SampLds& L) {
+__device__ __forceinline__ RadixState locate_cut(RadixState s, const uint32_t* local, int C, ChunkLds& L) {
   if (threadIdx.x < VNX_WAVE) {
     const int lane = threadIdx.x;
-    const unsigned long long n = lane < C ? (unsigned long long)local[lane * kBins + (s.prefix & 0xFFu)] : 0ull;
+    const unsigned long long n = lane < C ? (unsigned long long)local[lane * kPBins + (s.prefix & (kPBins - 1))] : 0ull;
     unsigned long long incl = n;
 #pragma unroll
     for (int o = 1; o < VNX_WAVE; o <<= 1) {
@@ -436,7 +519,7 @@ __device__ __forceinline__ void set_l32(RowCtx& r, double Lr) {
 }
 
 // The row LSE from the C chunk partials (one wave, fixed order).
-__device__ __forceinline__ void ctx_lse(const SampParams& p, int64_t b, RowCtx& r, SampLds& L) {
+__device__ __forceinline__ void ctx_lse(const SampParams& p, int64_t b, RowCtx& r, ChunkLds& L) {
   if (threadIdx.x < VNX_WAVE) {
     const int lane = threadIdx.x;
     float m = kNegInf;
@@ -475,16 +558,6 @@ __device__ __forceinline__ int64_t merged_argmax(const SampParams& p, int64_t b)
   return i == INT64_MAX ? 0 : i;
 }
 
-__global__ __launch_bounds__(kSNT) void k_samp_init(SampParams p) {
-  const int64_t b = blockIdx.x;
-  const int t = threadIdx.x;
-  for (int i = t; i < 4 * kBins; i += kSNT) p.phm[b * 4 * kBins + i] = 0ull;
-  if (t == 0) {
-    p.cnt[b] = 0u;
-    p.stp[b * 5] = RadixState{0u, 0u, (unsigned long long)p.p_target, 0, 0};
-  }
-}
-
 template <typename Tin, int PASS>
 __global__ __launch_bounds__(kSNT) void k_samp_calib(SampParams p) {
   __shared__ double red[kSNW];
@@ -514,11 +587,6 @@ struct LocalLds {
   uint32_t t;
   unsigned n;
 };
-
-__device__ __forceinline__ unsigned lane_rank(uint64_t m) {
-  // set bits of m below this lane
-  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
 
 // One chunk of a top-k row: its keys into LDS, a lower bound t of its kth
 // largest key, and every key >= t published as a candidate (see the header).
@@ -592,41 +660,62 @@ __global__ __launch_bounds__(kSNT) void k_samp_local(SampParams p) {
   }
 }
 
+// Bound by the exact scaling and the exps (the second read of the chunk comes
+// from the caches).  The argmax costs more than both, and a row needs it only
+// when nothing can be drawn from it: at T == 0, or when its maximum is not
+// finite -- and then the maximum lies in a chunk whose own is not finite,
+// since a = RN(l/T) keeps the order of l.  32 rows of 248,320 in fp32:
+// 17.3 us with an argmax per chunk (and 4.2 for a launch that zeroed the
+// histograms), 10.5 now.
 template <typename Tin, int SM, bool CAL>
 __global__ __launch_bounds__(kSNT) void k_samp_lse(SampParams p) {
-  __shared__ SampLds L;
+  __shared__ ChunkLds L;
   const int64_t b = blockIdx.x / p.C;
   const int c = blockIdx.x % p.C;
+  const int tid = threadIdx.x;
   const Tin* row = static_cast<const Tin*>(p.x) + b * p.ld;
   const int64_t j0 = c * p.clen, j1 = min(j0 + p.clen, p.V);
+  // what the launches below start from
+  if (c == 0 && tid == 0) {
+    p.cnt[b * kCntLd] = 0u;
+    p.stp[b * kPPass] = RadixState{0u, 0u, (unsigned long long)p.p_target, 0, 0};
+  }
+  if (p.use_p && !p.greedy)
+    for (int i = c * kSNT + tid; i < kPPass * kPBins; i += p.C * kSNT) p.phm[b * kPPass * kPBins + i] = 0ull;
   RowCtx r;
   ctx_init(p, b, r);
   const RowFns<SM, CAL> fn{p, r};
-  // chunk max (NaN -> +inf) and numpy.argmax of the (calibrated) row
-  float M = kNegInf, av = kNegInf;
-  bool nan = false;
-  int64_t ai = INT64_MAX;
-  for_range<Tin, kSNT>(row, j0, j1, [&](int64_t j, float x) {
-    const float v = fn.val(x);
-    if (ai == INT64_MAX || argmax_better(v, j, av, ai)) { av = v; ai = j; }
-    if (!p.greedy) {
-      const float a = tscale<SM>(v, p.sc);
-      nan |= __builtin_isnan(a);
-      M = fmaxf(M, a);
-    }
-  });
-  block_argmax<kSNT>(av, ai, L.f, L.i);
-  const float bm = block_max<kSNT>(nan ? kPosInf : M, L.f);
+  float bm = kNegInf;
   double s = 0.0;
-  if (!p.greedy && bm > kNegInf && bm < kPosInf) {
-    const float mt = mt_of(bm);
+  if (!p.greedy) {
+    // chunk max (NaN -> +inf)
+    float M = kNegInf;
+    bool nan = false;
     for_range<Tin, kSNT>(row, j0, j1, [&](int64_t, float x) {
       const float a = fn.scaled(x);
-      if (a > kNegInf) s += (double)exp2_term(a, mt);
+      nan |= __builtin_isnan(a);
+      M = fmaxf(M, a);
     });
+    bm = block_max<kSNT>(nan ? kPosInf : M, L.f);
+    if (bm > kNegInf && bm < kPosInf) {
+      const float mt = mt_of(bm);
+      for_range<Tin, kSNT>(row, j0, j1, [&](int64_t, float x) {
+        const float a = fn.scaled(x);
+        if (a > kNegInf) s += (double)exp2_term(a, mt);
+      });
+    }
+    s = block_sum<kSNT>(s, L.dd);
   }
-  s = block_sum<kSNT>(s, L.dd);
-  if (threadIdx.x == 0) {
+  float av = kNegInf;
+  int64_t ai = INT64_MAX;
+  if (!(bm > kNegInf && bm < kPosInf)) {  // uniform over the workgroup
+    for_range<Tin, kSNT>(row, j0, j1, [&](int64_t j, float x) {
+      const float v = fn.val(x);
+      if (ai == INT64_MAX || argmax_better(v, j, av, ai)) { av = v; ai = j; }
+    });
+    block_argmax<kSNT>(av, ai, L.f, L.i);
+  }
+  if (tid == 0) {
     p.pm[b * p.C + c] = bm;
     p.ps[b * p.C + c] = s;
     p.pav[b * p.C + c] = av;
@@ -636,244 +725,199 @@ __global__ __launch_bounds__(kSNT) void k_samp_lse(SampParams p) {
 
 template <typename Tin, int SM, bool CAL, int PASS>
 __global__ __launch_bounds__(kSNT) void k_samp_ppass(SampParams p) {
-  __shared__ SampLds L;
+  __shared__ PassLds L;
   const int64_t b = blockIdx.x / p.C;
   const int c = blockIdx.x % p.C;
-  const int wave = threadIdx.x / VNX_WAVE;
+  const int tid = threadIdx.x, copy = (tid / VNX_WAVE) & 1;
   const Tin* row = static_cast<const Tin*>(p.x) + b * p.ld;
   const int64_t j0 = c * p.clen, j1 = min(j0 + p.clen, p.V);
   RowCtx r;
   ctx_init(p, b, r);
+  // the state and the bins load under the merge of the LSE partials
+  RadixState s = p.stp[b * kPPass + (PASS > 0 ? PASS - 1 : 0)];
+  unsigned long long v[4];
+  if (PASS > 0) p_bins(p.phm + (b * kPPass + PASS - 1) * kPBins, v);
+  for (int i = tid; i < kPBins; i += kSNT) {
+    L.hm[0][i] = L.hm[1][i] = 0ull;
+    if (PASS == kPPass - 1) L.hc[i] = 0u;
+  }
   ctx_lse(p, b, r, L);
   if (r.fallback) return;  // uniform over the workgroup
   const RowFns<SM, CAL> fn{p, r};
-  RadixState s = p.stp[b * 5 + (PASS > 0 ? PASS - 1 : 0)];
   if (PASS > 0) {
-    s = p_step(s, PASS - 1, p.phm + (b * 4 + PASS - 1) * kBins, L);
-    if (c == 0 && threadIdx.x == 0) p.stp[b * 5 + PASS] = s;
+    s = p_step(s, PASS - 1, v, L);
+    if (c == 0 && tid == 0) p.stp[b * kPPass + PASS] = s;
   }
   if (s.done) return;  // uniform
-  for (int i = threadIdx.x; i < kSNW * kBins; i += kSNT) {
-    (&L.hc[0][0])[i] = 0u;
-    (&L.hm[0][0])[i] = 0ull;
-  }
   __syncthreads();
-  const int shift = 24 - 8 * PASS;
+  const int shift = kPBits * (kPPass - 1 - PASS);
   for_range<Tin, kSNT>(row, j0, j1, [&](int64_t, float x) {
     const float pp = fn.prob(x);
     const uint32_t k = __float_as_uint(pp);
     if ((k & s.pmask) == s.prefix) {
-      const int d = (k >> shift) & 0xFFu;
-      if (PASS == 3) atomicAdd(&L.hc[wave][d], 1u);  // the last digit's ties are ranked by count
-      atomicAdd(&L.hm[wave][d], fix60(pp));
+      const int d = (k >> shift) & (kPBins - 1);
+      if (PASS == kPPass - 1) atomicAdd(&L.hc[d], 1u);  // the last digit's ties are ranked by count
+      atomicAdd(&L.hm[copy][d], fix60(pp));
     }
   });
   __syncthreads();
-  const int t = threadIdx.x;  // kSNT == kBins
-  unsigned cn = 0;
-  unsigned long long m = 0;
-#pragma unroll
-  for (int w = 0; w < kSNW; ++w) {
-    if (PASS == 3) cn += L.hc[w][t];
-    m += L.hm[w][t];
+  for (int i = tid; i < kPBins; i += kSNT) {
+    const unsigned long long m = L.hm[0][i] + L.hm[1][i];
+    if (m) atomicAdd(p.phm + (b * kPPass + PASS) * kPBins + i, m);
+    if (PASS == kPPass - 1) p.lp[(b * p.C + c) * kPBins + i] = L.hc[i];
   }
-  if (m) atomicAdd(p.phm + (b * 4 + PASS) * kBins + t, m);
-  if (PASS == 3) p.lp[(b * p.C + c) * kBins + t] = cn;
 }
 
+// Sub-blocks of 64 vectors, wave w those at w + kSNW*j of the chunk; as in
+// the acceptance draw, one rolled loop holds the only copy of the weights'
+// code, for the masses and for the sub-block drawn from.  The workgroup that
+// holds the nucleus' cut ranks its ties first.  32 rows of 248,320 in fp32
+// with top-p: 39 -> 27 us.
 template <typename Tin, int SM, bool CAL>
-__global__ __launch_bounds__(kSNT) void k_samp_mass(SampParams p) {
-  __shared__ SampLds L;
-  extern __shared__ double sh_m[];  // the draw: the row's sub-block masses
+__global__ __launch_bounds__(kSNT, 4) void k_samp_mass(SampParams p) {
+  __shared__ MassLds L;
+  extern __shared__ double sh_m[];  // match counts of the cut; the draw: the row's sub-block masses
   constexpr int VE = Vec<Tin>::N;
+  constexpr int U = 8 / VE;         // sub-blocks per turn of the loop
   const int64_t b = blockIdx.x / p.C;
   const int c = blockIdx.x % p.C;
-  const int tid = threadIdx.x;
-  const int wave = tid / VNX_WAVE, lane = tid % VNX_WAVE;
+  const int tid = threadIdx.x, lane = tid % VNX_WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / VNX_WAVE);
   const Tin* row = static_cast<const Tin*>(p.x) + b * p.ld;
-  const int64_t j0 = c * p.clen, j1 = min(j0 + p.clen, p.V);
-  const int64_t sbl = (int64_t)VNX_WAVE * VE;
+  const int nsb = (int)p.nsb;                         // <= kSampDraw
+  const int whole = (int)(p.V / (VNX_WAVE * VE));     // sub-blocks without an element past V
+  const int spc = (int)(p.clen / (VNX_WAVE * VE));    // chunks are whole sub-blocks
+  const int s0 = c * spc;
+  int s1 = min(s0 + spc, nsb);
+  int sb = s0 + wave, j = 0;
+  u32x4 rp[kSNB];
+  // the batch of this wave's sub-blocks from at, every load in flight
+  auto load = [&](int at) {
+    const Tin* bp = row + ((int64_t)at * VNX_WAVE + lane) * VE;
+    const int e1 = min(s1, whole);
+#pragma unroll
+    for (int t = 0; t < kSNB; ++t)
+      if (at + kSNW * t < e1) rp[t] = Vec<Tin>::load_raw(bp + kSNW * VNX_WAVE * VE * t);
+    j = 0;
+  };
   RowCtx r;
   ctx_init(p, b, r);
-  if (!p.greedy) ctx_lse(p, b, r, L);
+  RadixState s = p.stp[b * kPPass + kPPass - 1];
+  unsigned long long v[4];
+  if (!p.greedy) {
+    if (p.use_p) p_bins(p.phm + (b * kPPass + kPPass - 1) * kPBins, v);
+    load(sb);
+    ctx_lse(p, b, r, L);
+  }
   const RowFns<SM, CAL> fn{p, r};
-  const bool draw = !p.greedy && !r.fallback;
-  if (draw && p.use_p) {
-    RadixState s = p_step(p.stp[b * 5 + 3], 3, p.phm + (b * 4 + 3) * kBins, L);
+  const bool live = !p.greedy && !r.fallback;  // uniform
+  if (live && p.use_p) {
+    s = p_step(s, kPPass - 1, v, L);
     if (!s.done) {
       r.pstar = __uint_as_float(s.prefix);
       // the nucleus needs m ties of value p* (each adds fix60(p*) > 0: a
       // zero-mass bin is never chosen); the chunk holding the m-th ranks them
       const unsigned long long P = fix60(r.pstar);
       s.rem = (s.rem + P - 1) / P;
-      s = locate_cut(s, p.lp + b * p.C * kBins, p.C, L);
+      s = locate_cut(s, p.lp + b * p.C * kPBins, p.C, L);
       if (c < s.cstar) {
         r.jbound = INT64_MAX;
       } else if (c > s.cstar) {
         r.jbound = -1;
       } else {
         const float ps = r.pstar;
-        r.jbound = nth_in_range<Tin, kSNT>(row, j0, j1, s.rem, L, [&](int64_t, float x) { return fn.prob(x) == ps; });
+        r.jbound = nth_match<Tin>(row, s0, s1, p.V, (unsigned)s.rem, reinterpret_cast<unsigned*>(sh_m), L,
+                                  [&](float x) { return fn.prob(x) == ps; });
         if (tid == 0) st_agent(p.jstar + b, r.jbound);
       }
     }
   }
-  if (draw) {
-    // this chunk's sub-blocks (chunks are whole sub-blocks); lane w sums its
-    // VE weights in fp64, the wave sums the lanes
-    const int64_t s0 = j0 / sbl, s1 = (j1 + sbl - 1) / sbl;
-    for (int64_t sbi = s0 + wave; sbi < s1; sbi += kSNW) {
-      const int64_t e0 = (sbi * VNX_WAVE + lane) * VE;
-      double m = 0.0;
-      if (e0 + VE <= p.V) {
-        float x[VE];
-        Vec<Tin>::load(row + e0, x);
+  bool draw = false;  // uniform
+  double total = 0.0, target = 0.0;
+  float w[U][VE];
+  double lm[U];
+  if (!live) sb = s1;
+#pragma unroll 1
+  for (;;) {
+    if (sb >= s1) {  // this wave's masses are out (never while drawing)
+      // every wave's published masses complete before the workgroup arrives
+      __builtin_amdgcn_s_waitcnt(0);
+      if (!arrive_last(p.cnt + b * kCntLd, (unsigned)p.C, &L.flag)) return;
+      if (!live) break;
+      // the nucleus ties of the whole row now hold by id: jbound = j*
+      if (r.pstar >= 0.0f) r.jbound = ld_agent(p.jstar + b);
+      walk_load<kSNT>(p.sbm + b * nsb, nsb, sh_m);
+      double own;
+      total = walk_total<kSNT>(sh_m, nsb, L.walk, &own);
+      target = samp_u(p, b) * total;
+      walk_find<kSNT>(sh_m, nsb, own, target, L.walk);
+      if (wave) return;
+      draw = true;
+      sb = __builtin_amdgcn_readfirstlane(L.walk.sb);
+      if (sb < 0) break;
+      s1 = nsb;
+    }
+    // one sub-block (past the whole ones, or the one drawn from), or U
+    const bool one = draw || sb + kSNW * (U - 1) >= whole;
+    float x[U][VE];
+    if (one) {
+      sub_block<Tin>(row, sb, p.V, x[0]);
 #pragma unroll
-        for (int i = 0; i < VE; ++i) m += (double)fn.weight(e0 + i, x[i]);
-      } else {
-        for (int i = 0; i < VE; ++i)
-          if (e0 + i < p.V) m += (double)fn.weight(e0 + i, Vec<Tin>::load1(row + e0 + i));
-      }
-      m = wave_sum(m);
-      if (lane == 0) st_agent(p.sbm + b * p.nsb + sbi, m);
-    }
-  }
-  // every wave's published masses complete before the workgroup arrives
-  __builtin_amdgcn_s_waitcnt(0);
-  if (!arrive_last(p.cnt + b, (unsigned)p.C, &L.flag)) return;
-
-  // ---- the workgroup that completes the row ----
-  auto finish = [&](int64_t token, int fl, float lse, float ps, int64_t js) {
-    if (tid == 0) {
-      p.out[b] = token;
-      if (p.flags) p.flags[b] = (uint8_t)fl;
-      if (p.lse) p.lse[b] = lse;
-      if (p.kth) p.kth[b] = kNegInf;
-      if (p.p_star) p.p_star[b] = ps;
-      if (p.j_star) p.j_star[b] = js;
-      if (p.k_star) p.k_star[b] = -1;
-    }
-  };
-  if (!draw) {
-    int64_t am = 0;
-    if (tid < VNX_WAVE) am = merged_argmax(p, b);
-    if (tid == 0) L.found = am;
-    __syncthreads();
-    finish(L.found, r.fl, __builtin_nanf(""), -1.0f, -1);
-    return;
-  }
-  // the nucleus ties of the whole row now hold by id: jbound = j*
-  if (r.pstar >= 0.0f) r.jbound = ld_agent(p.jstar + b);
-  // thread t owns sub-blocks [t*q, (t+1)*q); the total is sum_t (sum_i) in
-  // that nested order, and the walk follows it
-  const int64_t nsb = p.nsb;
-  const int64_t q = (nsb + kSNT - 1) / kSNT;  // <= kSampDraw / kSNT (host check)
-  {
-    double t = 0.0;
-    for (int64_t i = (int64_t)tid * q; i < min((int64_t)(tid + 1) * q, nsb); ++i) {
-      const double m = ld_agent(p.sbm + b * nsb + i);
-      sh_m[i] = m;
-      t += m;
-    }
-    const double incl = block_inclusive_scan<kSNT>(t, L.dd);
-    L.T[tid] = t;
-    L.E[tid] = incl;
-    __syncthreads();
-    if (tid == kSNT - 1) L.total = incl;
-    if (tid == 0) { L.tstar = kSNT; L.tlast = -1; }
-    __syncthreads();
-  }
-  const double total = L.total;
-  const double target = samp_u(p, b) * total;
-  {
-    const double T = L.T[tid], end = L.E[tid];
-    const double start = tid ? L.E[tid - 1] : 0.0;
-    if (T > 0.0 && start <= target && target < end) atomicMin(&L.tstar, tid);
-    if (T > 0.0) atomicMax(&L.tlast, tid);
-  }
-  __syncthreads();
-  if (tid == 0) {
-    int ts = L.tstar;
-    if (ts == kSNT) ts = L.tlast;
-    int64_t sstar = -1;
-    double base = 0.0;
-    if (ts >= 0) {
-      const double b0 = ts ? L.E[ts - 1] : 0.0;
-      double r2 = b0, b_last = b0;
-      int64_t slast = -1;
-      for (int64_t i = (int64_t)ts * q; i < min((int64_t)(ts + 1) * q, nsb); ++i) {
-        const double m = sh_m[i];
-        if (m > 0.0) {
-          if (sstar < 0 && r2 + m > target) { sstar = i; base = r2; }
-          slast = i;
-          b_last = r2;
-        }
-        r2 += m;
-      }
-      if (sstar < 0) { sstar = slast; base = b_last; }
-    }
-    L.sb = sstar;
-    L.target = target;
-    L.base = base;
-  }
-  __syncthreads();
-  const int64_t sstar = L.sb;
-  if (wave != 0) return;
-  int fl = r.fl;
-  int64_t token = 0;
-  if (sstar < 0) {
-    fl |= VNX_FLAG_ZERO_RESIDUAL;
-  } else {
-    const int64_t e0 = (sstar * VNX_WAVE + lane) * VE;
-    float w[VE];
-    double lm = 0.0;
+      for (int q = 1; q < U; ++q)
 #pragma unroll
-    for (int i = 0; i < VE; ++i) {
-      w[i] = e0 + i < p.V ? fn.weight(e0 + i, Vec<Tin>::load1(row + e0 + i)) : 0.0f;
-      lm += (double)w[i];
-    }
-    const double incl = wave_inclusive_scan(lm);
-    const double start = L.base + (incl - lm), end = L.base + incl;
-    const double tgt = L.target;
-    const bool hit = lm > 0.0 && start <= tgt && tgt < end;
-    const uint64_t hits = __ballot(hit), pos = __ballot(lm > 0.0);
-    int lstar;
-    bool edge = false;
-    if (hits) {
-      lstar = __builtin_ctzll(hits);
+        for (int i = 0; i < VE; ++i) x[q][i] = x[0][i];
     } else {
-      lstar = pos ? 63 - __builtin_clzll(pos) : -1;
-      edge = true;
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        u32x4 a = rp[q];
+#pragma unroll
+        for (int t = U; t < kSNB; t += U)
+          if (j == t) a = rp[t + q];
+        Vec<Tin>::cvt_raw(a, x[q]);
+      }
+      j += U;
+      if (j == kSNB) load(sb + kSNW * U);  // under this turn's weights
     }
-    if (lstar < 0) {
-      token = (sstar * VNX_WAVE) * VE;
-      edge = true;
-    } else if (lane == lstar) {
-      double run = start, before = start, after = end;
-      int pick = -1, lastpos = -1;
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      const int64_t e0 = ((int64_t)(sb + kSNW * q) * VNX_WAVE + lane) * VE;
+      lm[q] = 0.0;
 #pragma unroll
       for (int i = 0; i < VE; ++i) {
-        if (w[i] > 0.0f) {
-          lastpos = i;
-          if (pick < 0) {
-            const double nr = run + (double)w[i];
-            if (nr > tgt) { pick = i; before = run; after = nr; }
-            run = nr;
-          }
-        }
+        w[q][i] = fn.weight(e0 + i, x[q][i]);
+        lm[q] += (double)w[q][i];
       }
-      if (pick < 0) { pick = lastpos; edge = true; }
-      token = e0 + pick;
-      const double tol = 1e-12 * L.total;
-      if (tgt - before < tol || after - tgt < tol) edge = true;
     }
-    if (lstar >= 0) {
-      token = __shfl(token, lstar, VNX_WAVE);
-      edge = __shfl((int)edge, lstar, VNX_WAVE) != 0;
-    }
+    if (draw) break;
+    static_assert(U <= 2, "");
+    const double m = U == 1 ? wave_sum(lm[0]) : wave_sum2(lm[0], lm[U - 1]);
+    const int at = sb + (lane >> 5) * kSNW;
+    if ((lane & 31) == 0 && (lane == 0 || (U == 2 && !one && at < s1))) st_agent(p.sbm + b * nsb + at, m);
+    sb += one ? kSNW : kSNW * U;
+  }
+  // wave 0 of the workgroup that completes the row (every wave if nothing can
+  // be drawn from it)
+  int64_t token = 0;
+  int fl = r.fl;
+  if (!live) {
+    if (tid >= VNX_WAVE) return;
+    token = merged_argmax(p, b);
+  } else if (sb < 0) {
+    fl |= VNX_FLAG_ZERO_RESIDUAL;
+  } else {
+    bool edge;
+    token = walk_pick<VE>(w[0], lm[0], ((int64_t)sb * VNX_WAVE + lane) * VE, L.walk.base, target, total, &edge);
     if (edge) fl |= VNX_FLAG_CDF_EDGE;
   }
-  finish(token, fl, r.L32, r.pstar, r.pstar >= 0.0f ? r.jbound : -1);
+  if (tid == 0) {
+    p.out[b] = token;
+    if (p.flags) p.flags[b] = (uint8_t)fl;
+    if (p.lse) p.lse[b] = live ? r.L32 : __builtin_nanf("");
+    if (p.kth) p.kth[b] = kNegInf;
+    if (p.p_star) p.p_star[b] = live ? r.pstar : -1.0f;
+    if (p.j_star) p.j_star[b] = live && r.pstar >= 0.0f ? r.jbound : -1;
+    if (p.k_star) p.k_star[b] = -1;
+  }
 }
 
 // ===========================================================================
@@ -1826,10 +1870,10 @@ static SampPlan samp_plan(int64_t B, int64_t V, int dtype, bool local) {
 
 static size_t samp_carve(void* ws, int64_t B, const SampPlan& pl, SampParams* p) {
   Carve cv(ws);
-  const size_t nb = (size_t)B * 4 * kBins, nc = (size_t)B * pl.C;
+  const size_t nb = (size_t)B * kPPass * kPBins, nc = (size_t)B * pl.C;
   unsigned long long* phm = cv.take<unsigned long long>(nb);
-  uint32_t* lp = cv.take<uint32_t>(nc * kBins);
-  RadixState* stp = cv.take<RadixState>((size_t)B * 5);
+  uint32_t* lp = cv.take<uint32_t>(nc * kPBins);
+  RadixState* stp = cv.take<RadixState>((size_t)B * kPPass);
   double* cs1 = cv.take<double>(nc);
   double* cs2 = cv.take<double>(nc);
   float* pm = cv.take<float>(nc);
@@ -1838,7 +1882,7 @@ static size_t samp_carve(void* ws, int64_t B, const SampPlan& pl, SampParams* p)
   int64_t* pai = cv.take<int64_t>(nc);
   int64_t* jstar = cv.take<int64_t>((size_t)B);
   double* sbm = cv.take<double>((size_t)B * pl.nsb);
-  unsigned* cnt = cv.take<unsigned>((size_t)B);
+  unsigned* cnt = cv.take<unsigned>((size_t)B * kCntLd);
   unsigned long long* cand = cv.take<unsigned long long>(nc * kSegCap);
   unsigned* nct = cv.take<unsigned>(nc);
   uint32_t* tc = cv.take<uint32_t>(nc);
@@ -1907,10 +1951,6 @@ int vnx_sampler_sample(const void* logits, int dtype, int64_t B, int64_t V, int6
   samp_carve(workspace, B, pl, &p);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)(B * pl.C)), blk(kSNT);
-  if (!cand) {
-    hipLaunchKernelGGL(k_samp_init, dim3((unsigned)B), blk, 0, s, p);
-    VNX_LAUNCH_CHECK();
-  }
   return dispatch_tsm(dtype, sm, false, [&](auto tin, auto smc, auto) {
     using Tin = decltype(tin);
     constexpr int SM = decltype(smc)::value;
@@ -1930,7 +1970,6 @@ int vnx_sampler_sample(const void* logits, int dtype, int64_t B, int64_t V, int6
           hipLaunchKernelGGL((k_samp_ppass<Tin, SM, CAL, 0>), grid, blk, 0, s, p);
           hipLaunchKernelGGL((k_samp_ppass<Tin, SM, CAL, 1>), grid, blk, 0, s, p);
           hipLaunchKernelGGL((k_samp_ppass<Tin, SM, CAL, 2>), grid, blk, 0, s, p);
-          hipLaunchKernelGGL((k_samp_ppass<Tin, SM, CAL, 3>), grid, blk, 0, s, p);
         }
         hipLaunchKernelGGL((k_samp_mass<Tin, SM, CAL>), grid, blk, (size_t)pl.nsb * sizeof(double), s, p);
       }
