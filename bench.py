@@ -661,8 +661,7 @@ def trace_summary(d: str, top: int = 40) -> None:
     if len(marks) < 2:
         raise SystemExit("no marker kernels in the trace (run bench.py --workload e2e --e2e-mark)")
     win = rows[marks[0] + 1:marks[1]]
-    lm = sum(1 for r in win if "k_lm_head" in r["Kernel_Name"])  # one verify head per round
-    rounds = max(1, lm)
+    rounds = max(1, sum(1 for r in win if "k_spec_commit" in r["Kernel_Name"]))  # one commit per round
     agg = collections.defaultdict(lambda: [0, 0.0])
     busy = 0.0
     for r in win:

@@ -97,27 +97,37 @@ int by_dtype(int dt, F&& f) {
 constexpr int kRnThreads = 256;
 constexpr int kRnPer = 16;
 
-template <typename TY>
-__device__ __forceinline__ void rms_tail(const float (&v)[kRnPer], const float (&wv)[kRnPer], float ss,
+// Columns per thread: 4 for rows of up to 1,024 columns, else 16 (the same sums
+// in the same order; the 16-column form of a 1,024-column row skips 12 of its 16
+// steps, at a branch and a fetch of skipped code each).  2,048 rows of 1,024:
+// 7.8 us, 8.8 with the 16-column form; 224 rows 3.6, 4.4.
+template <typename F>
+void by_rn_per(int64_t D, F&& f) {
+  if (D <= 4 * (int64_t)kRnThreads) f(IntC<4>{});
+  else f(IntC<kRnPer>{});
+}
+
+template <int NP, typename TY>
+__device__ __forceinline__ void rms_tail(const float (&v)[NP], const float (&wv)[NP], float ss,
                                          float* red, float eps, int64_t D, int64_t row, float* xo, int64_t ldxo,
                                          TY* y, int64_t ldy);
 
-template <typename TR, typename TY>
+template <int NP, typename TR, typename TY>
 __global__ __launch_bounds__(kRnThreads) void k_rmsnorm(const float* x, int64_t ldx, const TR* r, int64_t ldr,
                                                         const float* w, float eps, int64_t D, float* xo,
                                                         int64_t ldxo, TY* y, int64_t ldy) {
   __shared__ float red[kRnThreads / VNX_WAVE];
   const int64_t row = blockIdx.x;
   const int tid = threadIdx.x;
-  float v[kRnPer], wv[kRnPer], rv[kRnPer];
+  float v[NP], wv[NP], rv[NP];
   float ss = 0.0f;
   // Every load (x, residual, weight) is issued before any value is used, with
   // no per-lane condition between them (columns past D re-read column D - 1
   // and count as 0 below): a use or a select beside a conditional load would
   // wait there for every load in flight.  nb (wave-uniform) bounds the blocks.
-  const int nb = (int)min((int64_t)kRnPer, (D + kRnThreads - 1) / kRnThreads);
+  const int nb = (int)min((int64_t)NP, (D + kRnThreads - 1) / kRnThreads);
 #pragma unroll
-  for (int j = 0; j < kRnPer; ++j) {
+  for (int j = 0; j < NP; ++j) {
     if (j < nb) {
       const int64_t c = min((int64_t)(tid + j * kRnThreads), D - 1);
       v[j] = x[row * ldx + c];
@@ -126,7 +136,7 @@ __global__ __launch_bounds__(kRnThreads) void k_rmsnorm(const float* x, int64_t 
     }
   }
 #pragma unroll
-  for (int j = 0; j < kRnPer; ++j) {
+  for (int j = 0; j < NP; ++j) {
     const bool in = j < nb && tid + j * kRnThreads < D;
     float a = 0.0f;
     if (j < nb) {
@@ -138,19 +148,18 @@ __global__ __launch_bounds__(kRnThreads) void k_rmsnorm(const float* x, int64_t 
     v[j] = a;
     ss = __builtin_fmaf(a, a, ss);
   }
-  rms_tail<TY>(v, wv, ss, red, eps, D, row, xo, ldxo, y, ldy);
+  rms_tail<NP, TY>(v, wv, ss, red, eps, D, row, xo, ldxo, y, ldy);
 }
 
 // x_out[row] = x (the residual stream), y[row] = x / sqrt(mean(x^2) + eps) * w
-// from a workgroup's values v (kRnPer per thread, column tid + j*256) and
+// from a workgroup's values v (NP per thread, column tid + j*256) and
 // their per-thread sum of squares ss.
-template <typename TY>
-__device__ __forceinline__ void rms_tail(const float (&v)[kRnPer], const float (&wv)[kRnPer], float ss,
+template <int NP, typename TY>
+__device__ __forceinline__ void rms_tail(const float (&v)[NP], const float (&wv)[NP], float ss,
                                          float* red, float eps, int64_t D, int64_t row, float* xo, int64_t ldxo,
                                          TY* y, int64_t ldy) {
   const int tid = threadIdx.x;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, VNX_WAVE);
+  ss = wave_reduce(ss, [](float a, float b) { return a + b; });
   if ((tid & 63) == 0) red[tid >> 6] = ss;
   __syncthreads();
   float tot = 0.0f;
@@ -158,7 +167,7 @@ __device__ __forceinline__ void rms_tail(const float (&v)[kRnPer], const float (
   for (int i = 0; i < kRnThreads / VNX_WAVE; ++i) tot += red[i];
   const float inv = 1.0f / __builtin_sqrtf(tot / (float)D + eps);
 #pragma unroll
-  for (int j = 0; j < kRnPer; ++j) {
+  for (int j = 0; j < NP; ++j) {
     const int c = tid + j * kRnThreads;
     if (c < D) {
       if (xo) xo[row * ldxo + c] = v[j];
@@ -169,7 +178,7 @@ __device__ __forceinline__ void rms_tail(const float (&v)[kRnPer], const float (
 
 // The first layer's norm with the embedding lookup folded in: x[row] =
 // emb[tokens[row]] * scale (fp32), written to x_out as the residual stream.
-template <typename TE, typename TY>
+template <int NP, typename TE, typename TY>
 __global__ __launch_bounds__(kRnThreads) void k_embed_rmsnorm(const int64_t* tokens, const TE* emb, int64_t lde,
                                                               int64_t vocab, float scale, const float* w, float eps,
                                                               int64_t D, float* xo, int64_t ldxo, TY* y,
@@ -180,10 +189,10 @@ __global__ __launch_bounds__(kRnThreads) void k_embed_rmsnorm(const int64_t* tok
   int64_t tok = tokens[row];
   tok = tok < 0 ? 0 : (tok >= vocab ? vocab - 1 : tok);  // never outside the table
   const TE* e = emb + tok * lde;
-  float v[kRnPer], wv[kRnPer];
+  float v[NP], wv[NP];
   float ss = 0.0f;
 #pragma unroll
-  for (int j = 0; j < kRnPer; ++j) {
+  for (int j = 0; j < NP; ++j) {
     const int c = tid + j * kRnThreads;
     float a = 0.0f;
     wv[j] = 0.0f;
@@ -194,7 +203,7 @@ __global__ __launch_bounds__(kRnThreads) void k_embed_rmsnorm(const int64_t* tok
     v[j] = a;
     ss = __builtin_fmaf(a, a, ss);
   }
-  rms_tail<TY>(v, wv, ss, red, eps, D, row, xo, ldxo, y, ldy);
+  rms_tail<NP, TY>(v, wv, ss, red, eps, D, row, xo, ldxo, y, ldy);
 }
 
 // ---------------------------------------------------------------------------
@@ -305,7 +314,11 @@ constexpr int kModMaxE = 16;
 // is the number of its segment's logits that beat it (larger, or equal at a
 // lower index), it is selected when rank < topk, and the selected logits are
 // re-softmaxed with the sum taken in rank order (largest first).  Lane
-// P + p*E + e writes c[p*E + e].  All exchanges are wave shuffles.
+// P + p*E + e writes c[p*E + e].  All exchanges are wave shuffles and ballots;
+// every lane already knows its rank, so the value of a rank is one ballot away
+// (recomputing the ranks per term was a chain of topk * E * E shuffles: with
+// the wave sums on LDS permutes, the routing of 2,048 rows of 1,024, 4 parts
+// of 4 experts, took 39 us, now 25; of 224 rows 15, now 9).
 __device__ void route_wave(float lj, int P, int E, int topk, float* c) {
   const int lane = threadIdx.x & 63;
   const int R = P + P * E;
@@ -327,20 +340,14 @@ __device__ void route_wave(float lj, int P, int E, int topk, float* c) {
     rank += (v > lj || (v == lj && e2 < e)) ? 1 : 0;
     ms = fmaxf(ms, v);
   }
-  // sum of the selected terms in rank order
+  // sum of the selected terms in rank order (NaN logits can leave a rank out,
+  // which then counts as 0, or share one, which then goes to the last)
+  const uint64_t seg = ((1ull << E) - 1ull) << base;
   float ss = 0.0f;
   for (int i = 0; i < topk; ++i) {
-    float vi = 0.0f;
-    for (int e2 = 0; e2 < E; ++e2) {
-      const float v = __shfl(lj, base + e2);
-      int r2 = 0;
-      for (int e3 = 0; e3 < E; ++e3) {
-        const float w = __shfl(lj, base + e3);
-        r2 += (w > v || (w == v && e3 < e2)) ? 1 : 0;
-      }
-      if (r2 == i) vi = v;
-    }
-    ss += expf(vi - ms);
+    const uint64_t at = __ballot(rank == i) & seg;
+    const float v = __shfl(lj, at ? 63 - (int)__builtin_clzll(at) : base);
+    ss += expf((at ? v : 0.0f) - ms);
   }
   c[p * E + e] = rank < topk ? pw * (expf(lj - ms) / ss) : 0.0f;
 }
@@ -428,15 +435,12 @@ __global__ __launch_bounds__(256) void k_mod_route_x(const float* h, int64_t ldh
 #pragma unroll
   for (int r = 0; r < RM; ++r) {
     if (r < R) {
-      float v = acc[r];
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, VNX_WAVE);
+      const float v = wave_reduce(acc[r], [](float a, float b) { return a + b; });
       if (lane == 0) red[wave][r] = v;
     }
   }
   if (nw) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, VNX_WAVE);
+    ss = wave_reduce(ss, [](float a, float b) { return a + b; });
     if (lane == 0) ssr[wave] = ss;
   }
   __syncthreads();
@@ -626,8 +630,10 @@ int vnx_rmsnorm(const float* x, int64_t ldx, const void* res, int res_dtype, int
     using TR = decltype(tr);
     return by_dtype(y_dtype, [&](auto ty) {
       using TY = decltype(ty);
-      hipLaunchKernelGGL((k_rmsnorm<TR, TY>), dim3((unsigned)M), dim3(kRnThreads), 0, s, x, ldx,
-                         static_cast<const TR*>(res), ldr, w, eps, D, x_out, ldxo, static_cast<TY*>(y), ldy);
+      by_rn_per(D, [&](auto np) {
+        hipLaunchKernelGGL((k_rmsnorm<decltype(np)::value, TR, TY>), dim3((unsigned)M), dim3(kRnThreads), 0, s, x, ldx,
+                           static_cast<const TR*>(res), ldr, w, eps, D, x_out, ldxo, static_cast<TY*>(y), ldy);
+      });
       VNX_LAUNCH_CHECK();
       return (int)VNX_OK;
     });
@@ -647,9 +653,11 @@ int vnx_embed_rmsnorm(const int64_t* tokens, const void* emb, int emb_dtype, int
     using TE = decltype(te);
     return by_dtype(y_dtype, [&](auto ty) {
       using TY = decltype(ty);
-      hipLaunchKernelGGL((k_embed_rmsnorm<TE, TY>), dim3((unsigned)M), dim3(kRnThreads), 0, s, tokens,
-                         static_cast<const TE*>(emb), lde, vocab, scale, w, eps, D, x_out, ldxo, static_cast<TY*>(y),
-                         ldy);
+      by_rn_per(D, [&](auto np) {
+        hipLaunchKernelGGL((k_embed_rmsnorm<decltype(np)::value, TE, TY>), dim3((unsigned)M), dim3(kRnThreads), 0, s,
+                           tokens, static_cast<const TE*>(emb), lde, vocab, scale, w, eps, D, x_out, ldxo,
+                           static_cast<TY*>(y), ldy);
+      });
       VNX_LAUNCH_CHECK();
       return (int)VNX_OK;
     });

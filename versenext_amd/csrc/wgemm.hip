@@ -348,7 +348,7 @@ int wg_run(WgParams p, int epi, int y_dtype, hipStream_t s) {
   const dim3 grid((unsigned)wgs);
   // One row tile reads each byte of W once.  A W past 64 MB then leaves nothing
   // in the caches that this launch would read again, and pushes out the layers
-  // the next launches read, so it streams past them: the 248,320 x 512 head at
+  // the next launches read, so it streams past them: the 248,320 x 1,024 head at
   // 4-128 rows 89-110 -> 87-103 us, and a 4-layer verify of 8 x 7 tokens around
   // it 344 -> 330 us.  From two row tiles on the second read has to hit: at 224
   // rows 143 us cached, 181 us streamed.
