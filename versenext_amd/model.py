@@ -811,9 +811,8 @@ class CometSparkGPU:
         return o
 
     def _attn_torch(self, q, li, lens, n, Tmax):
-        """The same three paths with explicit fp32 masks: bf16 prefill chunks
-        longer than 64 rows or than the window, and head sizes the kernel does
-        not take.  q (B, H, n, d)."""
+        """The same three paths with explicit fp32 masks, for head sizes that
+        neither kernel takes.  q (B, H, n, d)."""
         cfg = self.cfg
         B, H, _, d = q.shape
         rep = H // cfg.n_kv_head
