@@ -837,8 +837,9 @@ int vnx_expert_gemm_bf16(const void* x, int64_t ldx, int64_t sxb, const void* w_
 
 /* The same products for any M (prefill): X_z[j] = x[z*sxb + rows[z*M + j]*ldx]
  * (rows NULL: row j), j < counts[z], with the lists vnx_mod_lists wrote; comb
- * (VNX_EPI_SWIGLU only) weights row j by comb[row*ldc + z].  total_rows: an
- * upper bound of the sum of counts (0: experts * M), which sizes the launch.
+ * (VNX_EPI_SWIGLU only) weights row j by comb[row*ldc + z].  total_rows: the
+ * expected sum of counts (0: experts * M), for the choice of a tile shape only:
+ * every listed row is computed however many there are.
  *
  * vnx_mod_lists: L_z = { m < M : comb[m*ldc + z] != 0 } ascending, as rows[z*M
  * + j] = l_j, counts[z] = n_z and slots[m*experts + z] = j for m = l_j, else

@@ -425,3 +425,30 @@ def test_verify_forward_is_reproducible(hip):
     h2 = m.logits(m.forward(new, lens, 30))
     torch.cuda.synchronize()
     assert torch.equal(h1, h2)
+
+
+@pytest.mark.parametrize("B,n,bad", [(2, 512, (0,)), (4, 130, (1, 2)), (8, 40, (3,)), (5, 7, (0,))])
+def test_a_nan_sequence_leaves_the_others_as_they_are(hip, B, n, bad):
+    """Sequences whose embeddings are NaN route to every expert with NaN
+    weights; the other sequences' hidden states and cache rows are those of
+    the batch without them, bit for bit."""
+    _say("nan sequences", B, n, bad)
+    cfg = VM.ModelConfig(vocab_size=500, dim=256, n_layer=2, n_head=4, n_kv_head=2, layer_pattern=("mod", "trisparse"),
+                         window_size=1024, num_global_tokens=8, use_alibi=False, use_rope=True, num_dense_parts=4,
+                         num_experts_per_part=4, top_k=2)
+    dev = hip.torch_device
+    m = VM.CometSparkGPU(cfg, VM.init_weights(cfg, seed=4), hip, batch=B, capacity=n + 8, dtype=torch.bfloat16)
+    m.emb[499] = float("nan")
+    tok = torch.randint(0, 499, (B, n), generator=torch.Generator().manual_seed(n)).to(dev)
+    lens = torch.zeros(B, dtype=torch.int32, device=dev)
+    with_nan = tok.clone()
+    with_nan[list(bad)] = 499
+    torch.full((64 << 20,), 1e30, device=dev)              # what a buffer not written would hold
+    got = m.forward(with_nan, lens, 0)
+    kv = [torch.stack([k, v]) for k, v in zip(m.kc, m.vc)]
+    assert bool(torch.isnan(got[list(bad)]).all())
+    ok = [b for b in range(B) if b not in bad]
+    want = m.forward(tok, lens, 0)
+    assert torch.equal(got[ok], want[ok])
+    for old, k, v in zip(kv, m.kc, m.vc):
+        assert torch.equal(old[:, ok], torch.stack([k, v])[:, ok])

@@ -135,3 +135,27 @@ def test_routed_rows(hip, M, N, K, E, kind, epi, dtype):
         for z, t in enumerate(ref):
             _check(y[z, :t.numel()], x[t], w[z], epi, comb[t, z] if epi else None)
             assert bool((y[z, t.numel():] == 9).all())
+
+
+@pytest.mark.parametrize("M,N,K,E", [(2048, 5376, 128, 16), (1024, 512, 192, 16), (300, 96, 64, 3)])
+def test_routed_rows_past_the_callers_bound(hip, M, N, K, E):
+    """total_rows below the counts' sum (rows whose router logits are NaN
+    select every expert): every listed row is computed all the same."""
+    print("routed rows past the bound", M, N, K, E, flush=True)
+    dev, L = hip.torch_device, hip._L
+    x, w = _inputs(hip, M, N, K, E, seed=M + K)
+    comb = torch.full((M, E), float("nan"), device=dev)
+    comb[M // 2:] = _routing(hip, M, E, "half")[M // 2:]
+    rows = torch.empty((E, M), dtype=torch.int32, device=dev)
+    counts = torch.empty((E,), dtype=torch.int32, device=dev)
+    slots = torch.empty((M, E), dtype=torch.int32, device=dev)
+    _lib.check(L.vnx_mod_lists(P(comb), E, M, E, P(rows), P(counts), P(slots), _st()))
+    wp, n = _pack(w), counts.tolist()
+    assert min(n) >= M // 2                                # a NaN weight is not 0: the row is on every list
+    for bound in (M * E // 2, 1):
+        y = torch.full((E, M, N), 9.0, dtype=torch.bfloat16, device=dev)
+        _lib.check(L.vnx_expert_gemm_bf16_rows(P(x), K, 0, P(wp), wp.stride(0), M, N, K, E, 0, None, E, P(rows), P(counts),
+                                               bound, P(y), _lib.DTYPE_CODES[torch.bfloat16], N, M * N, _st()))
+        for z in range(E):
+            _check(y[z, :n[z]], x[rows[z, :n[z]].long()], w[z], 0)
+            assert bool((y[z, n[z]:] == 9).all())

@@ -65,7 +65,7 @@ struct WgParams {
   const int32_t* counts;
   int64_t ldx, sxb, swb, ldy, syb, ldc;
   int M, N, K, batch;
-  int64_t total_rows;      // with counts: an upper bound of their sum (0: batch * M)
+  int64_t total_rows;      // with counts: their expected sum (0: batch * M), for the choice of a tile shape
   int nt, ng;              // 32-column tiles, N groups of a workgroup's (set by wg_run)
   int vec_out;
 };

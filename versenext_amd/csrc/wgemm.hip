@@ -323,13 +323,12 @@ int wg_run(WgParams p, int epi, int y_dtype, hipStream_t s) {
   p.nt = (int)(((int64_t)p.N + 31) / 32);
   const int ncols = epi == 1 ? p.N / 2 : p.N;
   p.vec_out = aligned16(p.y) && p.ldy % 8 == 0 && p.syb % 8 == 0 && (epi == 1 || p.N % 32 == 0) && ncols % 8 == 0;
-  // Row tiles over all groups for a shape of rt 32-row tiles: where counts
-  // rule, total_rows bounds the live ones.
+  // Row tiles over all groups for a shape of rt 32-row tiles: all of them, and
+  // as many as total_rows lets expect where counts rule.
+  auto all_tiles = [&](int rt) -> int64_t { return (int64_t)p.batch * ((p.M + 32 * rt - 1) / (32 * rt)); };
   auto row_tiles = [&](int rt) -> int64_t {
-    const int64_t all = (int64_t)p.batch * ((p.M + 32 * rt - 1) / (32 * rt));
-    if (!p.counts || p.total_rows <= 0) return all;
-    const int64_t most = p.total_rows / (32 * rt) + p.batch;
-    return most < all ? most : all;
+    const int64_t all = all_tiles(rt), most = p.total_rows / (32 * rt) + p.batch;
+    return p.counts && p.total_rows > 0 && most < all ? most : all;
   };
   auto groups = [&](int ct) { return (p.nt + 4 * ct - 1) / (4 * ct); };
   // 128 x 256 tiles where they fill two workgroups per CU, 64 x 256 where
@@ -340,8 +339,13 @@ int wg_run(WgParams p, int epi, int y_dtype, hipStream_t s) {
   // 2,048 x 2,048 x 1,024 17.2 / 13.3 / 13.9, 2,048 x 1,024 x 2,752 41 / 28 / 22.
   const int64_t cus = device_cus();
   const int sh = row_tiles(4) * groups(2) >= 2 * cus ? 0 : row_tiles(2) * groups(2) >= cus ? 1 : 2;
-  const int64_t tiles = sh == 0 ? row_tiles(4) * groups(2) : sh == 1 ? row_tiles(2) * groups(2)
-                                                                      : row_tiles(2) * groups(1);
+  // The launch covers all rows whatever total_rows says: how many rows the
+  // lists hold is the device's to know (a row whose router logits are NaN is on
+  // every expert's), and the workgroups past the live tiles return at once (a
+  // prefill of 4 x 512 tokens with one MoD layer: 875 us, as when the launch
+  // was cut to the expected rows).
+  const int64_t tiles = sh == 0 ? all_tiles(4) * groups(2) : sh == 1 ? all_tiles(2) * groups(2)
+                                                                      : all_tiles(2) * groups(1);
   p.ng = groups(sh == 2 ? 1 : 2);
   const int64_t wgs = (tiles + kVgXcds - 1) / kVgXcds * kVgXcds;
   if (wgs >= INT_MAX) return VNX_ERR_UNSUPPORTED;

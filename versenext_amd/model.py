@@ -891,7 +891,7 @@ class CometSparkGPU:
                 P_(act), He, M * He, P_(w2p), w2p.stride(0), M, D, He, PE, _lib.VNX_EPI_NONE, None, 0, 0, None,
                 P_(counts), None, P_(y), bf, D, M * D, self._st()), "expert_gemm w2")
         else:
-            total = M * P * min(k, E)
+            total = M * P * min(k, E)                      # (a row with NaN logits is on every list)
             _lib.check(L_.vnx_mod_lists(P_(comb), PE, M, PE, P_(rows), P_(counts), P_(slots), self._st()),
                        "mod_lists")
             _lib.check(L_.vnx_expert_gemm_bf16_rows(
