@@ -1113,19 +1113,32 @@ class CometSparkGPU:
         head, vnx_gemv_w4 for an INT4 draft, F.linear for an fp32 model."""
         B, n, D = hidden.shape
         V = self.cfg.vocab_size
+        if D != self.cfg.dim:
+            raise ValueError(f"hidden has {D} features, the model {self.cfg.dim}")
         h2 = hidden.reshape(B * n, D)
         if self.head is not None:
             if out is not None:
                 self.head(h2, out=out.view(B * n, V))
                 return out
             return self.head(h2).view(B, n, V)
-        if self.head_p is not None and (out is None or out.dtype in (torch.float32, torch.bfloat16)):
-            if out is None:
-                out = torch.empty((B, n, V), dtype=torch.float32, device=self.dev)
-            x, y = h2.to(torch.bfloat16).contiguous(), out.view(B * n, V)
+        if self.head_p is not None:
+            x = h2.to(self.dev, torch.bfloat16).contiguous()
+            o = out.view(B * n, V) if out is not None else None
+            direct = o is not None and o.device == x.device and o.dtype in (torch.float32, torch.bfloat16)
+            if direct and o.stride(1) != 1:
+                if B * n <= 256:
+                    raise ValueError(f"out must view as ({B * n}, {V}) with unit last stride")
+                direct = False
+            # an out that the kernel cannot write (many rows of other strides,
+            # another type or device) receives a copy
+            y = o if direct else torch.empty((B * n, V), dtype=torch.float32, device=x.device)
             _lib.check(self.hip._L.vnx_gemm_bf16(
                 x.data_ptr(), D, 0, self.head_p.data_ptr(), 0, B * n, V, D, 1, _lib.VNX_EPI_NONE, None, 0,
                 y.data_ptr(), _lib.DTYPE_CODES[y.dtype], y.stride(0), 0, self._st()), "logits")
+            if out is None:
+                return y.view(B, n, V)
+            if not direct:
+                o.copy_(y)
             return out
         y = torch.nn.functional.linear(h2.to(self.dtype), self.head_w).float()
         if out is not None:
