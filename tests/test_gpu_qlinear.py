@@ -78,3 +78,20 @@ def test_refusals(hip):
     L = hip._L
     assert L.vnx_linear_w8(lin.wq.data_ptr(), _lib.VNX_BF16, 128, lin.wq.data_ptr(), 128, lin.scale.data_ptr(), 1, 64, 128,
                            None, lin.scale.data_ptr(), 64, None) == _lib.VNX_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("rows", [3, 40])
+def test_lazily_negated_operands(hip, rows):
+    """The imaginary part of a conjugate is a view whose memory holds the
+    other sign: the product and the bias are those of its values."""
+    lin, g = _layer(hip, 128, 256, "int8", seed=rows, bias=True)
+    z = torch.complex(torch.randn((256, rows), generator=g, device=hip.torch_device),
+                      torch.randn((256, rows), generator=g, device=hip.torch_device))
+    planes = torch.stack([z.real.t(), z.imag.t()]).contiguous()
+    x = torch.view_as_complex(planes.permute(1, 2, 0).contiguous()).conj().imag
+    assert x.is_neg() and torch.equal(lin(x), lin(x.resolve_neg().contiguous()))
+    neg = torch._neg_view(planes[0].contiguous())          # unit strides: the form that is read in place
+    assert neg.is_neg() and torch.equal(lin(neg), lin(neg.resolve_neg()))
+    want = lin(planes[0]) - lin.bias - lin.bias
+    lin.bias = torch._neg_view(lin.bias)
+    torch.testing.assert_close(lin(planes[0]), want, rtol=1e-5, atol=1e-5)

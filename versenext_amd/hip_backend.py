@@ -403,7 +403,7 @@ class HipBackend(DeviceBackend):
         kernel).  Where many row tiles times many weight rows would round
         each value again and again, one cast first is cheaper (1,024 x 8,192
         outputs of K = 5,120: 120 + 10 us against 152)."""
-        t = _to_tensor(x, self._torch_device)
+        t = _to_tensor(x, self._torch_device).resolve_neg()
         if t.shape[-1] != K:
             raise ValueError(f"activations have {t.shape[-1]} features, the weight expects {K}")
         if t.dtype == torch.float32:
@@ -416,7 +416,7 @@ class HipBackend(DeviceBackend):
     def _bias(self, bias, N: int):
         if bias is None:
             return None
-        b = _to_tensor(bias, self._torch_device, torch.float32).reshape(-1).contiguous()
+        b = _to_tensor(bias, self._torch_device, torch.float32).reshape(-1).contiguous().resolve_neg()
         if b.numel() != N:
             raise ValueError(f"bias must have {N} entries")
         return b
