@@ -95,3 +95,33 @@ def test_lazily_negated_operands(hip, rows):
     want = lin(planes[0]) - lin.bias - lin.bias
     lin.bias = torch._neg_view(lin.bias)
     torch.testing.assert_close(lin(planes[0]), want, rtol=1e-5, atol=1e-5)
+
+
+def test_the_bias_of_a_user(hip):
+    """A bias set on the layer keeps PyTorch's rules: its type promotes, its
+    tangent and its batching pass through, another device is refused."""
+    lin, g = _layer(hip, 128, 256, "int4_g128", seed=5, bias=True)
+    x = torch.randn((5, 256), generator=g, device=hip.torch_device)
+    b, lin.bias = lin.bias, None
+    y = lin(x)
+    lin.bias = b.double()
+    assert lin(x).dtype == torch.float64 and torch.equal(lin(x), y + b.double())
+    lin.bias = b.half()
+    assert torch.equal(lin(x), y + b.half())
+    lin.bias = b.cpu()
+    with pytest.raises(RuntimeError):
+        lin(x)
+    import torch.autograd.forward_ad as fwd
+
+    with fwd.dual_level():
+        lin.bias = fwd.make_dual(b, torch.ones_like(b))
+        out = fwd.unpack_dual(lin(x))
+        assert torch.equal(out.primal, y + b) and torch.equal(out.tangent, torch.ones_like(y))
+
+    def call(v):
+        lin.bias = v
+        return lin(x)
+
+    bs = torch.stack([b, 2 * b])
+    assert torch.equal(torch.func.vmap(call)(bs), torch.stack([y + b, y + 2 * b]))
+    lin.bias = None

@@ -20,6 +20,7 @@ from typing import Optional
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 from .device import get_backend
 
@@ -149,12 +150,21 @@ class QuantizedLinear:
         return self.backend.dequant_w4(self.wq, self.scale, self.in_features, group)
 
     def forward(self, x) -> torch.Tensor:
-        # a plain (out,) bias is added by the kernel; one that a gradient flows
-        # to, or of another shape, by PyTorch
+        # a plain (out,) fp32 bias is added by the kernel, any other by PyTorch
         b = self.bias
-        fuse = b is not None and b.shape == (self.out_features,) and not (b.requires_grad and torch.is_grad_enabled())
+        fuse = b is not None and self._plain_bias(b)
         y = self._product(x, b if fuse else None)
         return y if b is None or fuse else y + b
+
+    def _plain_bias(self, b) -> bool:
+        """Whether adding b is no more than adding its values: not of another
+        type (PyTorch promotes), shape or device, and with nothing that follows
+        it (a gradient, a forward-mode tangent, a transform of torch.func)."""
+        return (type(b) in (torch.Tensor, torch.nn.Parameter) and b.dtype == torch.float32
+                and b.shape == (self.out_features,) and b.device == self.wq.device
+                and not (b.requires_grad and torch.is_grad_enabled())
+                and not torch._C._functorch.is_functorch_wrapped_tensor(b)
+                and forward_ad.unpack_dual(b).tangent is None)
 
     def _product(self, x, bias) -> torch.Tensor:
         if self.qtype == "int8":
