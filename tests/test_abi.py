@@ -162,3 +162,13 @@ def test_check_maps_status_to_reference_exceptions():
     with pytest.raises(RuntimeError):
         _lib.check(-5)
     _lib.check(0)
+
+
+def test_gemm_rows_past_the_kernels_index_range_are_refused():
+    """The kernel numbers rows and columns up to a tile past the last one in 32
+    bits; nothing is launched (the addresses are never read)."""
+    L, at = _lib.lib(), 1 << 20
+    for M, N in [(2 ** 31 - 100, 64), (64, 2 ** 31 - 100)]:
+        assert L.vnx_gemm_bf16(at, 64, 0, at, 0, M, N, 64, 1, _lib.VNX_EPI_NONE, None, 0, at, _lib.VNX_BF16, N, 0,
+                               None) == _lib.VNX_ERR_UNSUPPORTED
+        assert L.vnx_gemm_bf16_residual(at, 64, at, M, N, 64, at, N, None) == _lib.VNX_ERR_UNSUPPORTED

@@ -320,6 +320,8 @@ __global__ __launch_bounds__(1024) void k_mod_lists(const float* comb, int64_t l
 }  // namespace
 
 int wg_run(WgParams p, int epi, int y_dtype, hipStream_t s) {
+  // rows and columns are numbered to the end of their last tile in 32 bits
+  if (p.M >= INT_MAX - 256 || p.N >= INT_MAX - 256) return VNX_ERR_UNSUPPORTED;
   p.nt = (int)(((int64_t)p.N + 31) / 32);
   const int ncols = epi == 1 ? p.N / 2 : p.N;
   p.vec_out = aligned16(p.y) && p.ldy % 8 == 0 && p.syb % 8 == 0 && (epi == 1 || p.N % 32 == 0) && ncols % 8 == 0;
@@ -411,7 +413,7 @@ int vnx_expert_gemm_bf16_rows(const void* x, int64_t ldx, int64_t sxb, const voi
   if (M == 0 || N == 0 || experts == 0) return VNX_OK;
   if (K % kVgChunk || ldx % 8 || sxb % 8 || swb % 8 || !aligned16(x) || !aligned16(w_packed))
     return VNX_ERR_UNSUPPORTED;
-  if (M >= INT_MAX - 256 || N >= INT_MAX - 256 || K >= INT_MAX) return VNX_ERR_UNSUPPORTED;
+  if (M >= INT_MAX || N >= INT_MAX || K >= INT_MAX) return VNX_ERR_UNSUPPORTED;
   WgParams p{};
   p.x = static_cast<const uint16_t*>(x); p.w = static_cast<const uint16_t*>(w_packed); p.y = y; p.comb = comb;
   p.rows = rows; p.counts = counts; p.total_rows = total_rows;
