@@ -125,3 +125,17 @@ def test_the_bias_of_a_user(hip):
     bs = torch.stack([b, 2 * b])
     assert torch.equal(torch.func.vmap(call)(bs), torch.stack([y + b, y + 2 * b]))
     lin.bias = None
+
+
+@pytest.mark.parametrize("rows,N,K", [(3, 32905, 1024), (30, 32905, 1024), (16, 40001, 512), (45, 33000, 512)])
+def test_head_with_bias(hip, rows, N, K):
+    """The streaming kernel of a head's many weight rows: the bias travels with
+    the tiles' loads, fp16 and fp32 activations alike."""
+    lin, g = _layer(hip, N, K, "int4_g128", seed=rows, bias=True)
+    x = torch.randn((rows, K), generator=g, device=hip.torch_device)
+    y = lin(x)
+    _check(lin, x, y)
+    b, lin.bias = lin.bias, None
+    assert torch.equal(y, lin(x) + b) and torch.equal(lin(x), lin(x.half()))
+    lin.bias = b
+    assert torch.equal(y, lin(x.half()))

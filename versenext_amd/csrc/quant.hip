@@ -172,9 +172,9 @@ __device__ __forceinline__ u32x4 half8_bits(u32x4 lo, u32x4 hi) {
   return __builtin_bit_cast(u32x4, o);
 }
 
-// x[b, k .. k + 8) as fp16 (fp32 rows rounded).
-__device__ __forceinline__ u32x4 load_x8(const QGemvParams& p, int64_t b, int64_t k) {
-  if (p.x32) {
+// x[b, k .. k + 8) as fp16 (f32: fp32 rows rounded).
+__device__ __forceinline__ u32x4 load_x8(const QGemvParams& p, int64_t b, int64_t k, bool f32) {
+  if (f32) {
     const u32x4* src = reinterpret_cast<const u32x4*>(p.x32 + b * p.ldx + k);
     return half8_bits(src[0], src[1]);
   }
@@ -183,13 +183,18 @@ __device__ __forceinline__ u32x4 load_x8(const QGemvParams& p, int64_t b, int64_
 
 // v += bias[n0 .. n0 + 4) (columns past N repeat the last: not stored).
 __device__ __forceinline__ void add_bias4(const QGemvParams& p, int64_t n0, f32x4& v) {
-  if (!p.bias) return;
 #pragma unroll
   for (int j = 0; j < 4; ++j) v[j] += p.bias[min(n0 + j, p.N - 1)];
 }
 
-template <int BITS, int NC, int TPW>
+// XF: x is fp32; BIAS: p.bias is added.  INT8 up to 16 rows tests both at run
+// time, which keeps its staging loop short (us, 248,320 x 1,024, tested / known
+// at compile time: INT8 8 rows fp32 57.7 / 59.3, fp16 56.1 / 57.5; INT4 8 rows
+// 54.1 / 53.0; INT8 32 rows of 32,768 x 4,096 fp16 48.3 / 47.2).
+template <int BITS, int NC, int TPW, bool XF, bool BIAS>
 __global__ __launch_bounds__(kQNT) void k_qgemv(QGemvParams p) {
+  constexpr bool TEST = BITS == 8 && NC == 1;
+  const bool xf = TEST ? p.x32 != nullptr : XF;
   constexpr int KS = 1024 / NC;                 // k per slice
   constexpr int XS = KS + kXPad;                // LDS row pitch of x (fp16)
   constexpr int NG = KS / kGK;                  // groups per slice
@@ -222,7 +227,7 @@ __global__ __launch_bounds__(kQNT) void k_qgemv(QGemvParams p) {
     for (int idx = tid; idx < brows * (KS / 8); idx += kQNT) {
       const int b = idx / (KS / 8), c8 = idx % (KS / 8);
       u32x4 v = {0u, 0u, 0u, 0u};
-      if (b < p.B && c8 * 8 < ks) v = load_x8(p, b, k0 + c8 * 8);
+      if (b < p.B && c8 * 8 < ks) v = load_x8(p, b, k0 + c8 * 8, xf);
       if constexpr (BITS == 4) v = stage_perm_w4(v);
       *reinterpret_cast<u32x4*>(&xs[b * XS + c8 * 8]) = v;
     }
@@ -329,7 +334,7 @@ __global__ __launch_bounds__(kQNT) void k_qgemv(QGemvParams p) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[j] *= load_scale(p, min(n0 + j, p.N - 1), 0);
       }
-      add_bias4(p, n0, v);
+      if (TEST ? p.bias != nullptr : BIAS) add_bias4(p, n0, v);
       float* dst = out + b * ldo + n0;
       if (n0 + 4 <= p.N && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
         *reinterpret_cast<f32x4*>(dst) = v;
@@ -351,14 +356,15 @@ __global__ __launch_bounds__(kQNT) void k_qgemv(QGemvParams p) {
 // own LDS tile: coalesced 256-byte row reads in, the MFMA B-operand layout
 // out.
 // QE: 0 plain fp32 output, 1 SwiGLU (fp16), 2 RoPE + KV-cache store,
-// 3 residual (y += the product, fp32).  NX (W4): x is RMSNorm(xf) * nw: the
+// 3 residual (y += the product, fp32), 4 plain with the bias.  NX (W4): x is RMSNorm(xf) * nw: the
 // staged operand is fp16(xf * nw), each wave sums the squares of its groups'
 // values per row, and the epilogue scales row b by rstd_b = 1/sqrt(mean
 // xf^2 + eps) (vnnn.py:593-615, the per-row factor on the fp32 sums).
 // NX 2: the same with the rows gathered from the token embedding (the first
 // block's norm of CometSparkV05LM.forward, spark/src/base_model.py:170-208);
 // group g's values of every row go to xout from workgroup g % gridDim.x, so
-// the fp32 residual stream starts without a launch of its own.
+// the fp32 residual stream starts without a launch of its own.  NX 3 (QE 0, 4):
+// fp32 rows rounded to fp16.
 // TP: 16-row tiles per workgroup (2 for grids of more tiles than CUs: each
 // wave's x block is loaded and staged once for both tiles).  GP: groups per
 // pass of a wave (1 where K has at most one group per wave, or TP 2).
@@ -665,7 +671,7 @@ __device__ __forceinline__ void qgemv_tile_body(const QGemvParams& p, char* smem
     }
     return;
   }
-  add_bias4(p, n0, v);
+  if constexpr (QE == 4) add_bias4(p, n0, v);
   float* dst = p.y + b * p.ldy + n0;
   if (n0 + 4 <= p.N && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
     *reinterpret_cast<f32x4*>(dst) = v;
@@ -694,8 +700,11 @@ __global__ __launch_bounds__(NW * 64) void k_qgemv_tile(QGemvParams p) {
 // through a ring of RS tiles in flight.  KG = K / 128 groups.  The MFMA takes
 // x as its A operand and the weights as B, so a lane's four outputs belong to
 // the one weight row it loads (batch rows 4kq .. 4kq + 3): each lane needs
-// only its own row's scales.
-template <int NC, int KG, int RS>
+// only its own row's scales.  BIAS (and XF) are template parameters because
+// any conditional load among a tile's math would make the compiler wait there
+// for the whole ring: with the bias behind a runtime test, 32 rows x 248,320 x
+// 1,024 took 50.7 us, without 43.4.  A bias travels in the ring.
+template <int NC, int KG, int RS, bool XF, bool BIAS>
 __global__ __launch_bounds__(kQNT) void k_qgemv_stream(QGemvParams p, int tiles_per_wg) {
   static_assert(KG == 4 || KG == 8, "K of 512 or 1024");
   using SV = std::conditional_t<KG == 8, u32x4, uint2>;  // one row's KG fp16 scales
@@ -708,7 +717,7 @@ __global__ __launch_bounds__(kQNT) void k_qgemv_stream(QGemvParams p, int tiles_
   for (int idx = tid; idx < NC * 16 * KG * 16; idx += kQNT) {
     const int b = idx / (KG * 16), c8 = idx % (KG * 16);
     u32x4 v = {0u, 0u, 0u, 0u};
-    if (b < p.B) v = load_x8(p, b, c8 * 8);
+    if (b < p.B) v = load_x8(p, b, c8 * 8, XF);
     *reinterpret_cast<u32x4*>(&xs[b * XS + c8 * 8]) = stage_perm_w4(v);
   }
   __syncthreads();
@@ -723,7 +732,7 @@ __global__ __launch_bounds__(kQNT) void k_qgemv_stream(QGemvParams p, int tiles_
   const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint8_t*>(p.w) + r_lo * p.ldw, (short)0, (int)((r_hi - r_lo) * p.ldw), 0x00020000);
   // one tile's loads: the lane's weight row (KG x 16 bytes) and its scales
-  auto load = [&](int64_t tile, u32x4 (&wv)[KG], SV& sv) {
+  auto load = [&](int64_t tile, u32x4 (&wv)[KG], SV& sv, float& bv) {
     const int64_t t = min(tile, tiles - 1);
     const int64_t rw = min(t * 16 + m, p.N - 1);
     const int64_t ra = min(rw, r_hi - 1);             // scale rows stay in the range (a cache hit past it)
@@ -733,6 +742,7 @@ __global__ __launch_bounds__(kQNT) void k_qgemv_stream(QGemvParams p, int tiles_
       wv[g] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wres, off + g * 64, 0, 2));
     (void)rw;
     sv = *reinterpret_cast<const SV*>(static_cast<const uint16_t*>(p.sc) + ra * p.lds);
+    if constexpr (BIAS) bv = p.bias[ra];
   };
   auto scale = [&](const SV& sv, int g) {
     uint32_t wd;
@@ -744,7 +754,7 @@ __global__ __launch_bounds__(kQNT) void k_qgemv_stream(QGemvParams p, int tiles_
     }
     return (float)__builtin_bit_cast(_Float16, (uint16_t)(wd >> (16 * (g % 2))));
   };
-  auto compute_store = [&](int64_t tile, const u32x4 (&wv)[KG], const SV& sv) {
+  auto compute_store = [&](int64_t tile, const u32x4 (&wv)[KG], const SV& sv, float bv) {
     f32x4 yacc[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) yacc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -775,27 +785,27 @@ __global__ __launch_bounds__(kQNT) void k_qgemv_stream(QGemvParams p, int tiles_
     if (tile >= t_hi) return;
     const int64_t n = tile * 16 + m;
     if (n >= p.N) return;
-    const float bv = p.bias ? p.bias[n] : 0.0f;
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int64_t b = c * 16 + 4 * kq + j;
-        if (b < p.B) p.y[b * p.ldy + n] = p.bias ? yacc[c][j] + bv : yacc[c][j];
+        if (b < p.B) p.y[b * p.ldy + n] = BIAS ? yacc[c][j] + bv : yacc[c][j];
       }
   };
   // RS slots: slot j holds tile ta + 4j; each slot is reloaded (tiles past
   // the range load the last tile again) as soon as its math is issued
   u32x4 wr[RS][KG];
   SV sr[RS];
+  float br[RS] = {};
   const int64_t t0 = t_lo + wave;
 #pragma unroll
-  for (int j = 0; j < RS; ++j) load(t0 + 4 * j, wr[j], sr[j]);
+  for (int j = 0; j < RS; ++j) load(t0 + 4 * j, wr[j], sr[j], br[j]);
   for (int64_t ta = t0; ta < t_hi; ta += 4 * RS) {
 #pragma unroll
     for (int j = 0; j < RS; ++j) {
-      compute_store(ta + 4 * j, wr[j], sr[j]);
-      load(ta + 4 * (j + RS), wr[j], sr[j]);
+      compute_store(ta + 4 * j, wr[j], sr[j], br[j]);
+      load(ta + 4 * (j + RS), wr[j], sr[j], br[j]);
     }
   }
 }
@@ -1294,10 +1304,15 @@ static int qgemv_launch(QGemvParams p, int bits, hipStream_t s) {
       const int64_t tiles = (c.N + 15) / 16;
       const bool wide = tiles <= device_cus();
       const dim3 grid((unsigned)tiles);
+#define VNX_QTILE_X(BITS, NC, NW, QE) \
+  do { \
+    if (c.x32) hipLaunchKernelGGL((k_qgemv_tile<BITS, NC, NW, QE, 3>), grid, dim3(NW * 64), 0, s, c); \
+    else hipLaunchKernelGGL((k_qgemv_tile<BITS, NC, NW, QE, 0>), grid, dim3(NW * 64), 0, s, c); \
+  } while (0)
 #define VNX_QTILE(BITS, NC, NW) \
   do { \
-    if (c.x32) hipLaunchKernelGGL((k_qgemv_tile<BITS, NC, NW, 0, 3>), grid, dim3(NW * 64), 0, s, c); \
-    else hipLaunchKernelGGL((k_qgemv_tile<BITS, NC, NW>), grid, dim3(NW * 64), 0, s, c); \
+    if (c.bias) VNX_QTILE_X(BITS, NC, NW, 4); \
+    else VNX_QTILE_X(BITS, NC, NW, 0); \
   } while (0)
 #define VNX_QTILE_E(NC, NW, QE, NX) \
   hipLaunchKernelGGL((k_qgemv_tile<4, NC, NW, QE, NX>), grid, dim3(NW * 64), 0, s, c)
@@ -1334,6 +1349,7 @@ static int qgemv_launch(QGemvParams p, int bits, hipStream_t s) {
         else { if (wide) VNX_QTILE(8, 1, 8); else VNX_QTILE(8, 1, 4); }
       }
 #undef VNX_QTILE
+#undef VNX_QTILE_X
 #undef VNX_QTILE_E
 #undef VNX_QTILE_E1
 #undef VNX_QTILE_E2
@@ -1353,23 +1369,36 @@ static int qgemv_launch(QGemvParams p, int bits, hipStream_t s) {
       const int nc = two ? 2 : 1;
       const size_t lds = (size_t)nc * 16 * (c.K + kXPad) * 2;
       // (a ring of 4 tiles measured 1.2x slower at B = 32: 199 VGPRs)
+#define VNX_QSTREAM_B(NC, KG, XF) \
+  do { \
+    if (c.bias) hipLaunchKernelGGL((k_qgemv_stream<NC, KG, 2, XF, true>), grid, dim3(kQNT), lds, s, c, (int)tpw); \
+    else hipLaunchKernelGGL((k_qgemv_stream<NC, KG, 2, XF, false>), grid, dim3(kQNT), lds, s, c, (int)tpw); \
+  } while (0)
 #define VNX_QSTREAM(NC, KG) \
-  hipLaunchKernelGGL((k_qgemv_stream<NC, KG, 2>), grid, dim3(kQNT), lds, s, c, (int)tpw)
+  do { if (c.x32) VNX_QSTREAM_B(NC, KG, true); else VNX_QSTREAM_B(NC, KG, false); } while (0)
       if (c.K == 512) { if (two) VNX_QSTREAM(2, 4); else VNX_QSTREAM(1, 4); }
       else { if (two) VNX_QSTREAM(2, 8); else VNX_QSTREAM(1, 8); }
 #undef VNX_QSTREAM
+#undef VNX_QSTREAM_B
     } else {
       const int tpw = c.B > 16 && c.N >= 256 * kQTargetWgs ? 4 : 1;
       const dim3 grid((unsigned)((c.N + 64 * tpw - 1) / (64 * tpw)));
-#define VNX_QLAUNCH(BITS, NC, TPW) hipLaunchKernelGGL((k_qgemv<BITS, NC, TPW>), grid, dim3(kQNT), 0, s, c)
+#define VNX_QLAUNCH_1(BITS, NC, TPW, XF, BIAS) \
+  hipLaunchKernelGGL((k_qgemv<BITS, NC, TPW, XF, BIAS>), grid, dim3(kQNT), 0, s, c)
+#define VNX_QLAUNCH_B(BITS, NC, TPW, XF) \
+  do { if (c.bias) VNX_QLAUNCH_1(BITS, NC, TPW, XF, true); else VNX_QLAUNCH_1(BITS, NC, TPW, XF, false); } while (0)
+#define VNX_QLAUNCH(BITS, NC, TPW) \
+  do { if (c.x32) VNX_QLAUNCH_B(BITS, NC, TPW, true); else VNX_QLAUNCH_B(BITS, NC, TPW, false); } while (0)
       if (bits == 4) {
         if (two) { if (tpw == 4) VNX_QLAUNCH(4, 2, 4); else VNX_QLAUNCH(4, 2, 1); }
         else { if (tpw == 4) VNX_QLAUNCH(4, 1, 4); else VNX_QLAUNCH(4, 1, 1); }
       } else {
         if (two) { if (tpw == 4) VNX_QLAUNCH(8, 2, 4); else VNX_QLAUNCH(8, 2, 1); }
-        else { if (tpw == 4) VNX_QLAUNCH(8, 1, 4); else VNX_QLAUNCH(8, 1, 1); }
+        else { if (tpw == 4) VNX_QLAUNCH_1(8, 1, 4, false, false); else VNX_QLAUNCH_1(8, 1, 1, false, false); }
       }
 #undef VNX_QLAUNCH
+#undef VNX_QLAUNCH_B
+#undef VNX_QLAUNCH_1
     }
     VNX_LAUNCH_CHECK();
   }
