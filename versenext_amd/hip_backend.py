@@ -400,23 +400,44 @@ class HipBackend(DeviceBackend):
     def _linear_x(self, x, K: int, N: int):
         """(lead shape, rows, dtype code): the activations as the GEMV
         entries read them, fp16 (B, K) or fp32 rows (rounded to fp16 in the
-        kernel).  Where many row tiles times many weight rows would round
-        each value again and again, one cast first is cheaper (1,024 x 8,192
-        outputs of K = 5,120: 120 + 10 us against 152)."""
-        t = _to_tensor(x, self._torch_device).resolve_neg()
+        kernel).  Every workgroup reads and rounds the rows again, so from
+        some size on one cast first is cheaper:
+        - a workgroup per 16 weight rows (up to 32 rows, fewer than 32,768
+          weight rows): from 2^30 of weight rows x K x staged rows, or K so
+          long that one workgroup's own rows weigh (us, rounded in the kernel
+          / cast first: INT8 16 rows x 16,384 x 2,048 14 / 17, x 4,096 27 /
+          22, 32 rows x 8,192 x 5,120 28 / 21, x 24,576 x 5,120 81 / 57; INT4
+          16 rows x 2,048 x 16,384 24 / 18);
+        - the tiled GEMM: from 2^22 outputs (1,024 x 8,192 of K = 5,120: 152 /
+          120 + 10);
+        - an LM head's kernels stage the rows once per many weight rows and
+          round them as fast as a cast writes them (INT4, 32 rows x 248,320 x
+          1,024: 45 / 45)."""
+        t = _to_tensor(x, self._torch_device)
+        if t.is_neg():
+            t = t.resolve_neg()
         if t.shape[-1] != K:
             raise ValueError(f"activations have {t.shape[-1]} features, the weight expects {K}")
         if t.dtype == torch.float32:
-            t2 = t.reshape(-1, K)
-            if (t2.shape[0] * N < 1 << 22 and t2.stride(1) == 1 and t2.stride(0) % 4 == 0 and t2.stride(0) >= K
-                    and t2.data_ptr() % 16 == 0):
-                return t.shape[:-1], t2, _lib.VNX_F32
+            t2 = t if t.dim() == 2 else t.reshape(-1, K)
+            M = t2.shape[0]
+            if M <= 32 and N < 32768:
+                staged = K * ((M + 15) // 16 * 16)
+                direct = staged < 1 << 18 and N * staged < 1 << 30
+            else:
+                direct = M * N < 1 << 22
+            if direct:
+                s0, s1 = t2.stride()
+                if s1 == 1 and s0 % 4 == 0 and s0 >= K and t2.data_ptr() % 16 == 0:
+                    return t.shape[:-1], t2, _lib.VNX_F32
         return t.shape[:-1], self._acts(t, K), _lib.VNX_F16
 
     def _bias(self, bias, N: int):
         if bias is None:
             return None
-        b = _to_tensor(bias, self._torch_device, torch.float32).reshape(-1).contiguous().resolve_neg()
+        b = _to_tensor(bias, self._torch_device, torch.float32)
+        if b.dim() != 1 or b.is_neg() or not b.is_contiguous():
+            b = b.reshape(-1).contiguous().resolve_neg()
         if b.numel() != N:
             raise ValueError(f"bias must have {N} entries")
         return b

@@ -164,7 +164,7 @@ class QuantizedLinear:
                 and b.shape == (self.out_features,) and b.device == self.wq.device
                 and not (b.requires_grad and torch.is_grad_enabled())
                 and not torch._C._functorch.is_functorch_wrapped_tensor(b)
-                and forward_ad.unpack_dual(b).tangent is None)
+                and (forward_ad._current_level < 0 or forward_ad.unpack_dual(b).tangent is None))
 
     def _product(self, x, bias) -> torch.Tensor:
         if self.qtype == "int8":
