@@ -159,3 +159,22 @@ def test_routed_rows_past_the_callers_bound(hip, M, N, K, E):
         for z in range(E):
             _check(y[z, :n[z]], x[rows[z, :n[z]].long()], w[z], 0)
             assert bool((y[z, n[z]:] == 9).all())
+
+
+# a head's columns: one and two row tiles with both tile shapes, a W that the
+# last-level cache holds beside the logits, one that it does not, and one that
+# streams (fp32 and 16-bit logits past the caches each, and not)
+@pytest.mark.parametrize("M,N,K,dtype", [
+    (224, 64000, 64, torch.bfloat16), (150, 64000, 64, torch.float32), (129, 100352, 64, torch.float16),
+    (256, 32768, 64, torch.float32), (131, 65536, 1984, torch.bfloat16), (97, 131104, 1088, torch.float32),
+    (128, 131104, 1088, torch.bfloat16), (33, 131111, 1088, torch.bfloat16)])
+def test_head_gemm(hip, M, N, K, dtype):
+    print("head gemm", M, N, K, dtype, flush=True)
+    x, w = _inputs(hip, M, N, K, 1, seed=M + K)
+    ldy = (N + 7) // 8 * 8 + 8
+    y = torch.full((M + 1, ldy), 7.0, dtype=dtype, device=hip.torch_device)
+    _lib.check(hip._L.vnx_gemm_bf16(P(x), K, 0, P(_pack(w)), 0, M, N, K, 1, 0, None, 0, P(y), _lib.DTYPE_CODES[dtype],
+                                    ldy, 0, _st()))
+    for n in range(0, N, 16384):
+        _check(y[:M, n:min(n + 16384, N)], x, w[0][n:n + 16384], 0)
+    assert bool((y[M] == 7).all()) and bool((y[:, N:] == 7).all())

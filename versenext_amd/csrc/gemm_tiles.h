@@ -25,8 +25,8 @@ __device__ __forceinline__ void vg_store(char* y, int64_t off, float v) {
 }
 
 // Eight consecutive outputs of type OT from fp32 (16 bytes for bf16 / fp16,
-// 32 for fp32).
-template <int OT>
+// 32 for fp32); NT: 16-bit ones past the caches.
+template <int OT, bool NT = false>
 __device__ __forceinline__ void vg_store8(char* y, int64_t off, const float (&v)[8]) {
   if constexpr (OT == 0) {
     float* d = reinterpret_cast<float*>(y) + off;
@@ -36,12 +36,16 @@ __device__ __forceinline__ void vg_store8(char* y, int64_t off, const float (&v)
     __bf16 t[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) t[e] = static_cast<__bf16>(v[e]);
-    *reinterpret_cast<u32x4*>(reinterpret_cast<__bf16*>(y) + off) = __builtin_bit_cast(u32x4, t);
+    u32x4* d = reinterpret_cast<u32x4*>(reinterpret_cast<__bf16*>(y) + off);
+    if constexpr (NT) __builtin_nontemporal_store(__builtin_bit_cast(u32x4, t), d);
+    else *d = __builtin_bit_cast(u32x4, t);
   } else {
     _Float16 t[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) t[e] = static_cast<_Float16>(v[e]);
-    *reinterpret_cast<u32x4*>(reinterpret_cast<_Float16*>(y) + off) = __builtin_bit_cast(u32x4, t);
+    u32x4* d = reinterpret_cast<u32x4*>(reinterpret_cast<_Float16*>(y) + off);
+    if constexpr (NT) __builtin_nontemporal_store(__builtin_bit_cast(u32x4, t), d);
+    else *d = __builtin_bit_cast(u32x4, t);
   }
 }
 

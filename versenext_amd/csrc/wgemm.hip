@@ -29,6 +29,8 @@
 namespace vnx {
 namespace {
 
+constexpr int kWgNtW = 1, kWgNtY = 2;
+
 // 16 bytes of W; NT: past the caches.
 template <bool NT>
 __device__ __forceinline__ u32x4 ld_w(const uint16_t* p) {
@@ -38,10 +40,12 @@ __device__ __forceinline__ u32x4 ld_w(const uint16_t* p) {
 
 // RT x CT tiles per wave; PD register sets of W and X (PD 1: one set, each W
 // register reloaded as soon as its products are issued); LA: A operands of LA
-// 16-k steps read ahead (PD 1; else the whole chunk's); OCC workgroups per CU; NT: W
-// is read past the caches (wg_run's rule).
-template <int OT, int EPI, int RT, int CT, int PD, int LA, int OCC, bool NT = false>
+// 16-k steps read ahead (PD 1; else the whole chunk's); OCC workgroups per CU; CP:
+// W is read (kWgNtW) or the outputs are written (kWgNtY) past the caches
+// (wg_run's rules).
+template <int OT, int EPI, int RT, int CT, int PD, int LA, int OCC, int CP = 0>
 __global__ __launch_bounds__(256, OCC) void k_wgemm(WgParams p) {
+  constexpr bool NT = CP & kWgNtW, NTY = CP & kWgNtY;
   constexpr int ROWS = 32 * RT;
   constexpr int UN = PD;
   constexpr int SLAB = ROWS * kVgRowB;
@@ -215,12 +219,16 @@ __global__ __launch_bounds__(256, OCC) void k_wgemm(WgParams p) {
     for (int t = 0; t < CT; ++t) {
       if (ni[t] >= p.nt) continue;             // uniform per wave
       if (p.vec_out) {
+        // fp32: lane l's piece q is row 8q + l / 8, columns 4 (l % 8) .. + 4, so
+        // eight lanes write (and EPI 3 reads) a whole 128-byte line of a row
+        constexpr bool F32 = OT == 0 && EPI != 1;
+        const int fr = m0 + i * 32 + (lane >> 3);
+        float* yf = reinterpret_cast<float*>(ybase) + (int64_t)fr * p.ldy + ni[t] * 32 + 4 * (lane & 7);
         f32x4 old[EPI == 3 ? 4 : 1];
-        float* yf = reinterpret_cast<float*>(ybase) + (int64_t)j * p.ldy + ni[t] * 32 + 16 * hf;
         if constexpr (EPI == 3) {
-          if (live)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) old[q] = *reinterpret_cast<const f32x4*>(yf + 4 * q);
+          for (int q = 0; q < 4; ++q)
+            if (fr + 8 * q < cnt) old[q] = *reinterpret_cast<const f32x4*>(yf + (int64_t)(8 * q) * p.ldy);
         }
 #pragma unroll
         for (int ii = 0; ii < 4; ++ii)
@@ -230,11 +238,16 @@ __global__ __launch_bounds__(256, OCC) void k_wgemm(WgParams p) {
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         const float* row = tr + (lane >> 1) * TP;
-        if constexpr (EPI == 3) {
+        if constexpr (F32) {
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(row + 16 * hf + 4 * q);
-            if (live) *reinterpret_cast<f32x4*>(yf + 4 * q) = old[q] + v;
+            f32x4 v = *reinterpret_cast<const f32x4*>(tr + (8 * q + (lane >> 3)) * TP + 4 * (lane & 7));
+            if constexpr (EPI == 3) v = old[q] + v;
+            f32x4* d = reinterpret_cast<f32x4*>(yf + (int64_t)(8 * q) * p.ldy);
+            if (fr + 8 * q < cnt) {
+              if constexpr (NTY) __builtin_nontemporal_store(v, d);
+              else *d = v;
+            }
           }
         } else if constexpr (EPI == 0) {
           float v0[8], v1[8];
@@ -242,8 +255,8 @@ __global__ __launch_bounds__(256, OCC) void k_wgemm(WgParams p) {
           for (int e = 0; e < 8; ++e) { v0[e] = row[16 * hf + e]; v1[e] = row[16 * hf + 8 + e]; }
           if (live) {
             const int64_t o = (int64_t)j * p.ldy + ni[t] * 32 + 16 * hf;
-            vg_store8<OT>(ybase, o, v0);
-            vg_store8<OT>(ybase, o + 8, v1);
+            vg_store8<OT, NTY>(ybase, o, v0);
+            vg_store8<OT, NTY>(ybase, o + 8, v1);
           }
         } else {
           // hidden units ni*16 + 8*hf .. +8: gates in columns 0-15, ups in 16-31
@@ -319,6 +332,9 @@ __global__ __launch_bounds__(1024) void k_mod_lists(const float* comb, int64_t l
 
 }  // namespace
 
+constexpr int64_t kWgLlcBytes = (int64_t)256 << 20;  // last-level cache
+constexpr int kWgHeadCols = 32768;                   // an LM head's columns
+
 int wg_run(WgParams p, int epi, int y_dtype, hipStream_t s) {
   // rows and columns are numbered to the end of their last tile in 32 bits
   if (p.M >= INT_MAX - 256 || p.N >= INT_MAX - 256) return VNX_ERR_UNSUPPORTED;
@@ -341,6 +357,7 @@ int wg_run(WgParams p, int epi, int y_dtype, hipStream_t s) {
   // 2,048 x 2,048 x 1,024 17.2 / 13.3 / 13.9, 2,048 x 1,024 x 2,752 41 / 28 / 22.
   const int64_t cus = device_cus();
   const int sh = row_tiles(4) * groups(2) >= 2 * cus ? 0 : row_tiles(2) * groups(2) >= cus ? 1 : 2;
+  const int64_t wbytes = (int64_t)p.N * p.K * 2;
   // The launch covers all rows whatever total_rows says: how many rows the
   // lists hold is the device's to know (a row whose router logits are NaN is on
   // every expert's), and the workgroups past the live tiles return at once (a
@@ -358,19 +375,28 @@ int wg_run(WgParams p, int epi, int y_dtype, hipStream_t s) {
   // 4-128 rows 89-110 -> 87-103 us, and a 4-layer verify of 8 x 7 tokens around
   // it 344 -> 330 us.  From two row tiles on the second read has to hit: at 224
   // rows 143 us cached, 181 us streamed.
-  const bool nt = p.M <= 128 && (int64_t)p.N * p.K * 2 > ((int64_t)64 << 20);
+  const bool nt = p.M <= 128 && wbytes > ((int64_t)64 << 20);
+  // Logits past the caches (a head's columns): fp32 ones always, as they come in
+  // whole lines (128 rows x 32,768 x 1,024 14.3 us, 15.6 through the caches); 16-bit
+  // ones where they would push out a W that the caches hold between two calls
+  // (224 rows x 64,000 x 2,048 68 us, 85), and not otherwise: the kernel that
+  // reads them next finds them there.
+  const int64_t obytes = (int64_t)p.M * p.N * (y_dtype == VNX_F32 ? 4 : 2);
+  const bool nty = p.N >= kWgHeadCols &&
+                   (y_dtype == VNX_F32 || (wbytes <= kWgLlcBytes && wbytes + obytes > kWgLlcBytes / 4 * 3));
   auto shape = [&](auto ot, auto ep) -> int {
     constexpr int OT = decltype(ot)::value, EP = decltype(ep)::value;
-    if constexpr (EP == 0) {
-      if (sh == 0 && nt) {
-        hipLaunchKernelGGL((k_wgemm<OT, EP, 4, 2, 1, 2, 2, true>), grid, dim3(256), 0, s, p);
-        VNX_LAUNCH_CHECK();
-        return VNX_OK;
-      }
-    }
-    if (sh == 0) hipLaunchKernelGGL((k_wgemm<OT, EP, 4, 2, 1, 2, 2>), grid, dim3(256), 0, s, p);
-    else if (sh == 1) hipLaunchKernelGGL((k_wgemm<OT, EP, 2, 2, 1, 1, 3>), grid, dim3(256), 0, s, p);
-    else hipLaunchKernelGGL((k_wgemm<OT, EP, 2, 1, 2, 4, 2>), grid, dim3(256), 0, s, p);
+    auto go = [&](auto cp) {
+      constexpr int CP = decltype(cp)::value;
+      if (sh == 0) hipLaunchKernelGGL((k_wgemm<OT, EP, 4, 2, 1, 2, 2, CP>), grid, dim3(256), 0, s, p);
+      else if (sh == 1) hipLaunchKernelGGL((k_wgemm<OT, EP, 2, 2, 1, 1, 3, CP & kWgNtY>), grid, dim3(256), 0, s, p);
+      else hipLaunchKernelGGL((k_wgemm<OT, EP, 2, 1, 2, 4, 2, CP & kWgNtY>), grid, dim3(256), 0, s, p);
+    };
+    constexpr int W = EP == 0 ? kWgNtW : 0, Y = EP == 0 ? kWgNtY : 0;
+    if (EP == 0 && sh == 0 && nt && nty) go(IntC<W | Y>{});
+    else if (EP == 0 && sh == 0 && nt) go(IntC<W>{});
+    else if (EP == 0 && nty) go(IntC<Y>{});
+    else go(IntC<0>{});
     VNX_LAUNCH_CHECK();
     return VNX_OK;
   };
