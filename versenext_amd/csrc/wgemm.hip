@@ -369,13 +369,16 @@ int wg_run(WgParams p, int epi, int y_dtype, hipStream_t s) {
   const int64_t wgs = (tiles + kVgXcds - 1) / kVgXcds * kVgXcds;
   if (wgs >= INT_MAX) return VNX_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)wgs);
-  // One row tile reads each byte of W once.  A W past 64 MB then leaves nothing
-  // in the caches that this launch would read again, and pushes out the layers
-  // the next launches read, so it streams past them: the 248,320 x 1,024 head at
-  // 4-128 rows 89-110 -> 87-103 us, and a 4-layer verify of 8 x 7 tokens around
-  // it 344 -> 330 us.  From two row tiles on the second read has to hit: at 224
-  // rows 143 us cached, 181 us streamed.
-  const bool nt = p.M <= 128 && wbytes > ((int64_t)64 << 20);
+  // One row tile reads each byte of W once.  A W that the last-level cache cannot
+  // hold then leaves nothing there that this launch or the next would read
+  // again, and pushes out what the other layers read, so it streams past the
+  // caches: 128 rows x 200,064 x 1,024 101 -> 93 us, 8 x 151,936 x 2,048 120 -> 110,
+  // and a 4-layer verify of 8 x 7 tokens around the 248,320 x 1,024 head 344 ->
+  // 330.  One that fits is better left there (64 rows x 131,072 x 512 28.7 us
+  // streamed, 25.0 not; x 1,024, the whole cache, 49.6 and 45.1).
+  // From two row tiles on the second read has to hit: at 224 rows of the
+  // 248,320 head 143 us cached, 181 streamed.
+  const bool nt = p.M <= 128 && wbytes > kWgLlcBytes;
   // Logits past the caches (a head's columns): fp32 ones always, as they come in
   // whole lines (128 rows x 32,768 x 1,024 14.3 us, 15.6 through the caches); 16-bit
   // ones where they would push out a W that the caches hold between two calls
