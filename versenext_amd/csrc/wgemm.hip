@@ -356,8 +356,19 @@ int wg_run(WgParams p, int epi, int y_dtype, hipStream_t s) {
   // 71 / 66 / 68; one product: 2,048 x 5,504 x 1,024 32.3 / 28.7 / 35.9,
   // 2,048 x 2,048 x 1,024 17.2 / 13.3 / 13.9, 2,048 x 1,024 x 2,752 41 / 28 / 22.
   const int64_t cus = device_cus();
-  const int sh = row_tiles(4) * groups(2) >= 2 * cus ? 0 : row_tiles(2) * groups(2) >= cus ? 1 : 2;
+  int sh = row_tiles(4) * groups(2) >= 2 * cus ? 0 : row_tiles(2) * groups(2) >= cus ? 1 : 2;
   const int64_t wbytes = (int64_t)p.N * p.K * 2;
+  if (!p.counts && p.batch == 1 && p.M > 128 && p.M <= 256 && sh != 2 && wbytes <= kWgLlcBytes) {
+    // Two or fewer 128-row tiles: what counts is how many turns of the chip the
+    // tiles take (2 x 128 or 3 x 64 rows a CU and turn, the latter at 1.09 times
+    // the cost per row) and how much of the last row tile is empty.  129 rows x
+    // 100,352 x 1,024 59 us by the rule above, 48; 224 x 64,000 x 1,024 39 and 35.  A
+    // W that the last-level cache cannot hold is read once per row tile: 129 x
+    // 248,320 x 1,024 145 with two, 148 with three.
+    const int64_t turns0 = (row_tiles(4) * groups(2) + 2 * cus - 1) / (2 * cus);
+    const int64_t turns1 = (row_tiles(2) * groups(2) + 3 * cus - 1) / (3 * cus);
+    sh = row_tiles(4) * groups(2) > cus && turns0 * 256 <= turns1 * 209 ? 0 : 1;
+  }
   // The launch covers all rows whatever total_rows says: how many rows the
   // lists hold is the device's to know (a row whose router logits are NaN is on
   // every expert's), and the workgroups past the live tiles return at once (a
