@@ -452,3 +452,26 @@ def test_a_nan_sequence_leaves_the_others_as_they_are(hip, B, n, bad):
     assert torch.equal(got[ok], want[ok])
     for old, k, v in zip(kv, m.kc, m.vc):
         assert torch.equal(old[:, ok], torch.stack([k, v])[:, ok])
+
+
+@pytest.mark.parametrize("window,alibi,n,T", [(1024, False, 65, 0), (48, True, 100, 300), (4096, False, 130, 2000)])
+def test_both_paths_of_a_long_forward_agree(hip, window, alibi, n, T):
+    """vnx_chain_attn and vnx_tree_attn over chunks, on the same rows and cache
+    with ragged lengths: each rounds fp32 sums to bf16 once, so they differ by
+    one rounding of a value at most (2^-7 of it), or by the sums' own error
+    near 0."""
+    _say("both paths", window, alibi, n, T)
+    cfg = _toy_cfg(window, alibi)
+    dev = hip.torch_device
+    B = 3
+    m = VM.CometSparkGPU(cfg, VM.init_weights(cfg, seed=6), hip, batch=B, capacity=T + n + 8, dtype=torch.bfloat16)
+    g = torch.Generator(device=dev).manual_seed(n)
+    for t in m.kc + m.vc:
+        t.copy_(torch.randn(t.shape, generator=g, device=dev))
+    q = torch.randn((B, cfg.n_head, n, cfg.head_dim), generator=g, device=dev).to(torch.bfloat16)
+    lens = torch.tensor([T, T // 2, T // 3], dtype=torch.int32, device=dev)
+    a = m._attn_chain(q, 1, lens, n, T).float()
+    b = m._attn_tree_chunks(q, 1, lens, n, T).float()
+    assert bool(((a - b).abs() <= 2.0 ** -7 * a.abs() + 2.0 ** -14).all()), float((a - b).abs().max())
+    assert torch.equal(m._attn_long(q, 1, lens, n, T).float(), a if VM.chain_pays(
+        B, cfg.n_head, cfg.n_kv_head, cfg.head_dim, window, n, T, m.cus) else b)

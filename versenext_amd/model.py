@@ -29,8 +29,9 @@ same keys either way.
 Kernels of libvnx_hip.so (gfx950) on the decode and verify forwards:
 - attention of the new rows over the cache, all three TriSparse paths
   (vnx_tree_attn with per-row prefix lengths; RoPE and the cache write of
-  the new rows inside the call for bf16 verify-size forwards; vnx_chain_attn
-  for more rows than a tree call takes: prefill);
+  the new rows inside the call for bf16 verify-size forwards; for more rows
+  than a tree call takes, prefill, vnx_chain_attn, or chunks of them where a
+  long context meets few workgroups: chain_pays);
 - the target's verify-size projections and SwiGLU FFNs on vnx_gemm_bf16
   (RMSNorm staged into the q|k|v and gate-up products, the residual add in
   the output and down products' epilogues, the first layer's token
@@ -296,6 +297,37 @@ def _cat(ws):
     if isinstance(ws[0], Int4Weight):
         return Int4Weight.cat(ws)
     return torch.cat(ws, 0)
+
+
+def chain_pays(B: int, H: int, Hkv: int, d: int, window: int, n: int, Tmax: int, cus: int) -> bool:
+    """Whether the n > 64 new rows of B sequences attend faster through
+    vnx_chain_attn than through vnx_tree_attn over chunks of 64 rows.
+
+    The first is one launch whose workgroups each walk all keys of their
+    columns, a step of 64-256 keys at a time, so a long walk by few workgroups
+    leaves the chip waiting; the second splits the keys over workgroups, at
+    two launches a chunk.  Both costs below are us fitted to 500 shapes (B
+    1-32, 65-512 rows, 500-16,000 keys, windows 1,024-16,384, heads of 64 and
+    128); the path taken is the faster one within 3% at 466 of them, and within
+    31% at all but one.  Measured, chain / chunks: one sequence, 65 rows,
+    16 heads of 64, 2,000 keys 37 / 37, 8,000 keys 102 / 49; 8 heads of 128, 8,000
+    keys 178 / 58; 512 rows, 16 heads of 64, 4,000 keys 64 / 197."""
+    rep, heads = H // Hkv, B * Hkv
+    cols = rep * n
+    # 32 cw query columns a workgroup (ca_column_waves in chain.hip)
+    cw = 4 if heads * -(-cols // 128) >= 2 * cus else 2 if heads * -(-cols // 64) >= cus else 1
+    tiles = heads * -(-cols // (32 * cw))
+    keys = Tmax + n
+    walk = min(keys, window + 32 * cw // rep) if window > 0 else keys
+    steps = -(-walk // (256 // cw))
+    if d == 64:                                            # two workgroups a CU
+        step = (2.3 if cw == 2 else 2.8) * (1.25 if cw < 4 and tiles > cus else 1.0)
+        chain = 12 + step * steps * -(-tiles // (2 * cus))
+    else:
+        chain = (22 if cw == 1 else 14) + (4.85 if cw == 1 else 3.8) * steps * -(-tiles // cus)
+    calls = -(-n // (min(64, window) if window > 0 else 64))
+    work = B * H * n * d * (min(keys, window) if window > 0 else keys) * 1e-9
+    return max(18.5 * calls, 17 * calls + (16 if d == 64 else 19.5) * work) >= 0.95 * chain
 
 
 def _pack(w: torch.Tensor, hip) -> torch.Tensor:
@@ -665,6 +697,7 @@ class CometSparkGPU:
         self.kc = [torch.zeros((self.B, Hkv, self.cap, d), dtype=dtype, device=dev) for _ in self.layers]
         self.vc = [torch.zeros((self.B, Hkv, self.cap, d), dtype=dtype, device=dev) for _ in self.layers]
         self._words = {}
+        self.cus = torch.cuda.get_device_properties(dev).multi_processor_count
         self._neg = torch.full((), -1e9, dtype=torch.float32, device=dev)  # the reference's mask value
         # vnx_tree_attn covers all three paths (window, global rows, ALiBi) for
         # bf16 heads of 64 / 128 (verify-size chunks) and fp32 heads of 8 / 16 /
@@ -726,7 +759,7 @@ class CometSparkGPU:
         return w
 
     def _tree_call(self, q, kc, vc, cstr, tree_k, tree_v, tstr, anc, B, H, Hkv, Tp, n, d, tp, follows, out,
-                   seg2=None, gates=None, qkv=None):
+                   seg2=None, gates=None, qkv=None, out_sb=None, alibi_max=1024):
         a = _lib.TreeAttnArgs()
         if qkv is not None:
             # queries from the q|k|v rows, RoPE and the cache write in the kernel
@@ -742,12 +775,12 @@ class CometSparkGPU:
         a.f32_rows = int(self.f32_rows)
         # output rows in (B, n, H, d) order: the proj input layout
         a.out = out.data_ptr(); a.out_dtype = _lib.DTYPE_CODES[out.dtype]
-        a.out_strides[:] = [n * H * d, d, H * d]
+        a.out_strides[:] = [n * H * d if out_sb is None else out_sb, d, H * d]
         a.B, a.H, a.Hkv, a.Tp, a.N, a.d = B, H, Hkv, Tp, n, d
         a.scale = 1.0 / math.sqrt(d)
         a.window = self.cfg.window_size
         if self.cfg.use_alibi:
-            a.alibi_slopes = self.slopes.data_ptr(); a.alibi_max_keys = 1024
+            a.alibi_slopes = self.slopes.data_ptr(); a.alibi_max_keys = max(0, int(alibi_max))
             a.gates = gates.data_ptr()
         a.tp_batch = tp.data_ptr() if tp is not None else None
         a.tree_follows_prefix = 1 if follows else 0
@@ -783,10 +816,15 @@ class CometSparkGPU:
                         True, o, seg2=(Ly.gk, Ly.gv), gates=Ly.gates, qkv=qkv)
         return o
 
-    def _attn_chain(self, q, li, lens, n, Tmax):
+    def _attn_long(self, q, li, lens, n, Tmax):
         """bf16 forwards of more rows than one vnx_tree_attn call takes
-        (prefill): vnx_chain_attn over the cache, which already holds the n
-        new rows, all paths in one launch.  q (B, H, n, d) bf16."""
+        (prefill); the cache already holds the n new rows.  q (B, H, n, d)."""
+        cfg = self.cfg
+        pays = chain_pays(self.B, cfg.n_head, cfg.n_kv_head, cfg.head_dim, cfg.window_size, n, Tmax, self.cus)
+        return (self._attn_chain if pays else self._attn_tree_chunks)(q, li, lens, n, Tmax)
+
+    def _attn_chain(self, q, li, lens, n, Tmax):
+        """vnx_chain_attn: all rows and paths in one launch.  q (B, H, n, d) bf16."""
         cfg = self.cfg
         B, H, d = self.B, cfg.n_head, cfg.head_dim
         kc, vc = self.kc[li], self.vc[li]
@@ -808,6 +846,29 @@ class CometSparkGPU:
         a.seg2_strides[:] = [0, Ly.gk.stride(1), Ly.gk.stride(2)]
         a.T2 = Ly.gk.shape[2]
         _lib.check(self.hip._L.vnx_chain_attn(ctypes.byref(a), self._st()), "chain_attn")
+        return o
+
+    def _attn_tree_chunks(self, q, li, lens, n, Tmax):
+        """vnx_tree_attn over chunks of the rows, which splits a long walk of keys
+        over workgroups: chunks of at most min(64, window) queries, chunk [c0,
+        c1) seeing each row's lens[b] + c0 prefix rows and its own rows under
+        the chain mask.  The ALiBi path keeps the whole call's rule (lens[b] +
+        n <= 1024, tri_sparse_attn.py:600-607): a chunk passes 1024 - (n - c1)
+        as its key limit.  q (B, H, n, d) bf16."""
+        cfg = self.cfg
+        B, H, d = self.B, cfg.n_head, cfg.head_dim
+        kc, vc = self.kc[li], self.vc[li]
+        Ly = self.layers[li]
+        o = torch.empty((B * n, H * d), dtype=self.act_dtype, device=self.dev)
+        cstr = list(kc.stride()[:3])
+        step = min(64, cfg.window_size) if cfg.window_size > 0 else 64
+        for c0 in range(0, n, step):
+            c1 = min(n, c0 + step)
+            m = c1 - c0
+            lens_c = lens + c0 if c0 else lens
+            self._tree_call(q[:, :, c0:c1], kc, vc, cstr, kc, vc, cstr, self._chain_words(m), B, H, cfg.n_kv_head,
+                            Tmax + c0, m, d, lens_c, True, o[c0:], seg2=(Ly.gk, Ly.gv), gates=Ly.gates,
+                            out_sb=n * H * d, alibi_max=1024 - (n - c1))
         return o
 
     def _attn_torch(self, q, li, lens, n, Tmax):
@@ -1000,8 +1061,8 @@ class CometSparkGPU:
         else:
             x = torch.empty((M, D), dtype=torch.float32, device=self.dev)                # fp32 residual stream
         use_kernel = self.kernel_attention and (self.f32_rows or (n <= 64 and n <= cfg.window_size))
-        # longer bf16 forwards (prefill): one vnx_chain_attn call
-        chain = self.kernel_attention and not use_kernel
+        # longer bf16 forwards (prefill)
+        long = self.kernel_attention and not use_kernel
         pending = None
         for li, L in enumerate(self.layers):
             # bf16 forwards: the residual adds live in the projections
@@ -1065,8 +1126,8 @@ class CometSparkGPU:
                 return None                                # every layer's new cache rows are written
             if use_kernel:
                 o = self._attn_kernel(q, li, lens, n, Tmax, qkv=attn_qkv)
-            elif chain:
-                o = self._attn_chain(q, li, lens, n, Tmax)
+            elif long:
+                o = self._attn_long(q, li, lens, n, Tmax)
             else:
                 o = self._attn_torch(q, li, lens, n, Tmax).permute(0, 2, 1, 3).reshape(M, H * d)
                 o = o.to(self.act_dtype).contiguous()
