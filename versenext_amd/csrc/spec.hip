@@ -569,7 +569,10 @@ static SpecPlan spec_plan(int64_t B, int k, int64_t V, int dtype, int rows_a = -
   pl.chunks = (int)((V + len - 1) / len);
   const int64_t sbl = (int64_t)VNX_WAVE * ve;
   pl.nsb = (V + sbl - 1) / sbl;
-  int64_t c2 = ((int64_t)device_cus() * (k == 0 ? kMassPerCuDraw : kMassPerCu) + B - 1) / B;
+  // (rounded down: the kernel's registers leave room for kMassPerCu workgroups
+  // a CU, and the few past that would run after all others: 48 rows, k = 8, with
+  // 1,056 workgroups 163 us in fp32 and 118 in bf16, with 1,008 157 and 114)
+  int64_t c2 = (int64_t)device_cus() * (k == 0 ? kMassPerCuDraw : kMassPerCu) / B;
   const int64_t max_c2 = (pl.nsb + kNW - 1) / kNW;  // at least one sub-block per wave
   if (c2 > max_c2) c2 = max_c2;
   if (c2 < 1) c2 = 1;
