@@ -44,7 +44,8 @@ namespace vnx {
 constexpr int kNT = 256;   // threads per workgroup
 constexpr int kNW = kNT / VNX_WAVE;
 constexpr int kNB = 8;     // vectors per thread in flight, lse pass
-constexpr int kNB2 = 4;    // sub-blocks per wave in flight, mass pass
+constexpr int kNB2 = 2;    // sub-blocks per wave in flight beside the ones at work, mass pass (with 4 the
+                           // registers and the selects between them cost more than the loads' latency)
 constexpr int kMaxK = 64;
 constexpr int kMaxChunks = 256;
 constexpr int kDrawLds = 4096;  // draw: sub-block masses held in LDS (V <= 4096*64*VE)
@@ -378,7 +379,7 @@ __global__ __launch_bounds__(kNT) void k_spec_lse(SpecParams p) {
 // 40 KB with each form inlined and unrolled).  Launch B of a draw of 8 rows of
 // 248,320 in the engine's rounds: 18.6 -> 12.0 us; of one row's acceptance
 // (k = 4) 12.2 -> 10.1; both launches of 8 rows' (k = 6, bf16) 40 -> 30.5, of
-// 64 rows' (k = 8) 154 -> 151 in bf16, 202 -> 203 in fp32.
+// 64 rows' (k = 8) 158 -> 154 in bf16, 201 either way in fp32.
 // ---------------------------------------------------------------------------
 union MassDrawLds {
   AcceptLds acc;
