@@ -544,11 +544,12 @@ struct SpecPlan {
 // about kMassPerCu workgroups per CU.
 constexpr int64_t kLseWgs = 16384;
 constexpr int64_t kMassPerCu = 4;
-// k = 0 (a plain draw from p_0) streams one row per batch row, not p_n and
-// q_n: half the bytes per workgroup, so half the workgroups (32 rows of
-// 248,320: a 10 us shorter config-5 round; the acceptance at B = 64, k = 8
-// ran its launch B 8 us slower with 2 per CU)
+// A plain draw (k = 0) of few rows takes half as many: its workgroups are short,
+// and the one that draws waits for each of them (4 rows of 248,320 in fp32, 2 / 4
+// per CU, 15.4 / 17.6 us; 16 rows 20.6 / 19.7, 32 28.9 / 27.0, 64 46.0 / 40.3; in
+// bf16 25.4 / 23.4 and 37.5 / 32.8).
 constexpr int64_t kMassPerCuDraw = 2;
+constexpr int64_t kDrawFewRows = 16;
 
 static SpecPlan spec_plan(int64_t B, int k, int64_t V, int dtype, int rows_a = -1) {
   const int ve = dtype == VNX_F32 ? 4 : 8;
@@ -573,7 +574,7 @@ static SpecPlan spec_plan(int64_t B, int k, int64_t V, int dtype, int rows_a = -
   // (rounded down: the kernel's registers leave room for kMassPerCu workgroups
   // a CU, and the few past that would run after all others: 48 rows, k = 8, with
   // 1,056 workgroups 163 us in fp32 and 118 in bf16, with 1,008 157 and 114)
-  int64_t c2 = (int64_t)device_cus() * (k == 0 ? kMassPerCuDraw : kMassPerCu) / B;
+  int64_t c2 = (int64_t)device_cus() * (k == 0 && B < kDrawFewRows ? kMassPerCuDraw : kMassPerCu) / B;
   const int64_t max_c2 = (pl.nsb + kNW - 1) / kNW;  // at least one sub-block per wave
   if (c2 > max_c2) c2 = max_c2;
   if (c2 < 1) c2 = 1;
