@@ -226,34 +226,21 @@ __device__ __forceinline__ double lse_of(float M, double S) {
   return (double)mt_of(M) * kLn2 + log(S);
 }
 
-// Arrival of n pieces at a group counter; true in the workgroup whose
-// arrival completes the group (total pieces).  Same publication contract as
-// arrive_last.
-__device__ __forceinline__ bool arrive_n(unsigned* counter, unsigned n, unsigned total, int* lds_flag) {
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __builtin_amdgcn_s_waitcnt(0);
-    const unsigned prev = __hip_atomic_fetch_add(counter, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    *lds_flag = (prev + n == total) ? 1 : 0;
-  }
-  __syncthreads();
-  return *lds_flag != 0;
-}
-
 // Arrival counter for "last workgroup of a group finishes the group".
-// Contract: the data a group publishes is written by thread 0 of each
-// workgroup with st_agent (agent-scope atomic stores) before it arrives, and
-// read by the last workgroup with ld_agent (agent-scope atomic loads).  Those
-// accesses are coherent across the XCDs by themselves, so no fence is needed,
-// only ordering: s_waitcnt(0) completes thread 0's stores before its counter
-// increment issues.  (A __threadfence here would write back and invalidate
-// the whole L2 of the XCD for every workgroup; with thousands of workgroups
-// per launch that costs more than streaming the rows.)  The counter is zeroed
-// by k_zero_u32 at the start of every call.
+// Contract: the data a group publishes is written by any wave of its workgroups
+// with st_agent (agent-scope atomic stores) before they arrive, and read by
+// the last workgroup with ld_agent (agent-scope atomic loads).  Those accesses
+// are coherent across the XCDs by themselves, so no fence is needed, only
+// ordering: every wave's s_waitcnt(0) completes its stores before the barrier,
+// after which thread 0's counter increment issues.  (A __threadfence here
+// would write back and invalidate the whole L2 of the XCD for every workgroup;
+// with thousands of workgroups per launch that costs more than streaming the
+// rows.)  The counter is 0 at the start of the launch: an earlier launch of the
+// call clears it.
 __device__ __forceinline__ bool arrive_last(unsigned* counter, unsigned total, int* lds_flag) {
+  __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   if (threadIdx.x == 0) {
-    __builtin_amdgcn_s_waitcnt(0);
     const unsigned prev = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     *lds_flag = (prev == total - 1) ? 1 : 0;
   }

@@ -840,8 +840,6 @@ __global__ __launch_bounds__(kSNT, 4) void k_samp_mass(SampParams p) {
 #pragma unroll 1
   for (;;) {
     if (sb >= s1) {  // this wave's masses are out (never while drawing)
-      // every wave's published masses complete before the workgroup arrives
-      __builtin_amdgcn_s_waitcnt(0);
       if (!arrive_last(p.cnt + b * kCntLd, (unsigned)p.C, &L.flag)) return;
       if (!live) break;
       // the nucleus ties of the whole row now hold by id: jbound = j*

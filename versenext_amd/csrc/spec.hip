@@ -436,8 +436,6 @@ __global__ __launch_bounds__(kNT, 4) void k_spec_mass_draw(SpecParams p) {
   for (;;) {
     if (sb >= s1) {  // this wave's masses are out (never while drawing)
       if (!redo) {
-        // every wave's published masses complete before the workgroup arrives
-        __builtin_amdgcn_s_waitcnt(0);
         if (!arrive_last(&p.cnt[b * p.cnt_ld], (unsigned)p.chunks2, &last_flag)) return;
         walk_load<kNT>(p.sbm + b * nsb, nsb, dyn);
       }
