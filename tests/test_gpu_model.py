@@ -475,3 +475,20 @@ def test_both_paths_of_a_long_forward_agree(hip, window, alibi, n, T):
     assert bool(((a - b).abs() <= 2.0 ** -7 * a.abs() + 2.0 ** -14).all()), float((a - b).abs().max())
     assert torch.equal(m._attn_long(q, 1, lens, n, T).float(), a if VM.chain_pays(
         B, cfg.n_head, cfg.n_kv_head, cfg.head_dim, window, n, T, m.cus) else b)
+
+
+@pytest.mark.parametrize("parts,experts,dtype", [(2, 4, torch.bfloat16), (8, 4, torch.bfloat16), (2, 4, torch.float32)])
+def test_expert_weights_are_held_once(hip, parts, experts, dtype):
+    """Packed for the routed products (up to 32 router rows, bf16), or as the
+    operands of the batched ones, never both; either form runs."""
+    cfg = VM.ModelConfig(vocab_size=200, dim=128, n_layer=1, n_head=2, n_kv_head=1, layer_pattern=("mod",),
+                         window_size=64, num_global_tokens=4, use_alibi=False, use_rope=True, num_dense_parts=parts,
+                         num_experts_per_part=experts, top_k=2)
+    m = VM.CometSparkGPU(cfg, VM.init_weights(cfg, seed=1), hip, batch=2, capacity=320, dtype=dtype)
+    routed = parts + parts * experts <= 32 and dtype == torch.bfloat16
+    assert ("w1p" in m.layers[0].ffn, "w2p" in m.layers[0].ffn) == (routed, routed)
+    assert ("w1" in m.layers[0].ffn, "w2" in m.layers[0].ffn) == (not routed, not routed)
+    lens = torch.zeros(2, dtype=torch.int32, device=hip.torch_device)
+    for n in (3, 300):
+        h = m.forward(torch.arange(2 * n, device=hip.torch_device).view(2, n) % 200, lens, 0)
+        assert bool(torch.isfinite(h).all())

@@ -676,18 +676,19 @@ class CometSparkGPU:
                         ep = p + f"ffn.parts.{q}.experts.{e}."
                         w1.append(torch.cat([W[ep + "w_gate.weight"], W[ep + "w_up.weight"]], 0))
                         w2.append(W[ep + "w_down.weight"])
-                # batched-product operands, untransposed and contiguous:
-                # (P*E, D, 2He) gate|up and (P*E, He, D) down
-                L.ffn["w1"] = torch.stack([w.t() for w in w1]).to(dtype).contiguous()
-                L.ffn["w2"] = torch.stack([w.t() for w in w2]).to(dtype).contiguous()
-                if dtype == torch.bfloat16 and D % 64 == 0 and cfg.expert_hidden_eff % 64 == 0:
-                    # packed per-expert copies for the routed products of
-                    # verify-size forwards (vnx_expert_gemm_bf16); gate|up
-                    # rows interleaved in blocks of 16 for the SwiGLU epilogue
-                    He = cfg.expert_hidden_eff
+                He = cfg.expert_hidden_eff
+                if dtype == torch.bfloat16 and D % 64 == 0 and He % 64 == 0 and P + P * E <= 32:
+                    # packed per expert for the routed products (_mod_routed);
+                    # gate|up rows interleaved in blocks of 16 for the SwiGLU
+                    # epilogue
                     L.ffn["w1p"] = torch.stack([_pack(w.to(dtype).view(2, He // 16, 16, D).transpose(0, 1)
                                                       .reshape(2 * He, D).contiguous(), hip) for w in w1])
                     L.ffn["w2p"] = torch.stack([_pack(w.to(dtype).contiguous(), hip) for w in w2])
+                else:
+                    # batched-product operands, untransposed and contiguous:
+                    # (P*E, D, 2He) gate|up and (P*E, He, D) down
+                    L.ffn["w1"] = torch.stack([w.t() for w in w1]).to(dtype).contiguous()
+                    L.ffn["w2"] = torch.stack([w.t() for w in w2]).to(dtype).contiguous()
             self.layers.append(L)
         cos, sin = rope_tables(d, self.cap + 64, cfg.rope_theta)
         self.cos = torch.from_numpy(cos).to(dev)
@@ -978,7 +979,7 @@ class CometSparkGPU:
         P_ = ctypes.c_void_p
         L_ = self.hip._L
         out = torch.empty((M, D), dtype=torch.float32, device=self.dev)
-        if P + PE <= 32 and "w1p" in L.ffn:
+        if "w1p" in L.ffn:
             self._mod_routed(L, h, None, out, False)
             return out
         comb = torch.empty((M, PE), dtype=torch.float32, device=self.dev)
@@ -1074,7 +1075,7 @@ class CometSparkGPU:
             fused = (L.wqkv.wp is not None and L.proj.wp is not None
                      and self.dtype == torch.bfloat16
                      and pending is None
-                     and ("w1p" in L.ffn and len(L.ffn["route"]) <= 32 if L.kind == "mod" else
+                     and ("w1p" in L.ffn if L.kind == "mod" else
                           (L.ffn["gu"].wp is not None and L.ffn["gu"].swiglu and L.ffn["down"].wp is not None)))
             norm_in = fused and M <= _Linear.GEMM_MAX_M and D <= 2048
             # the INT4 draft's decode: the same fusions on its GEMVs
