@@ -1267,15 +1267,15 @@ static int qwgemm_launch(const QGemvParams& p, int bits, hipStream_t s) {
 
 static int qgemv_launch(QGemvParams p, int bits, hipStream_t s) {
   if (p.B == 0 || p.N == 0) return VNX_OK;
-  // The tiled GEMM from 33 rows on, where the narrow kernels would take a second
-  // 32-row pass: 40 rows x 2,048 x 2,048 9.2 us there, 8.6 here; 1,024 rows 162
-  // and 21; an LM head's 33 rows x 248,320 x 1,024 in INT4 group-128 73 and 59, INT8
-  // 117 and 69; 64 rows x 32,784 x 1,024 24 and 17.  The widest tile that leaves a workgroup
+  // The tiled GEMM from 33 rows on (a second 32-row pass of the narrow
+  // kernels: 40 rows x 2,048 x 2,048 9.2 us there, 8.6 here; 1,024 rows 162
+  // and 21), except for the many weight rows of an LM head, whose streaming
+  // kernels take up to two passes.  The widest tile that leaves a workgroup
   // per CU, else the K split of four waves (us, 64 x 128 / 32 x 128 / 32 x 64 /
   // 32 x 32): 1,024 rows x 2,048 x 2,048 21 / 22 / 28 / 43, 512 rows 19 / 14 /
   // 15 / 22, 256 rows 18 / 13 / 10 / 12, 128 rows 18 / 13 / 9.8 / 8.9.
   const bool plain = !p.yh && !p.rope_on && !p.resid && !p.xf;
-  if (plain && p.B > 32) {
+  if (plain && p.B > 32 && (p.N < kQTileMaxN || p.B > 64)) {
     auto tiles = [&](int64_t rt, int64_t ct) { return ((p.B + rt - 1) / rt) * ((p.N + ct - 1) / ct); };
     const int64_t cus = device_cus();
     if (tiles(64, 128) >= cus) return qwgemm_launch<2, 4>(p, bits, s);
