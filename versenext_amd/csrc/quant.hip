@@ -1269,8 +1269,10 @@ static int qgemv_launch(QGemvParams p, int bits, hipStream_t s) {
   if (p.B == 0 || p.N == 0) return VNX_OK;
   // The tiled GEMM from 33 rows on (a second 32-row pass of the narrow
   // kernels: 40 rows x 2,048 x 2,048 9.2 us there, 8.6 here; 1,024 rows 162
-  // and 21), except for the many weight rows of an LM head, whose streaming
-  // kernels take up to two passes.  The widest tile that leaves a workgroup
+  // and 21), except for 33-64 rows of an LM head: up to 64 rows its row layout
+  // gives the bits of its tiled one (vnx_gemv_w4_tiles), which a caller may take
+  // instead, at 73 us for 33 rows x 248,320 x 1,024 in INT4 group-128 against 59
+  // here, and 117 against 69 in INT8.  The widest tile that leaves a workgroup
   // per CU, else the K split of four waves (us, 64 x 128 / 32 x 128 / 32 x 64 /
   // 32 x 32): 1,024 rows x 2,048 x 2,048 21 / 22 / 28 / 43, 512 rows 19 / 14 /
   // 15 / 22, 256 rows 18 / 13 / 10 / 12, 128 rows 18 / 13 / 9.8 / 8.9.
