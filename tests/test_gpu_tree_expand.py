@@ -1,10 +1,12 @@
-"""vnx_tree_expand against the row top-b it replaces (vnx_row_topk on every
-row, then each node's rank), and tree attention with the ancestor words passed
-by value against the same words on the device: both bit for bit."""
+"""vnx_tree_expand against the oracle and against the row top-b it replaces
+(vnx_row_topk on every row, then each node's rank), and tree attention with the
+ancestor words passed by value against the same words on the device: all bit
+for bit."""
 import numpy as np
 import pytest
 import torch
 
+from oracle import tree as OT
 from versenext_amd import tree as T
 
 pytestmark = pytest.mark.gpu
@@ -67,3 +69,19 @@ def test_ancestor_words_by_value(hip, N, Tp, d, window, alibi):
         kw.update(alibi_slopes=torch.rand(H, generator=g, device=hip.torch_device), gates=torch.tensor([0.5, 0.2, 0.9]))
     args = (r(B, H, N, d), kc, vc, r(B, Hkv, N, d), r(B, Hkv, N, d))
     assert torch.equal(hip.tree_attention(*args, words, **kw), hip.tree_attention(*args, np.tile(words, (B, 1)), **kw))
+
+
+@pytest.mark.parametrize("par", [T.chain(6), [-1] * 16, T.tree_from_branching((4, 3, 2)), [-1, 0, -1, 0, 2, 1, 0, 2, 4]],
+                         ids=["chain", "wide", "432", "mixed"])
+@pytest.mark.parametrize("V,dtype", [(17, torch.float32), (8193, torch.bfloat16), (20011, torch.float32)])
+def test_expand_equals_the_oracle(hip, par, V, dtype):
+    par = np.asarray(par, np.int32)
+    B, R = 3, par.size + 1
+    print("expand against the oracle", par.size, V, dtype, flush=True)
+    g = torch.Generator().manual_seed(V + R)
+    draft = torch.randn((B, R, V), generator=g).to(dtype)
+    draft[0, 0, V // 2:] = 9.0                           # ties go to the lower id
+    draft[1, :, 1] = float("-inf")
+    draft[1, 0, 3], draft[2, R // 2, 5], draft[2, 0, 7] = float("nan"), float("nan"), float("inf")
+    got = hip.expand_tree(draft, par)
+    assert np.array_equal(got.cpu().numpy(), OT.expand_tree(draft.float().numpy(), par))
