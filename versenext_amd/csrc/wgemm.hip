@@ -219,16 +219,12 @@ __global__ __launch_bounds__(256, OCC) void k_wgemm(WgParams p) {
     for (int t = 0; t < CT; ++t) {
       if (ni[t] >= p.nt) continue;             // uniform per wave
       if (p.vec_out) {
-        // fp32: lane l's piece q is row 8q + l / 8, columns 4 (l % 8) .. + 4, so
-        // eight lanes write (and EPI 3 reads) a whole 128-byte line of a row
-        constexpr bool F32 = OT == 0 && EPI != 1;
-        const int fr = m0 + i * 32 + (lane >> 3);
-        float* yf = reinterpret_cast<float*>(ybase) + (int64_t)fr * p.ldy + ni[t] * 32 + 4 * (lane & 7);
         f32x4 old[EPI == 3 ? 4 : 1];
+        float* yf = reinterpret_cast<float*>(ybase) + (int64_t)j * p.ldy + ni[t] * 32 + 16 * hf;
         if constexpr (EPI == 3) {
+          if (live)
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
-            if (fr + 8 * q < cnt) old[q] = *reinterpret_cast<const f32x4*>(yf + (int64_t)(8 * q) * p.ldy);
+            for (int q = 0; q < 4; ++q) old[q] = *reinterpret_cast<const f32x4*>(yf + 4 * q);
         }
 #pragma unroll
         for (int ii = 0; ii < 4; ++ii)
@@ -238,12 +234,23 @@ __global__ __launch_bounds__(256, OCC) void k_wgemm(WgParams p) {
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         const float* row = tr + (lane >> 1) * TP;
-        if constexpr (F32) {
+        if constexpr (EPI == 3) {
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            f32x4 v = *reinterpret_cast<const f32x4*>(tr + (8 * q + (lane >> 3)) * TP + 4 * (lane & 7));
-            if constexpr (EPI == 3) v = old[q] + v;
-            f32x4* d = reinterpret_cast<f32x4*>(yf + (int64_t)(8 * q) * p.ldy);
+            const f32x4 v = *reinterpret_cast<const f32x4*>(row + 16 * hf + 4 * q);
+            if (live) *reinterpret_cast<f32x4*>(yf + 4 * q) = old[q] + v;
+          }
+        } else if constexpr (OT == 0 && EPI == 0) {
+          // lane l's piece q is row 8q + l / 8, columns 4 (l % 8) .. + 4: eight
+          // lanes write a whole 128-byte line of a row (the residual add above
+          // is faster in the other order, its loads under one condition: 23.8 us
+          // against 24.6 for 2,048 x 1,024 x 2,752)
+          const int fr = m0 + i * 32 + (lane >> 3);
+          float* yl = reinterpret_cast<float*>(ybase) + (int64_t)fr * p.ldy + ni[t] * 32 + 4 * (lane & 7);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(tr + (8 * q + (lane >> 3)) * TP + 4 * (lane & 7));
+            f32x4* d = reinterpret_cast<f32x4*>(yl + (int64_t)(8 * q) * p.ldy);
             if (fr + 8 * q < cnt) {
               if constexpr (NTY) __builtin_nontemporal_store(v, d);
               else *d = v;
