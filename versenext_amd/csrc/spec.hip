@@ -379,7 +379,7 @@ __global__ __launch_bounds__(kNT) void k_spec_lse(SpecParams p) {
 // 40 KB with each form inlined and unrolled).  Launch B of a draw of 8 rows of
 // 248,320 in the engine's rounds: 18.6 -> 12.0 us; of one row's acceptance
 // (k = 4) 12.2 -> 10.1; both launches of 8 rows' (k = 6, bf16) 40 -> 30.5, of
-// 64 rows' (k = 8) 158 -> 154 in bf16, 201 either way in fp32.
+// 64 rows' (k = 8) 148 -> 144 in bf16, 197 -> 195 in fp32.
 // ---------------------------------------------------------------------------
 union MassDrawLds {
   AcceptLds acc;
@@ -461,42 +461,53 @@ __global__ __launch_bounds__(kNT, 4) void k_spec_mass_draw(SpecParams p) {
     }
     // one sub-block (past the whole ones, or the one drawn from), or U
     const bool one = draw || sb + kNW * (U - 1) >= whole;
-    u32x4 ap[U], aq[U];
     if (one) {
-      ap[0] = aq[0] = lane_raw<Tin>(P, sb, p.V);
-      if (resid) aq[0] = lane_raw<Tin>(Q, sb, p.V);
-#pragma unroll
-      for (int q = 1; q < U; ++q) { ap[q] = ap[0]; aq[q] = aq[0]; }
-    } else {
-#pragma unroll
-      for (int q = 0; q < U; ++q) {
-        ap[q] = rp[q];
-        aq[q] = rq[q];
-#pragma unroll
-        for (int t = U; t < kNB2; t += U)
-          if (j == t) { ap[q] = rp[t + q]; aq[q] = rq[t + q]; }
-      }
-      j += U;
-      if (j == kNB2) load(sb + kNW * U);  // under this turn's weights
+      rp[0] = lane_raw<Tin>(P, sb, p.V);
+      if (resid) rq[0] = lane_raw<Tin>(Q, sb, p.V);
+      j = 0;
     }
+    // The exponents first, which frees the raw registers for the next batch
+    // without a copy of them.
+    float tq[U][VE];
 #pragma unroll
     for (int q = 0; q < U; ++q) {
-      float xp[VE];
-      Vec<Tin>::cvt_raw(ap[q], xp);
+      u32x4 a = rp[q];
 #pragma unroll
-      for (int i = 0; i < VE; ++i) w[q][i] = vnx_exp_canon(scaled<SM, THR>(xp[i], p.sc, d.thr_p) - jb.Lp);
+      for (int t = U; t < kNB2; t += U)
+        if (j == t) a = rp[t + q];
+      float x[VE];
+      Vec<Tin>::cvt_raw(a, x);
+#pragma unroll
+      for (int i = 0; i < VE; ++i) w[q][i] = scaled<SM, THR>(x[i], p.sc, d.thr_p) - jb.Lp;
     }
     if (resid)
 #pragma unroll
       for (int q = 0; q < U; ++q) {
-        float xq[VE];
-        Vec<Tin>::cvt_raw(aq[q], xq);
+        u32x4 a = rq[q];
+#pragma unroll
+        for (int t = U; t < kNB2; t += U)
+          if (j == t) a = rq[t + q];
+        float x[VE];
+        Vec<Tin>::cvt_raw(a, x);
+#pragma unroll
+        for (int i = 0; i < VE; ++i) tq[q][i] = scaled<SM, THR>(x[i], p.sc, d.thr_q) - jb.Lq;
+      }
+    if (!one) {
+      j += U;
+      if (j == kNB2) load(sb + kNW * U);  // under this turn's weights
+    }
+#pragma unroll
+    for (int q = 0; q < U; ++q)
+#pragma unroll
+      for (int i = 0; i < VE; ++i) w[q][i] = vnx_exp_canon(w[q][i]);
+    if (resid)
+#pragma unroll
+      for (int q = 0; q < U; ++q)
 #pragma unroll
         for (int i = 0; i < VE; ++i) {
-          const float r = w[q][i] - vnx_exp_canon(scaled<SM, THR>(xq[i], p.sc, d.thr_q) - jb.Lq);
+          const float r = w[q][i] - vnx_exp_canon(tq[q][i]);
           w[q][i] = r > 0.0f ? r : 0.0f;
         }
-      }
 #pragma unroll
     for (int q = 0; q < U; ++q) {
       lm[q] = 0.0;
