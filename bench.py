@@ -442,7 +442,8 @@ def cpu_tree(h, par, reps: int = 5):
 
 
 def bench_lmhead(args):
-    """Verify-pass LM head (vnx_lm_head): logits (M, V) = x (M, 1024) . W^T with
+    """LM head on row-major weights (vnx_lm_head; the model's own verify forward
+    runs its packed copy on vnx_gemm_bf16): logits (M, V) = x (M, 1024) . W^T with
     M = B*(k+1) = 32*7 = 224 (config 5's verify batch), W the 248,320 x 1024
     bf16 tied embedding (N(0, 0.02)), x bf16 N(0, 1).  bytes = 2*V*K (W) +
     2*M*K (x) + out_bytes*M*V; flop = 2*M*V*K.  Timed back to back on

@@ -1,4 +1,4 @@
-"""GPU parity of the verify-pass LM head (vnx_lm_head, matrix cores).
+"""GPU parity of the LM head on row-major weights (vnx_lm_head, matrix cores).
 
 Reference: the fp64 product of the same bf16 inputs (x @ w.T, the tied head
 of cometspark.py:396-398).  Bar: |out - ref| <= RTOL * sum_k |x_k w_k| per

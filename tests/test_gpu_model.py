@@ -6,7 +6,7 @@ Bars:
 - fp32 model (torch attention path): logits within 1e-4 of the reference's
   (fp32 sums in a different order than numpy's);
 - bf16 model on the kernel path (vnx_tree_attn with per-row prefix lengths,
-  vnx_lm_head): logits within 3e-2 of the fp32 oracle's scale (bf16 weights
+  the packed head on vnx_gemm_bf16): logits within 3e-2 of the fp32 oracle's scale (bf16 weights
   and activations; the north star's bf16 bar is 2e-2 on probabilities);
 - greedy speculative decode: the emitted stream equals the target's greedy
   stream bit for bit."""
@@ -117,7 +117,7 @@ def _toy_cfg(window=1024, alibi=False):
 def test_bf16_kernel_path_matches_oracle(hip, window, alibi):
     """head_dim 64, RoPE, with and without a window the contexts cross and
     ALiBi: the new rows attend through vnx_tree_attn (per-row prefix
-    lengths, rows written in place) and the head runs on vnx_lm_head;
+    lengths, rows written in place) and the head runs on vnx_gemm_bf16;
     compared with the fp32 oracle on each row's sequence."""
     _say(f"bf16 kernel path window={window} alibi={alibi}")
     cfg = _toy_cfg(window, alibi)
@@ -134,7 +134,7 @@ def test_bf16_kernel_path_matches_oracle(hip, window, alibi):
     rng = np.random.default_rng(8)
     committed = [list(rng.integers(0, 1000, 70)) for _ in range(B)]
     lens = torch.zeros(B, dtype=torch.int32, device=dev)
-    m.forward(torch.tensor(committed, device=dev), lens, 0)   # prefill: the kernel over query chunks
+    m.forward(torch.tensor(committed, device=dev), lens, 0)   # prefill: more rows than a tree call takes
     lens += 70
     worst = 0.0
     for step, adv in enumerate([(1, 7, 3, 5), (7, 2, 1, 4), (3, 3, 7, 1)]):
@@ -154,7 +154,8 @@ def test_bf16_kernel_path_matches_oracle(hip, window, alibi):
 @pytest.mark.parametrize("window,alibi", [(48, True), (1024, False)])
 def test_bf16_long_forwards_run_the_kernel_in_chunks(hip, window, alibi):
     """bf16 forwards of more rows than one attention call takes (prefill)
-    run vnx_tree_attn over query chunks: a 100-row prefill, then 70 rows on
+    run vnx_chain_attn, or vnx_tree_attn over query chunks where that is
+    faster (chain_pays): a 100-row prefill, then 70 rows on
     top of 960 cached ones, where the whole call passes 1024 keys, so the
     ALiBi path is off for every chunk (the reference's rule for the call,
     not for each chunk); all rows compared with the fp32 oracle."""

@@ -726,7 +726,7 @@ class HipBackend(DeviceBackend):
         return acc.view(torch.bool), pred, alen, out   # the kernel writes 0 / 1
 
     def lm_head(self, x, weight, out=None, out_dtype=torch.float32) -> torch.Tensor:
-        """Verify-pass LM head (vnx_lm_head): x (..., K) . weight (V, K)^T on the
+        """LM head on row-major weights (vnx_lm_head): x (..., K) . weight (V, K)^T on the
         matrix cores, bf16 in, fp32 accumulate; returns (..., V) in out_dtype
         (or writes `out`, a (rows, V) view with unit last stride)."""
         dev = self._torch_device

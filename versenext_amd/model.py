@@ -1162,8 +1162,8 @@ class CometSparkGPU:
 
     def head_writes_bf16(self) -> bool:
         """Whether logits(out=<bf16 tensor>) is written by the head itself:
-        the bf16 LM head (vnx_lm_head), or an INT4 head on its tiled copy
-        (vnx_gemv_w4_tiles_out)."""
+        the bf16 LM head (vnx_gemm_bf16 on its packed copy), or an INT4 head on
+        its tiled copy (vnx_gemv_w4_tiles_out)."""
         if self.head is not None:
             return self.head.wt is not None if self.head.int4 else self.dtype == torch.bfloat16
         return self.dtype == torch.bfloat16
